@@ -72,11 +72,11 @@ typedef struct spz_config {
                                 1 = no split; at most 1048576 */
     int32_t max_split_depth; /* cap on that split depth (0 = 24) */
     int32_t workgroup_size;  /* 64, 128 or 256 lanes (0 = 256) */
-    int32_t lanes;           /* DFS lanes in flight (0 = fill the device;
-                                at most 2^24) */
-    int32_t round_budget;    /* DFS steps per lane per round (0 = auto:
-                                2048 for Manhattan when the batch has work
-                                for every lane, else 1024; at most 2^20) */
+    int32_t lanes;           /* DFS lanes in flight (0 = auto; no more than
+                                the device runs at once are used; at most
+                                2^24) */
+    int32_t round_budget;    /* DFS steps per lane per round (0 = auto: 8192;
+                                at most 2^20) */
     int32_t lds_stack_depth; /* DFS stack levels per lane kept in LDS (0 =
                                 80 for width 4, 96 for width 5 Manhattan, 64
                                 for the PDB search; at most 160);
@@ -109,11 +109,8 @@ typedef struct spz_config {
                                 (src/24puzzle.cc:146-152) */
     int32_t round_time_us;   /* a search round also ends this many
                                 microseconds after its start (whichever comes
-                                first with round_budget steps), so that waves
-                                that step faster under load do not wait for
-                                the slowest; 0 = auto (4500 for the PDB search;
-                                Manhattan 3500 when the batch has work for
-                                every lane, else 700), < 0 = off */
+                                first with round_budget steps); 0 = auto
+                                (4500), < 0 = off */
     int32_t dedup;           /* 1: duplicate pruning in the root split: a
                                 top-tree node whose board an earlier kept node
                                 of its instance holds with a path-max f no
@@ -267,7 +264,8 @@ int spz_get_samples(spz_ctx *ctx, uint8_t *boards, int32_t *thr, uint64_t *loads
 int spz_get_paths(spz_ctx *ctx, uint8_t *moves, int32_t max_len, int32_t *lens);
 
 /* Statistics of the last solve (stats must hold SPZ_STATS_LEN doubles):
- *  0 rounds run            1 solve wall ms        2 items donated
+ *  0 rounds run            1 solve wall ms        2 nodes given to waves
+ *                                                  without work
  *  3 lanes                 4,5 PDB BFS levels     6 PDB build ms
  *  7 stack-overflow items  8 round-kernel ms (sum, when time_kernels)
  *  9 round launches timed  10 split ms            11 instances

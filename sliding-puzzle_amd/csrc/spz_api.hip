@@ -146,13 +146,14 @@ struct spz_ctx {
     bool have_pdb = false;
 
     // lane contexts
-    DBuf c_st, c_rows, c_root, c_meta, c_rmeta, c_inst, c_cnt, c_pdb, c_stack;
+    DBuf c_st, c_rows, c_meta, c_inst, c_cnt, c_pdb, c_stack;
     // queue and control
     DBuf q, q_ctl, ctl;
+    DBuf list, mail, mail_head, ticket, mail_path; // waves without work
     size_t qcap = 0;
     // per instance
-    DBuf roots, L, it, cnt, pend, found, done, opt, iter_counts, restart_list;
-    DBuf itn, drained, dead, nlive, Lbase, listed, want_next; // iteration slots (lookahead)
+    DBuf roots, L, it, cnt, pend, found, done, opt, iter_counts;
+    DBuf itn, drained, dead, nlive, Lbase, want_next; // iteration slots (lookahead)
     DBuf frontier, nfront, topgen, top_goal, frozen, lvl[2], nlvl[2];
     // load balancing
     DBuf c_origin, load, samples, nsamp, pred;
@@ -257,44 +258,32 @@ void spz_default_config(spz_config *cfg, int32_t width, int32_t heuristic) {
     cfg->lookahead = 1;
 }
 
-// Steps per lane and round when the configuration leaves it open: shorter
-// rounds refill idle lanes sooner, longer ones spend less on the context save
-// and restore.  `full`: the solve has work for every lane of the context (its
-// automatic lane count reached the capacity).  Measured on MI355X: 1024 beats
-// 256 and 512 for the PDB search, where 2048 is level with it; the Manhattan
-// search gains from longer rounds only when the batch fills every lane (4096
-// mixed 15-puzzles: 2048 steps / 3.5 ms 829 instances/s, 1024 / 2.5 ms 773),
-// and loses with one instance on a part of them (44.8 -> 39.6).
-static int default_round_budget(int heur, bool full) { return (heur != SPZ_H_PDB666 && full) ? 2048 : 1024; }
+// Step budget and time limit of a round when the configuration leaves them
+// open.  Waves share work while a round runs and end it themselves when many
+// have none, so a round is long: what it costs is that an instance whose
+// iteration ends inside it waits for its next one.  Measured on MI355X, 250
+// mixed 15-puzzles: 2 ms 1048 ms, 3.5 ms 1053, 4.5 ms 1037, 10 ms 1035; 24
+// 24-puzzles with the PDB 181 / 178 / 179 / 180.  The step budget only bounds
+// rounds whose time limit is off.
+constexpr int kRoundSteps = 8192;
+constexpr int kRoundTimeUs = 4500;
 
-// Time limit of a round when the configuration leaves it open.  With a step
-// budget alone, waves that step faster (fewer lanes on divergent paths) end
-// early and wait for the slowest -- in the 24-puzzle PDB search under load,
-// waves end 4.75 ms (10th percentile) to 5.5 ms (last) into a 1024-step
-// round.  The limit cuts that tail; lightly loaded rounds, which step faster,
-// still end at their step budget (measured on MI355X: PDB 4500 us beat 3200,
-// 4000, 4800 and 5600; Manhattan batches with work for every lane, 3500 us
-// beat 2000 and 3000 at 2048 steps).  A solve with fewer items than lanes
-// (one random 15-puzzle per call, 2048 frontier nodes on 65536 lanes) keeps
-// lanes fed only by the donations made at each round's end, so its rounds
-// are short: 700 us, 48.1 instances/s against 47.9 at 500, 47.3 at 1000 and
-// 45.9 at 2500 (1024 steps).
-static int default_round_time_us(int heur, bool full) {
-    return heur == SPZ_H_PDB666 ? 4500 : (full ? 3500 : 700);
-}
-
-// Lanes per compute unit of the 24-puzzle searches: more resident lanes than
-// this lose more to L2 sharing and finer work splitting than they gain in
-// latency hiding (measured on MI355X: 768 beat 1024 and 512 for both
-// heuristics).
-constexpr int kLanesPerCu5 = 768;
+// Lanes per compute unit of the PDB search: three waves per SIMD are what its
+// LDS holds (stack, boards, sibling values: 53.6 KB per 256 lanes).
+constexpr int kLanesPerCuPdb = 768;
 // Lanes per initial work item (root-split frontier node) when the lane count
-// is automatic: a batch with little work runs on fewer lanes, which split it
-// less finely (a single 15-puzzle instance, 2048 frontier nodes: 65536 lanes
-// ran 2.4x as fast as 524288, and faster than 32768 or 131072).
-constexpr size_t kLanesPerItem = 32;
-// step budget of the rounds that run while the queue holds little work
-constexpr int kShortRoundSteps = 128;
+// is automatic: a small search is over before many waves are fed (one random
+// 15-puzzle, 2048 frontier nodes: 65536 lanes 5.2 ms, 131072 4.7, 262144 5.0,
+// 524288 5.4; 250 mixed ones, 16 each: 131072 lanes 1513 ms, 256000 1040,
+// 524288 1030).
+constexpr size_t kLanesPerItem = 64;
+// A round ends early once the waves that ran out of work have waited, summed
+// over them and divided by all waves, this long: about what it costs to end a
+// round, save and restore the lanes, start iterations and feed the waves again.
+// 150 / 300 / 600 us: one random 15-puzzle 4.7 / 4.7 / 4.8 ms, 100 short walks
+// 6.5 / 6.0 / 5.9, one 24-puzzle with the PDB 5.3 / 5.0 / 4.4, 24 of them 182 /
+// 178 / 174.
+constexpr double kTurnUs = 300.0;
 
 // Lane capacity (from occupancy unless given) and lane-context arrays for
 // the context's workgroup size and LDS stack depth.
@@ -302,13 +291,15 @@ static int configure_lanes(spz_ctx *ctx) {
     const spz_config *cfg = &ctx->cfg;
     const int wg = ctx->wg;
     hipError_t e;
-    int lanes = cfg->lanes;
+    int blocks = 0;
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, round_kernel_ptr(cfg->width, cfg->heuristic), wg,
+                                                     round_lds_bytes(cfg->width, cfg->lds_stack_depth, wg, cfg->heuristic));
+    if (e != hipSuccess || blocks <= 0) blocks = 2;
+    // at most what runs at once: in a round, waves without work wait for those
+    // that have some, so none may still wait to start
+    int lanes = cfg->lanes > 0 ? std::min(cfg->lanes, ctx->n_cu * blocks * wg) : 0;
     if (lanes <= 0) {
-        int blocks = 0;
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, round_kernel_ptr(cfg->width, cfg->heuristic), wg,
-                                                         round_lds_bytes(cfg->width, cfg->lds_stack_depth, wg, cfg->heuristic));
-        if (e != hipSuccess || blocks <= 0) blocks = 2;
-        if (cfg->width == 5) blocks = std::max(1, std::min(blocks, kLanesPerCu5 / wg));
+        if (cfg->heuristic == SPZ_H_PDB666) blocks = std::max(1, std::min(blocks, kLanesPerCuPdb / wg));
         lanes = ctx->n_cu * blocks * wg;
     }
     lanes = (lanes + wg - 1) / wg * wg;
@@ -316,8 +307,7 @@ static int configure_lanes(spz_ctx *ctx) {
     size_t L = (size_t)lanes;
     int maxd = cfg->lds_stack_depth;
     if ((e = ctx->c_st.ensure(L * 4)) != hipSuccess || (e = ctx->c_rows.ensure(L * 4 * 5)) != hipSuccess ||
-        (e = ctx->c_root.ensure(L * 4 * 4)) != hipSuccess || (e = ctx->c_meta.ensure(L * 4)) != hipSuccess ||
-        (e = ctx->c_rmeta.ensure(L * 4)) != hipSuccess || (e = ctx->c_inst.ensure(L * 4)) != hipSuccess ||
+        (e = ctx->c_meta.ensure(L * 4)) != hipSuccess || (e = ctx->c_inst.ensure(L * 4)) != hipSuccess ||
         (e = ctx->c_cnt.ensure(L * 4)) != hipSuccess || (e = ctx->c_pdb.ensure(L * 4 * 10)) != hipSuccess ||
         (e = ctx->c_origin.ensure(L * 4)) != hipSuccess || (e = ctx->c_stack.ensure(L * (size_t)maxd * 2)) != hipSuccess)
         return fail(ctx, SPZ_E_HIP, "lane context allocation: %s", hipGetErrorString(e));
@@ -409,7 +399,7 @@ int spz_create(spz_ctx **out, const spz_config *cfg) try {
         pdb_geo_build(&ctx->geo_h);
         if ((e = ctx->geo_d.ensure(sizeof(PdbGeo))) != hipSuccess ||
             (e = hipMemcpy(ctx->geo_d.p, &ctx->geo_h, sizeof(PdbGeo), hipMemcpyHostToDevice)) != hipSuccess ||
-            (e = ctx->q_ctl.ensure(2 * kQCtl * 8)) != hipSuccess || (e = ctx->ctl.ensure(64 * 4)) != hipSuccess) {
+            (e = ctx->q_ctl.ensure(kQCtlWords * 8)) != hipSuccess || (e = ctx->ctl.ensure(64 * 4)) != hipSuccess) {
             rc = fail(ctx, SPZ_E_HIP, "context allocation: %s", hipGetErrorString(e));
             break;
         }
@@ -496,9 +486,7 @@ int spz_autotune(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_ite
         return SPZ_OK;
     };
     spz_config bc = base;
-    if (bc.round_budget <= 0)
-        bc.round_budget = default_round_budget(bc.heuristic, kLanesPerItem * (size_t)n * (size_t)std::max(1, bc.frontier_target) >=
-                                                                 (size_t)ctx->n_lanes);
+    if (bc.round_budget <= 0) bc.round_budget = kRoundSteps;
     double bms = 0;
     int count = 0;
     int rc = run(bc, &bms, false); // reference result (also warms the buffers)
@@ -548,19 +536,20 @@ const char *spz_last_error(spz_ctx *ctx) { return ctx ? ctx->err.c_str() : "null
 void spz_destroy(spz_ctx *ctx) {
     if (!ctx) return;
     DBuf *all[] = {&ctx->geo_d,       &ctx->pdb_compact[0], &ctx->pdb_compact[1], &ctx->pdb_direct,
-                   &ctx->c_st,         &ctx->c_rows,         &ctx->c_root,
-                   &ctx->c_meta,      &ctx->c_rmeta,        &ctx->c_inst,         &ctx->c_cnt,
+                   &ctx->c_st,         &ctx->c_rows,
+                   &ctx->c_meta,      &ctx->c_inst,         &ctx->c_cnt,
                    &ctx->c_pdb,       &ctx->c_stack,        &ctx->q,              &ctx->q_ctl,
                    &ctx->ctl,         &ctx->roots,          &ctx->L,              &ctx->it,
                    &ctx->cnt,         &ctx->pend,           &ctx->found,          &ctx->done,
-                   &ctx->opt,         &ctx->iter_counts,    &ctx->restart_list,   &ctx->frontier,
+                   &ctx->opt,         &ctx->iter_counts,    &ctx->frontier,
                    &ctx->nfront,      &ctx->topgen,         &ctx->top_goal,       &ctx->frozen,
                    &ctx->lvl[0],      &ctx->lvl[1],         &ctx->nlvl[0],        &ctx->nlvl[1],
                    &ctx->c_origin,    &ctx->load,           &ctx->samples,        &ctx->nsamp,
                    &ctx->pred,        &ctx->qpath,          &ctx->c_ipath,        &ctx->fpath,
                    &ctx->lpath[0],    &ctx->lpath[1],       &ctx->sol,            &ctx->sol_len,
                    &ctx->itn,         &ctx->drained,        &ctx->nlive,          &ctx->Lbase,
-                   &ctx->listed,      &ctx->want_next,      &ctx->dead,           &ctx->prof,
+                   &ctx->list,        &ctx->mail,           &ctx->mail_head,      &ctx->ticket,
+                   &ctx->mail_path,   &ctx->want_next,      &ctx->dead,           &ctx->prof,
                    &ctx->wtime};
     for (DBuf *b : all) b->release();
     ctx->dd_items.release();
@@ -783,6 +772,7 @@ static KParams base_params(spz_ctx *ctx, int n, int max_iters, int capl) {
     p.q = ctx->q.as<Item>();
     p.qmask = ctx->qcap - 1;
     p.q_ctl = ctx->q_ctl.as<unsigned long long>();
+    p.stop = (unsigned *)(p.q_ctl + kQStop);
     p.n_inst = n;
     p.max_iters = max_iters;
     p.mode = ctx->cfg.mode;
@@ -794,7 +784,6 @@ static KParams base_params(spz_ctx *ctx, int n, int max_iters, int capl) {
     p.dead = ctx->dead.as<int>();
     p.nlive = ctx->nlive.as<int>();
     p.Lbase = ctx->Lbase.as<int>();
-    p.listed = ctx->listed.as<int>();
     p.want_next = ctx->want_next.as<int>();
     p.cnt = ctx->cnt.as<unsigned long long>();
     p.pend = ctx->pend.as<unsigned>();
@@ -802,7 +791,6 @@ static KParams base_params(spz_ctx *ctx, int n, int max_iters, int capl) {
     p.done = ctx->done.as<int>();
     p.opt = ctx->opt.as<int>();
     p.iter_counts = ctx->iter_counts.as<unsigned long long>();
-    p.restart_list = ctx->restart_list.as<int>();
     p.ctl = ctx->ctl.as<unsigned>();
     p.frontier = ctx->frontier.as<Item>();
     p.nfront = ctx->nfront.as<unsigned>();
@@ -814,9 +802,7 @@ static KParams base_params(spz_ctx *ctx, int n, int max_iters, int capl) {
     p.prof = nullptr; // a solve turns the counters on (env SPZ_PROFILE)
     p.c_st = ctx->c_st.as<uint32_t>();
     p.c_rows = ctx->c_rows.as<uint32_t>();
-    p.c_root = ctx->c_root.as<uint32_t>();
     p.c_meta = ctx->c_meta.as<uint32_t>();
-    p.c_rmeta = ctx->c_rmeta.as<uint32_t>();
     p.c_inst = ctx->c_inst.as<uint32_t>();
     p.c_cnt = ctx->c_cnt.as<uint32_t>();
     p.c_origin = ctx->c_origin.as<uint32_t>();
@@ -928,20 +914,26 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     HIPCHK(ctx->roots.ensure(N * sizeof(Item)));
     HIPCHK(ctx->L.ensure(2 * N * 4));
     HIPCHK(ctx->itn.ensure(2 * N * 4));
-    HIPCHK(ctx->cnt.ensure(2 * N * 8));
-    HIPCHK(ctx->pend.ensure(2 * N * 4));
+    const size_t gstride = (2 * N + 31) / 32 * 32; // each group's part on lines of its own
+    HIPCHK(ctx->cnt.ensure(kGroups * gstride * 8));
+    HIPCHK(ctx->pend.ensure(kGroups * gstride * 4));
+    // lists, mailboxes and tickets of the waves
+    const size_t waves = lanes / 64, nblk = lanes / (size_t)ctx->wg;
+    const size_t list_n = next_pow2((nblk + kLists - 1) / kLists * ((size_t)ctx->wg / 64));
+    HIPCHK(ctx->list.ensure(kLists * list_n * 8));
+    HIPCHK(ctx->mail.ensure(waves * 64 * sizeof(Item)));
+    HIPCHK(ctx->mail_head.ensure(waves * kLine * 8));
+    HIPCHK(ctx->ticket.ensure(waves * 4));
     HIPCHK(ctx->found.ensure(2 * N * 4));
     HIPCHK(ctx->drained.ensure(2 * N * 4));
     HIPCHK(ctx->dead.ensure(2 * N * 4));
     HIPCHK(ctx->it.ensure(N * 4));
     HIPCHK(ctx->nlive.ensure(N * 4));
     HIPCHK(ctx->Lbase.ensure(N * 4));
-    HIPCHK(ctx->listed.ensure(N * 4));
     HIPCHK(ctx->want_next.ensure(N * 4));
     HIPCHK(ctx->done.ensure(N * 4));
     HIPCHK(ctx->opt.ensure(N * 4));
     HIPCHK(ctx->iter_counts.ensure(N * (size_t)max_iters * 8));
-    HIPCHK(ctx->restart_list.ensure(N * 4));
     HIPCHK(ctx->frontier.ensure(front_items * sizeof(Item)));
     HIPCHK(ctx->nfront.ensure(N * 4));
     HIPCHK(ctx->topgen.ensure(N * kFBins * 4));
@@ -962,8 +954,17 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
 
     KParams p = base_params(ctx, n, max_iters, capl);
     p.n_lanes = (int)lanes;
+    p.gstride = (int)gstride;
+    p.list = ctx->list.as<unsigned long long>();
+    p.list_mask = (unsigned)(list_n - 1);
+    p.n_blocks = (int)nblk;
+    p.block_waves = ctx->wg / 64;
+    p.mail = ctx->mail.as<Item>();
+    p.mail_head = ctx->mail_head.as<unsigned long long>();
+    p.ticket = ctx->ticket.as<unsigned>();
     // lookahead runs two iterations of an instance at once; the per-node
     // loads (load-based LB, training samples) describe one iteration at a time
+    p.want_load = p.lb == SPZ_LB_PREVLOAD || p.max_samples > 0 ? 1 : 0;
     p.lookahead = ctx->cfg.lookahead != 0 && ctx->cfg.lb_policy != SPZ_LB_PREVLOAD && p.max_samples == 0 ? 1 : 0;
 
     // solution paths: every queued item carries its moves from the root
@@ -977,6 +978,8 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
             return fail(ctx, SPZ_E_ARG, "record_paths needs at most 2^27 queue items a ring (smaller batch)");
         HIPCHK(ctx->qpath.ensure(2 * qcap * kPathWords * 4));
         HIPCHK(ctx->c_ipath.ensure((size_t)kPathWords * lanes * 4));
+        HIPCHK(ctx->mail_path.ensure(lanes * kPathWords * 4));
+        p.mail_path = ctx->mail_path.as<uint32_t>();
         HIPCHK(ctx->fpath.ensure(front_items * 8));
         for (int k = 0; k < 2; ++k) HIPCHK(ctx->lpath[k].ensure(front_items * 8));
         HIPCHK(ctx->sol.ensure(2 * N * kPathWords * 4)); // per iteration slot
@@ -1033,8 +1036,8 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     }
 
     if (getenv("SPZ_PROFILE") && atoi(getenv("SPZ_PROFILE")) > 0) {
-        HIPCHK(ctx->prof.ensure(64));
-        HIPCHK(hipMemsetAsync(ctx->prof.p, 0, 64, s));
+        HIPCHK(ctx->prof.ensure(lanes));
+        HIPCHK(hipMemsetAsync(ctx->prof.p, 0, lanes, s));
         p.prof = ctx->prof.as<unsigned long long>();
         // with SPZ_WAVE_TIMES=r: every wave's start and end clock in round r
         if (getenv("SPZ_WAVE_TIMES")) {
@@ -1052,51 +1055,47 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     HIPCHK(hipStreamSynchronize(s));
     ctx->stats[10] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_split).count();
 
-    // per-instance iteration state: every instance on the restart list with
-    // no iteration started (k_restart starts iteration 0)
+    // per-instance iteration state: every instance with no iteration
+    // started (k_restart starts iteration 0)
     {
-        std::vector<int> Lh(N), nog(2 * N, kNoGoal), neg(N, -1), list(N), ones(N, 1);
+        std::vector<int> Lh(N), nog(2 * N, kNoGoal), neg(N, -1);
         for (int i = 0; i < n; ++i) {
             Lh[i] = meta_h(roots[i].meta);
-            list[i] = i;
         }
         HIPCHK(hipMemcpyAsync(ctx->Lbase.p, Lh.data(), N * 4, hipMemcpyHostToDevice, s));
         HIPCHK(hipMemsetAsync(ctx->L.p, 0, 2 * N * 4, s));
         HIPCHK(hipMemsetAsync(ctx->itn.p, 0, 2 * N * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->cnt.p, 0, 2 * N * 8, s));
-        HIPCHK(hipMemsetAsync(ctx->pend.p, 0, 2 * N * 4, s));
+        HIPCHK(hipMemsetAsync(ctx->cnt.p, 0, kGroups * gstride * 8, s));
+        HIPCHK(hipMemsetAsync(ctx->pend.p, 0, kGroups * gstride * 4, s));
+        HIPCHK(hipMemsetAsync(ctx->list.p, 0, kLists * list_n * 8, s));
+        HIPCHK(hipMemsetAsync(ctx->mail_head.p, 0, waves * kLine * 8, s));
+        HIPCHK(hipMemsetAsync(ctx->ticket.p, 0, waves * 4, s));
         HIPCHK(hipMemsetAsync(ctx->drained.p, 0, 2 * N * 4, s));
         HIPCHK(hipMemsetAsync(ctx->dead.p, 0, 2 * N * 4, s));
         HIPCHK(hipMemcpyAsync(ctx->found.p, nog.data(), 2 * N * 4, hipMemcpyHostToDevice, s));
         HIPCHK(hipMemsetAsync(ctx->it.p, 0, N * 4, s));
         HIPCHK(hipMemsetAsync(ctx->nlive.p, 0, N * 4, s));
-        HIPCHK(hipMemcpyAsync(ctx->listed.p, ones.data(), N * 4, hipMemcpyHostToDevice, s));
         HIPCHK(hipMemsetAsync(ctx->want_next.p, 0, N * 4, s));
         HIPCHK(hipMemsetAsync(ctx->done.p, 0, N * 4, s));
         HIPCHK(hipMemcpyAsync(ctx->opt.p, neg.data(), N * 4, hipMemcpyHostToDevice, s));
         HIPCHK(hipMemsetAsync(ctx->iter_counts.p, 0, N * (size_t)max_iters * 8, s));
-        HIPCHK(hipMemcpyAsync(ctx->restart_list.p, list.data(), N * 4, hipMemcpyHostToDevice, s));
         unsigned ctl[64];
         memset(ctl, 0, sizeof ctl);
-        ctl[0] = (unsigned)n; // restart list length
         ctl[1] = (unsigned)n; // active instances
-        const bool full = lanes >= (size_t)ctx->n_lanes;
-        int big = ctx->cfg.round_budget > 0 ? ctx->cfg.round_budget : default_round_budget(heur, full);
+        const int budget = ctx->cfg.round_budget > 0 ? ctx->cfg.round_budget : kRoundSteps;
         // a round ends after its step budget or its time limit, whichever
         // comes first
-        const int rt = ctx->cfg.round_time_us == 0 ? default_round_time_us(heur, full) : ctx->cfg.round_time_us;
+        const int rt = ctx->cfg.round_time_us == 0 ? kRoundTimeUs : ctx->cfg.round_time_us;
         p.round_ticks = (rt > 0 && ctx->wall_ticks_per_us > 0)
                             ? (unsigned long long)(rt * ctx->wall_ticks_per_us) : 0ull;
-        ctl[9] = (unsigned)big;
-        // rounds while the queue cannot keep half the lanes busy: short, so
-        // that donations refill idle lanes soon (measured on MI355X, 32 / 64
-        // / 128 / 256 / 512 steps: 100 40-move 15-puzzles 5270 / 6300 /
-        // 7270 / 7220 / 6040 instances/s, one random 15-puzzle per launch
-        // 44.7 / 45.2 / 46.5 / 45.1 / 39.4, the PDB search level)
-        ctl[10] = (unsigned)std::min(big, kShortRoundSteps);
-        ctl[5] = ctl[10];
+        p.turn_ticks = ctx->wall_ticks_per_us > 0 ? (unsigned long long)(kTurnUs * ctx->wall_ticks_per_us) : 1ull << 40;
+        ctl[5] = (unsigned)budget;
         HIPCHK(hipMemcpyAsync(ctx->ctl.p, ctl, sizeof ctl, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemsetAsync(ctx->q_ctl.p, 0, 2 * kQCtl * 8, s));
+        unsigned long long qc[kQCtlWords];
+        memset(qc, 0, sizeof qc);
+        for (int r = 0; r < 2; ++r)
+            for (int x = 0; x < kGroups; ++x) qc[kQHead + r * kQRing + x * kLine] = (unsigned long long)x;
+        HIPCHK(hipMemcpyAsync(ctx->q_ctl.p, qc, sizeof qc, hipMemcpyHostToDevice, s));
         HIPCHK(hipMemsetAsync(ctx->c_st.p, 0, lanes * 4, s));
         HIPCHK(hipStreamSynchronize(s));
     }
@@ -1119,9 +1118,8 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
         for (auto &x : ev) HIPCHK(hipEventCreate(&x));
     double round_ms = 0;
     long timed = 0;
-    unsigned *h_ctl = nullptr; // pinned: 64 control words, then the two rings' queue counters
-    HIPCHK(hipHostMalloc((void **)&h_ctl, 64 * 4 + 2 * kQCtl * 8, hipHostMallocDefault));
-    unsigned long long *h_qc = (unsigned long long *)(h_ctl + 64);
+    unsigned *h_ctl = nullptr; // pinned: 64 control words
+    HIPCHK(hipHostMalloc((void **)&h_ctl, 64 * 4, hipHostMallocDefault));
     int rc = SPZ_OK;
     long rounds = 0;
 
@@ -1138,7 +1136,6 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
             if (e == hipSuccess) e = launch_control(p, s);
         }
         if (e == hipSuccess) e = hipMemcpyAsync(h_ctl, ctx->ctl.p, 64 * 4, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipMemcpyAsync(h_qc, ctx->q_ctl.p, 2 * kQCtl * 8, hipMemcpyDeviceToHost, s);
         return e;
     };
     // hipGraph: the period is captured once and replayed; the kernels read
@@ -1181,24 +1178,24 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
             break;
         }
         if (trace) {
-            fprintf(stderr, "spz poll %ld: %.1f ms, busy lanes %u, active instances %u, queued %llu", rounds,
+            fprintf(stderr, "spz poll %ld: %.1f ms, busy lanes %u, active instances %u, queued %u", rounds,
                     std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_rounds).count(),
-                    h_ctl[12], h_ctl[1],
-                    (unsigned long long)(h_qc[2] - h_qc[0] + h_qc[kQCtl + 2] - h_qc[kQCtl]));
-            unsigned long long pf[4];
-            if (p.prof && hipMemcpy(pf, p.prof, sizeof pf, hipMemcpyDeviceToHost) == hipSuccess)
-                fprintf(stderr, ", lane-steps idle %llu expanding %llu popping %llu", pf[0], pf[1], pf[2]);
+                    64u * h_ctl[12], h_ctl[1], h_ctl[20]);
             fputc('\n', stderr);
+        }
+        if (h_ctl[3] & 2u) {
+            rc = fail(ctx, SPZ_E_STALL, "a word of the work lists was never written");
+            break;
         }
         if (h_ctl[3]) {
             rc = fail(ctx, SPZ_E_CAPACITY, "work queue overflow: raise queue_items (now %zu items)", ctx->qcap);
             break;
         }
         if (h_ctl[1] == 0) break;
-        // no lane busy at the end of the last round and nothing queued (a
+        // no wave with work at the end of the last round and nothing queued (a
         // finished iteration has queued its next one by now): no work can
         // appear any more
-        stalled = (h_qc[2] == h_qc[0] && h_qc[kQCtl + 2] == h_qc[kQCtl] && h_ctl[12] == 0) ? stalled + 1 : 0;
+        stalled = (h_ctl[20] == 0 && h_ctl[12] == 0) ? stalled + 1 : 0;
         if (stalled > 2) {
             rc = fail(ctx, SPZ_E_STALL, "search stalled with %u active instances", h_ctl[1]);
             break;
@@ -1257,9 +1254,13 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
         for (int i = 0; i < n; ++i) ctx->paths_slot[i] = its[i] & 1;
     }
     if (p.prof) {
-        unsigned long long pf[7];
-        HIPCHK(hipMemcpy(pf, p.prof, sizeof pf, hipMemcpyDeviceToHost));
-        for (int k = 0; k < 7; ++k) ctx->stats[16 + k] = (double)pf[k];
+        std::vector<unsigned long long> pf(lanes / 8); // 8 words a wave
+        HIPCHK(hipMemcpy(pf.data(), p.prof, lanes, hipMemcpyDeviceToHost));
+        for (int k = 0; k < 7; ++k) {
+            double t = 0;
+            for (size_t w = 0; w < lanes / 64; ++w) t += (double)pf[w * 8 + k];
+            ctx->stats[16 + k] = t;
+        }
     }
     if (p.wtime) {
         // end times of the recorded round's waves after its first start, on

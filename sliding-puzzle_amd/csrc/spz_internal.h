@@ -21,12 +21,27 @@ template <int W> __device__ __forceinline__ int dir_cell(int d) {
     return dir_byte(((uint32_t)W << 24) | 0x00FF0100u | (uint32_t)(uint8_t)(-W), d);
 }
 
-// Lane states of the DFS engine.
-// lane states; ST_DESC (children f-tested, descent into the first passing one
-// pending) never outlives a round
-constexpr int kQCtl = 16; // u64 stride between the two rings' counters
+// Queue-control words (u64), every group of them on 128-byte lines of its own:
+// atomics on one address are served one after another, 12 ns each.  Per ring r
+// at r * kQRing: tail and limit, then a head for each of the kGroups groups;
+// then the stop word; then the kLists lists of waiting waves; then each
+// group's count of waves started.
+constexpr int kGroups = 8;
+constexpr int kLine = 16;
+constexpr int kQTail = 0, kQHead = kLine, kQRing = (1 + kGroups) * kLine;
+constexpr int kQStop = 2 * kQRing, kQList = kQStop + kLine;
+constexpr int kLists = 64;
+constexpr int kQStart = kQList + kLists * kLine;
+constexpr int kQCtlWords = kQStart + kGroups * kLine;
 
-enum : int { ST_IDLE = 0, ST_FRESH = 1, ST_POP = 2, ST_DRAINED = 3, ST_DESC = 4 };
+// Lane states of the DFS engine.  Searching: FRESH (a node to expand), POP (a
+// subtree done, back up), DESC (children f-tested, the descent into the first
+// passing one pending).  Waiting for the end of a block of steps: DONE (the
+// item's subtree is done), FULL (passing children and no stack level left),
+// GOAL (a goal to record).  Only IDLE, FRESH and POP outlive a round, and GOAL
+// as a goal recorded but not expanded yet.
+enum : int { ST_IDLE = 0, ST_FRESH = 1, ST_POP = 2, ST_DESC = 3, ST_DONE = 4, ST_FULL = 5, ST_GOAL = 6 };
+__host__ __device__ inline bool searching(int st) { return (unsigned)(st - 1) < 3u; }
 
 constexpr int kMaxIters = 128;      // threshold iterations kept per instance
 constexpr int kFBins = 256;         // f-value histogram bins of the top tree
@@ -71,12 +86,23 @@ __host__ __device__ inline int meta_prev(uint32_t m) { return (int)(m >> 24); }
 struct KParams {
     // work queue: two rings of qcap (power of two) items each, ring 0 for
     // the current iterations, ring 1 for lookahead iterations (ring r at
-    // q + r * qcap); q_ctl[kQCtl*r + 0..2] = head, limit, tail of ring r
-    // (each ring's counters on a 128-byte line of their own: every idle
-    // wave's grab is an atomic on them)
+    // q + r * qcap); q_ctl: kQCtlWords control words (above)
     Item *q;
     unsigned long long qmask;
     unsigned long long *q_ctl;
+    unsigned *stop;              // 1: the running round is to end
+
+    // waves without work: the lists of them (entry: position + 1,
+    // wave), and a mailbox a wave: 64 items, the head word (list position + 1
+    // it answers, items) on a line of its own, and the position + 1 the wave
+    // waited at when it left the last round
+    unsigned long long *list;    // [kLists][list_mask + 1]
+    unsigned list_mask;
+    int n_blocks, block_waves;   // workgroups of a round, waves of a workgroup
+    Item *mail;                  // [waves][64]
+    unsigned long long *mail_head; // [waves][kLine]
+    unsigned *ticket;            // [waves]
+    uint32_t *mail_path;         // [waves][64][kPathWords], or null
 
     // instances
     int n_inst;
@@ -89,32 +115,29 @@ struct KParams {
     // also what items and lanes carry as their instance.
     int *L;                      // [2 n_inst] threshold of the slot's iteration
     int *itn;                    // [2 n_inst] iteration index held by the slot
-    unsigned long long *cnt;     // [2 n_inst] count of the slot's iteration
-    unsigned int *pend;          // [2 n_inst] its items not finished
+    int gstride;                 // entries of a group in cnt and pend
+    unsigned long long *cnt;     // [kGroups][gstride] count of the slot's iteration, in parts
+    unsigned int *pend;          // [kGroups][gstride] its queued items and the waves searching it
     int *found;                  // [2 n_inst] min goal depth (kNoGoal if none)
-    int *drained;                // [2 n_inst] 1 once pend reached zero
+    int *drained;                // [2 n_inst] 1 once pend's parts add up to zero
     int *dead;                   // [2 n_inst] 1: the slot's work is not needed
                                  // (instance done, or a goal in the older slot)
     int *it;                     // [n_inst] current (oldest unresolved) iteration
     int *nlive;                  // [n_inst] iterations started, not resolved (0-2)
     const int *Lbase;            // [n_inst] threshold of iteration 0 (h of the root)
-    int *listed;                 // [n_inst] 1 while on the restart list
     int *want_next;              // [n_inst] lookahead requested for the next restart
     int lookahead;               // 1: start iteration it+1 while `it` drains
     int *done;
     int *opt;
     unsigned long long *iter_counts; // [n_inst][max_iters]
-    int *restart_list;
-    unsigned int *ctl;           // 0 n_restart, 1 active, 2 busy, 3 queue overflow,
-                                 // 4 donate_per_lane, 5 budget, 6 rounds,
-                                 // 7 donated, 8 overflow exports, 9/10 big/small
-                                 // budget, 12 busy at last round end,
-                                 // 13 lookahead iterations started,
-                                 // 14/15 frontier nodes re-split / the items
-                                 // they became,
-                                 // 19 donate_per_lane of lanes on lookahead
-                                 // iterations, 34 how many are busy (own
-                                 // cache line: every wave adds to it)
+    unsigned int *ctl;           // 1 active, 3 queue error (1: full, 2: a word
+                                 // never written), 4 items a wave takes at
+                                 // once, 5 step budget, 6 rounds, 7 nodes given
+                                 // to waiting waves, 8 overflow exports, 12
+                                 // waves with work at the last round's end, 13
+                                 // lookahead iterations started, 14/15 frontier
+                                 // nodes re-split / the items they became, 20
+                                 // queued items
 
     // top tree of the root split (per instance)
     const Item *frontier;        // [n_inst][capl]
@@ -126,6 +149,7 @@ struct KParams {
     // load balancing: nodes generated below each frontier node in the
     // current iteration, dispatch policy, learned predictions, sample log
     unsigned long long *load;    // [n_inst][capl]
+    int want_load;               // 1: the loads are read (previous-load order, sample log)
     int lb;                      // 0 frontier order, 1 learned, 2 previous load
     int resplit;                 // heavy-node re-split factor (0: off)
     const float *pred;           // [n_inst][capl][kPredK] predicted log2(1+load)
@@ -136,15 +160,14 @@ struct KParams {
     // lane contexts, structure of arrays over n_lanes lanes
     int n_lanes;
     int maxd;          // LDS stack levels per lane in use
-    unsigned long long *prof; // null, or [4]: lane-steps idle, expanding, popping only, wave-steps
-    unsigned long long round_ticks; // big rounds end this many wall-clock ticks after a wave's start (0: off)
+    unsigned long long *prof; // null, or [waves][8]: lane-steps idle, expanding, popping only, wave-steps, table reads
+    unsigned long long turn_ticks;  // waves without work, together, wait this long times the waves before a round ends
+    unsigned long long round_ticks; // rounds end this many wall-clock ticks after a wave's start (0: off)
     unsigned long long *wtime; // null, or [2][waves]: start and end clock of each wave in round wtime_round
     unsigned wtime_round;
     uint32_t *c_st;    // state | sp<<8
     uint32_t *c_rows;  // [5][n_lanes]
-    uint32_t *c_root;  // [4][n_lanes] packed item root
     uint32_t *c_meta;  // blank,g,h,prev of the current node
-    uint32_t *c_rmeta; // meta of the item root
     uint32_t *c_inst;
     uint32_t *c_cnt;
     uint32_t *c_origin; // frontier node the lane's item descends from

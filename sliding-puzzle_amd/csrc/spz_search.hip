@@ -35,6 +35,23 @@ constexpr int kPops = 2;
 // sibling-value cache of the PDB search: per lane, the deepest kSibLevels
 // stack levels (ring, tagged with the level); see k_round
 constexpr int kSibLevels = 8;
+// steps between two looks of a wave at its idle lanes
+constexpr int kShareSteps = 8;
+// idle lanes of a wave that make sharing worth its cost
+constexpr int kShareMin = 4;
+// a node given to another lane of the wave, or to another wave, lies at least
+// this many levels above the giver's own
+constexpr int kGiveLevels = 2;
+constexpr int kFeedLevels = 4;
+// looks at a word another wave is about to write before the solve is given up
+// (tens of milliseconds; the writer is microseconds away)
+constexpr int kWriteSpins = 1 << 16;
+// naps of a wave waiting for work in one round at most (a round has its own
+// end; this bounds the wait whatever happens)
+constexpr int kMaxNaps = 1 << 16;
+// blocks of steps of a wave that starts late
+constexpr int kLateBlocks = 64;
+
 
 
 __device__ __forceinline__ uint64_t lanemask_lt() {
@@ -50,17 +67,70 @@ __device__ __forceinline__ unsigned long long shfl_u64(unsigned long long v, int
     return ((unsigned long long)hi << 32) | lo;
 }
 
-// The last item of a slot's iteration has ended.  Called by exactly one lane
-// (the one whose pend decrement reached zero): it marks the slot and puts the
-// instance on the restart list; k_restart resolves the instance's iterations
-// in order between rounds.
-__device__ void iteration_drained(const KParams &p, int isl) {
-    p.drained[isl] = 1;
-    const int inst = isl >> 1;
-    if (atomicExch(&p.listed[inst], 1) == 0) {
-        const unsigned k = atomicAdd(&p.ctl[0], 1u);
-        p.restart_list[k] = inst;
-    }
+__device__ __forceinline__ unsigned long long shfl_xor_u64(unsigned long long v, int off) {
+    const uint32_t lo = __shfl_xor((uint32_t)v, off), hi = __shfl_xor((uint32_t)(v >> 32), off);
+    return ((unsigned long long)hi << 32) | lo;
+}
+
+// Words that waves of other dies read or write while a round runs.  Relaxed
+// agent-scope accesses: no cache is written back or invalidated, which would
+// also drop the pattern-database lines.
+template <class T> __device__ __forceinline__ T ld_agent(const T *a) {
+    return __hip_atomic_load(a, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <class T> __device__ __forceinline__ void st_agent(T *a, T v) {
+    __hip_atomic_store(a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// what the wave stored so far has arrived before what it stores next
+__device__ __forceinline__ void arrival_fence() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0); // all counters: vector stores and atomics included
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ unsigned uniform(unsigned v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ unsigned long long uniform(unsigned long long v) {
+    return ((unsigned long long)uniform((unsigned)(v >> 32)) << 32) | uniform((unsigned)v);
+}
+
+// The waves of a round form kGroups groups by workgroup number (workgroups go
+// to the 8 dies in turn, so a group is a die's), each with words of its own
+// for what every wave changes.
+__device__ __forceinline__ unsigned group_of(unsigned block) { return block & (kGroups - 1); }
+// Waves waiting for work are on kLists lists, by workgroup number too (so the
+// waves of a list are a die's): a list's word is changed by compare-and-swap,
+// of which one in the time of a look and a swap succeeds, a microsecond, and
+// 8192 waves on 8 lists could not be fed at that rate.
+__device__ __forceinline__ unsigned list_of(unsigned block) { return block & (kLists - 1); }
+__device__ __forceinline__ unsigned list_waves(const KParams &p, unsigned x) {
+    return ((unsigned)p.n_blocks + kLists - 1 - x) / kLists * (unsigned)p.block_waves;
+}
+// a list's waves: pushed onto it (high half) and not taken off it by a wave
+// with work to give (low half)
+__device__ __forceinline__ unsigned waiting(unsigned long long w) { return (unsigned)(w >> 32) - (unsigned)w; }
+__device__ __forceinline__ unsigned wave_sum(unsigned n) {
+    for (int off = 1; off < 64; off <<= 1) n += __shfl_xor(n, off);
+    return uniform(n);
+}
+// both by a whole wave
+__device__ __forceinline__ unsigned idle_waves(const KParams &p) {
+    return wave_sum(waiting(ld_agent(&p.q_ctl[kQList + (threadIdx.x & 63u) * kLine])));
+}
+__device__ __forceinline__ unsigned started_waves(const KParams &p) {
+    const unsigned lane = threadIdx.x & 63u;
+    return wave_sum(lane < (unsigned)kGroups ? (unsigned)ld_agent(&p.q_ctl[kQStart + lane * kLine]) : 0u);
+}
+
+// Items and waves of slot isl not finished, and its node count: each group
+// keeps its part (a group's part alone may be negative)
+__device__ __forceinline__ unsigned slot_pend(const KParams &p, int isl) {
+    unsigned n = 0;
+    for (int x = 0; x < kGroups; ++x) n += p.pend[x * p.gstride + isl];
+    return n;
+}
+__device__ __forceinline__ unsigned long long slot_count(const KParams &p, int isl) {
+    unsigned long long n = 0;
+    for (int x = 0; x < kGroups; ++x) n += p.cnt[x * p.gstride + isl];
+    return n;
 }
 
 // A goal in slot isl makes a newer iteration in the other slot unnecessary
@@ -97,18 +167,21 @@ __device__ __forceinline__ void put_item(const KParams &p, int r, unsigned long 
     p.q[q_slot(p, r, pos)] = it;
 }
 
-// Reserve k slots at the tail of ring r (counters q_ctl[kQCtl*r + 0..2]:
-// head, limit, tail).  Items in [min(head, limit), tail) are not taken yet; a tail
-// more than the ring's capacity past them would overwrite some, so that sets
-// the error word (ctl[3]) and the host fails the solve with SPZ_E_CAPACITY
-// rather than return counts from a corrupt queue.  head is read as it
-// stands, possibly behind, which only makes the test stricter.
+// Position i of a ring belongs to group i % kGroups, whose head word holds its
+// next position not taken.  Reserve k positions at the tail of ring r; a tail
+// more than the ring's capacity past the oldest item not taken would
+// overwrite it, so that sets the error word (ctl[3]) and the host fails the
+// solve with SPZ_E_CAPACITY rather than return counts from a corrupt queue.
 __device__ __forceinline__ unsigned long long q_reserve(const KParams &p, int r, unsigned long long k) {
-    unsigned long long *c = p.q_ctl + kQCtl * r;
-    const unsigned long long pos = atomicAdd(&c[2], k);
-    const unsigned long long h = *(volatile unsigned long long *)&c[0], lim = c[1];
-    const unsigned long long live_from = h < lim ? h : lim;
-    if (pos + k - live_from > p.qmask + 1ull) atomicOr(&p.ctl[3], 1u);
+    unsigned long long *c = p.q_ctl + kQTail + r * kQRing;
+    const unsigned long long pos = atomicAdd(&c[0], k);
+    unsigned long long oldest = c[1]; // the limit: taken positions end there
+#pragma unroll 1
+    for (int x = 0; x < kGroups; ++x) {
+        const unsigned long long h = ld_agent(&p.q_ctl[kQHead + r * kQRing + x * kLine]);
+        oldest = h < oldest ? h : oldest;
+    }
+    if (pos + k - oldest > p.qmask + 1ull) atomicOr(&p.ctl[3], 1u);
     return pos;
 }
 
@@ -131,6 +204,13 @@ __device__ __forceinline__ void path_copy(const uint32_t *sb, uint32_t so, uint3
 #pragma unroll 1
     for (uint32_t k = 0; k < (uint32_t)kPathWords; ++k) db[dof + k * dstr] = sb[so + k * ss];
 }
+// the same in a mail, which a wave of another die reads
+__device__ __forceinline__ void path_put_agent(uint32_t *path, int i, int d) {
+    if (i >= kPathMax) return;
+    uint32_t *x = &path[i >> 4];
+    const int sh = 2 * (i & 15);
+    st_agent(x, (ld_agent(x) & ~(3u << sh)) | ((uint32_t)d << sh));
+}
 __device__ __forceinline__ void path_from_u64(unsigned long long v, uint32_t *db, uint32_t dof) {
     db[dof] = (uint32_t)v;
     db[dof + 1] = (uint32_t)(v >> 32);
@@ -146,38 +226,45 @@ __device__ __forceinline__ void pos_from_item(Pos<W, HEUR, BD> &s, const uint32_
     init_heur<W, HEUR>(s, P, meta);
 }
 
-// register copy of a lane position (the search kernel's 5x5 board is in LDS)
-template <int W, int HEUR, class BD>
-__device__ __forceinline__ Pos<W, HEUR> reg_pos(const Pos<W, HEUR, BD> &s) {
-    Pos<W, HEUR> c;
-    if constexpr (W == 5)
-        c.bd = s.bd.regs();
-    else
-        c.bd = s.bd;
-    if constexpr (W == 4) {
-        c.bl = s.bl;
-    } else {
-        c.br = s.br;
-        c.bc = s.bc;
-    }
-    c.hs = s.hs;
-    return c;
+// The kernel's arguments, read again where they are used: held from the
+// kernel's start they would not fit the scalar registers and be spilled to
+// vector ones, which the search needs.
+__device__ __forceinline__ const KParams &params_again() {
+    auto *a = (const __attribute__((address_space(4))) KParams *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(a));
+    return *(const KParams *)a;
 }
 
 // ---------------------------------------------------------------------------
-// k_round: every lane is an independent DFS engine.  A round runs `budget`
-// wave-uniform steps; each step a lane either takes an item, pops one stack
-// level, or expands the node it stands on.  Busy lanes keep their state
-// across rounds in the c_* context arrays.  The stack holds one byte per
-// level: the move taken from that level (2 bits) and the moves still to
-// try there (4-bit mask of children that passed the f-test).
+// k_round: a wave is a team of 64 depth-first search engines, one a lane.  A
+// round runs wave-uniform steps; each step a lane pops up to kPops stack
+// levels or makes one move down, and expands the node it stands on.  Every
+// kShareSteps steps the wave settles what the steps left (items done, goals,
+// full stacks) and evens out its work: its idle lanes take the shallowest
+// open nodes of its busy ones, by lane exchange.  A wave without any work
+// takes items of the queue, one where there are fewer items than waves, and
+// leaves the round when there are none; the round ends when the waves that
+// left have waited as long, together, as a new round costs, and the working
+// waves then queue nodes for them.  Busy lanes keep their state across rounds
+// in the c_* context arrays.
+//
+// What bounds the sharing is that atomics on one address are served one after
+// another, 12 ns each on MI355X whatever the die (83 M/s; loads of a line that
+// atomics change are no faster, loads of an unchanged line 16 G/s).  A single
+// search has one node count and one count of pending items, so both are kept
+// by the wave: it counts as one pending unit of an instance however many of
+// its lanes search it, and adds their node counts once, when that ends.
+//
+// The stack holds one byte per level (PDB: two): the move taken from that
+// level (2 bits) and the moves still to try there (4-bit mask of children
+// that passed the f-test).
 // The 15-puzzle kernel is held to 64 VGPRs (8 waves per SIMD: its LDS use is
-// small, and it fits without scratch); the 24-puzzle kernels are bounded by
-// their LDS (stack and boards) at 3 waves per SIMD.
-template <int W, int HEUR>
-__global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, const PdbGeo *geo_g) {
+// small); the 24-puzzle kernels are bounded by their LDS (stack and boards)
+// at 3 waves per SIMD.  PROF: with the lane-state counters (SPZ_PROFILE).
+template <int W, int HEUR, bool PROF>
+__global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, const PdbGeo *geo_g) {
     // every wave of the grid starts within microseconds of the others
-    const long long t_start = (p.wtime || p.round_ticks) ? wall_clock64() : 0;
+    const long long t_start = wall_clock64();
     const int MAXD = p.maxd;
     extern __shared__ uint8_t lds[];
     __shared__ PdbGeo geo_s;
@@ -202,14 +289,21 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, cons
         __syncthreads();
     }
 
-    const unsigned long long limit = p.q_ctl[1], limit1 = p.q_ctl[kQCtl + 1];
-    // a ring seen empty stays empty for the round (heads only grow): the
-    // wave then skips its atomic
-    bool q0_empty = p.q_ctl[0] >= limit, q1_empty = !p.lookahead || p.q_ctl[kQCtl] >= limit1;
-    const int budget = (int)p.ctl[5];
+    const unsigned grp = group_of(blockIdx.x);
+    const int wave_id = gl >> 6;
+    if (lane == 0) atomicAdd(&p.q_ctl[kQStart + grp * kLine], 1ull);
+    // a wave that starts when the round is already to end (the device did not
+    // hold all workgroups at once) runs a while all the same
+    const int least = uniform(ld_agent(p.stop)) ? kLateBlocks : 1;
+    // per ring the groups whose part of the queue the wave has seen empty
+    // (it stays empty for the round: heads only grow)
+    unsigned empty0 = 0, empty1 = p.lookahead ? 0u : (1u << kGroups) - 1u;
+    const int take_most = (int)p.ctl[4];
+    int steps_left = (int)p.ctl[5];
     const int mode = p.mode;
+    const unsigned n_waves = (unsigned)NL >> 6;
 
-    uint32_t stw = p.c_st[gl];
+    const uint32_t stw = p.c_st[gl];
     int st = (int)(stw & 0xff);
     int sp = (int)(stw >> 8);
     // stack levels, then (width 5) the lanes' boards
@@ -235,24 +329,22 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, cons
     }
     s.set_cell(0);
     s.hs.h = 0;
-    uint32_t root[4] = {0, 0, 0, 0};
-    uint32_t rmeta = 0;
-    // inst is the item's slot index (instance * 2 + iteration slot)
+    // inst is the item's slot index (instance * 2 + iteration slot); an idle
+    // lane keeps the one its node count belongs to
     int g = 0, prev = DIR_NONE, inst = 0, L = 0;
-    uint32_t cnt = 0, origin = 0;
+    uint32_t cnt = 0;
 
+    // a saved GOAL is a goal node recorded already, to be expanded
+    bool goal_seen = st == ST_GOAL;
+    if (goal_seen) st = ST_FRESH;
     if (st == ST_FRESH || st == ST_POP) {
         uint32_t b[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) b[k] = p.c_rows[k * NL + gl];
         s.bd.unpack(b);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) root[k] = p.c_root[k * NL + gl];
         uint32_t m = p.c_meta[gl];
-        rmeta = p.c_rmeta[gl];
         inst = (int)p.c_inst[gl];
         cnt = p.c_cnt[gl];
-        origin = p.c_origin[gl];
         s.set_cell(meta_blank(m));
         g = meta_g(m);
         prev = meta_prev(m);
@@ -273,24 +365,48 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, cons
             s.hs.B = (int)((v1 & 0xff) + ((v1 >> 8) & 0xff) + ((v1 >> 16) & 0xff) + (v1 >> 24));
         }
         L = p.L[inst];
-        if (p.lookahead && p.dead[inst]) sp = 0, st = ST_POP; // unwinds and finishes next step
-        for (int k = 0; k < sp; ++k) stk[k * sstride] = cstk[(size_t)k * NL + gl];
+        // dropped: unwinds and finishes next step
+        if (p.lookahead && p.dead[inst]) sp = 0, st = ST_POP, goal_seen = false;
+        // eight levels' loads in flight at once (the tail re-reads the last one)
+#pragma unroll 1
+        for (int k = 0; k < sp; k += 8) {
+            ST e[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) e[j] = cstk[(size_t)min(k + j, sp - 1) * NL + gl];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) stk[min(k + j, sp - 1) * sstride] = e[j];
+        }
     } else {
         st = ST_IDLE;
     }
 
+    // the lane's node count stays with the instance it was counted for: on a
+    // change of instance it is added there
+    auto relabel = [&](int to) {
+        const KParams &p = params_again();
+        if (cnt && inst != to) {
+            atomicAdd(&p.cnt[grp * p.gstride + inst], (unsigned long long)cnt);
+            cnt = 0;
+        }
+        inst = to;
+    };
+
+    // an item becomes the lane's; the PDB lookups of its board are computed
+    // for all lanes that start one together (init)
+    bool init = false;
     auto start_item = [&](const Item &it) {
-        pos_from_item<W, HEUR>(s, it.b, it.meta, P);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) root[k] = it.b[k];
-        rmeta = it.meta;
-        inst = (int)it.inst;
-        origin = it.x1;
+        const KParams &p = params_again();
+        s.bd.unpack(it.b);
+        s.set_cell(meta_blank(it.meta));
+        s.hs.h = meta_h(it.meta);
+        init = true;
+        relabel((int)it.inst);
+        if (p.want_load) p.c_origin[gl] = it.x1; // read when the item ends or is given away
         g = meta_g(it.meta);
         prev = meta_prev(it.meta);
         L = p.L[inst];
         sp = 0;
-        cnt = 0;
+        goal_seen = false;
         st = ST_FRESH;
         if (mode == 1 && p.found[inst] != kNoGoal) st = ST_POP; // first-solution: abandon
         if (p.lookahead && p.dead[inst]) st = ST_POP;
@@ -314,11 +430,438 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, cons
     // path of a new queue item: the item root's path, the moves of stack
     // levels 0..nst-1, then move last_d
     auto item_path = [&](int r, unsigned long long qpos, int nst, int last_d) {
+        const KParams &p = params_again();
         const uint32_t qo = (uint32_t)q_slot(p, r, qpos) * kPathWords;
         path_copy(p.c_ipath, (uint32_t)gl, (uint32_t)NL, p.qpath, qo, 1);
-        const int gr = meta_g(rmeta);
+        const int gr = g - sp; // depth of the item's root
         for (int k = 0; k < nst; ++k) path_put(p.qpath, qo, 1, gr + k, SE::dir(stk[k * sstride]));
         path_put(p.qpath, qo, 1, gr + nst, last_d);
+    };
+    // moves that give work away: the board, the blank and (Manhattan) h; for
+    // the PDB the board alone, as the lane that takes the node computes its
+    // lookups from the board
+    auto step_down = [&](int d) -> uint32_t {
+        if constexpr (HEUR == 1) {
+            move_board_only(s, d);
+            return 0u;
+        } else {
+            return move_md(s, d);
+        }
+    };
+    auto step_back = [&](int d, uint32_t nearer) {
+        if constexpr (HEUR == 1)
+            move_board_only(s, 3 - d);
+        else
+            unmove_md(s, d, nearer);
+    };
+    // back up to the node whose child the lane's path enters at level lev
+    auto go_back = [&](int lev) {
+#pragma unroll 1
+        for (int k = sp - 1; k >= lev; --k) {
+            const uint32_t e = stk[k * sstride];
+            step_back(SE::dir(e), SE::vals(e));
+        }
+    };
+    // where the lane stands, kept while it goes back up its path: board, blank
+    // and h (the PDB lookups do not move with step_back and step_down)
+    struct Here {
+        uint64_t b;
+        uint32_t w[kLdsBoardBytes / 4];
+        int c, h;
+    };
+    auto save_pos = [&](Here &o) {
+        if constexpr (W == 4) {
+            o.b = s.bd.b;
+        } else {
+#pragma unroll
+            for (int k = 0; k < kLdsBoardBytes / 4; ++k) o.w[k] = ((const uint32_t *)s.bd.p)[k];
+        }
+        o.c = s.cell();
+        if constexpr (HEUR == 0) o.h = s.hs.h;
+    };
+    auto load_pos = [&](const Here &o) {
+        if constexpr (W == 4) {
+            s.bd.b = o.b;
+        } else {
+#pragma unroll
+            for (int k = 0; k < kLdsBoardBytes / 4; ++k) ((uint32_t *)s.bd.p)[k] = o.w[k];
+        }
+        s.set_cell(o.c);
+        if constexpr (HEUR == 0) s.hs.h = o.h;
+    };
+    // the child in direction d of the node the lane stands on, at depth
+    // `depth`, to position pos of ring r; the lane stays where it is
+    auto queue_child = [&](int r, unsigned long long pos, int d, int depth) {
+        const KParams &p = params_again();
+        const uint32_t nearer = step_down(d);
+        put_item<W, HEUR>(p, r, pos, s, depth, d, inst, p.want_load ? p.c_origin[gl] : 0u);
+        step_back(d, nearer);
+    };
+    // a node of level k is given away: the level's cached sibling values no
+    // longer match the children left there
+    auto void_siblings = [&](int k) {
+        if constexpr (HEUR == 1) {
+            uint32_t &c = sibc[(k % kSibLevels) * blockDim.x];
+            if ((c >> 24) == (uint32_t)k) c = 0xffffffffu;
+        }
+    };
+    // the shallowest level with an open node, at least `above` levels above the
+    // node the lane stands on (a smaller subtree is searched sooner than it
+    // is handed over); 255: none
+    auto give_level = [&](int above) -> int {
+        int lev = 255;
+        if (searching(st))
+            for (int k = 0; k + above <= sp; ++k)
+                if (SE::rest(stk[k * sstride])) {
+                    lev = k;
+                    break;
+                }
+        return lev;
+    };
+    // of the lanes in `from`, the `n` with the smallest 8-bit keys
+    auto smallest = [&](uint64_t from, int key, int n) -> uint64_t {
+        uint64_t chosen = 0;
+#pragma unroll 1
+        for (int bit = 7; bit >= 0; --bit) {
+            const uint64_t zeros = __ballot(((key >> bit) & 1) == 0) & from;
+            const int nz = __popcll(zeros);
+            if (nz >= n) {
+                from = zeros;
+            } else {
+                chosen |= zeros;
+                n -= nz;
+                from &= ~zeros;
+            }
+        }
+        // equal keys: the lowest lanes
+        const bool in = ((from >> lane) & 1ull) && __popcll(from & lanemask_lt()) < n;
+        return chosen | __ballot(in);
+    };
+
+    // What the steps leave to be done between two blocks of them, so that
+    // the steps hold no atomics and none of this code.
+    auto settle = [&]() {
+        const KParams &p = params_again();
+        if (st == ST_GOAL) {
+            atomicMin(&p.found[inst], g);
+            if (p.lookahead) kill_newer(p, inst);
+            // the first goal of the slot's iteration records its path (the
+            // first iteration with a goal has threshold = optimum, and every
+            // goal it finds has that depth)
+            if (p.sol && g <= kPathMax && atomicCAS(&p.sol_len[inst], -1, g) == -1) {
+                const uint32_t so = (uint32_t)inst * kPathWords;
+                path_copy(p.c_ipath, (uint32_t)gl, (uint32_t)NL, p.sol, so, 1);
+                for (int k = 0; k < sp; ++k) path_put(p.sol, so, 1, g - sp + k, SE::dir(stk[k * sstride]));
+            }
+            goal_seen = mode != 1;
+            st = mode == 1 ? ST_POP : ST_FRESH;
+        }
+        if (st == ST_FULL) {
+            // stack full: the passing children become queue items
+            const int k = __builtin_popcount(dpass);
+            atomicAdd(&p.pend[grp * p.gstride + inst], (unsigned)k);
+            atomicAdd(&p.ctl[8], (unsigned)k);
+            const int r = ahead_ring(p, inst);
+            unsigned long long pos = q_reserve(p, r, (unsigned long long)k);
+#pragma unroll 1
+            for (uint32_t pass = dpass; pass; pass &= pass - 1) {
+                const int d = __builtin_ctz(pass);
+                if (p.qpath) item_path(r, pos, sp, d);
+                queue_child(r, pos++, d, g + 1);
+            }
+            st = ST_POP;
+        }
+        // items done: the wave's last one of an instance ends its pending
+        // unit and adds the lanes' counts (read by the next kernel, so
+        // nothing orders the two)
+        if (p.want_load && st == ST_DONE && cnt) {
+            atomicAdd(&p.cnt[grp * p.gstride + inst], (unsigned long long)cnt);
+            atomicAdd(&p.load[(size_t)(inst >> 1) * p.capl + p.c_origin[gl]], (unsigned long long)cnt);
+            cnt = 0;
+        }
+        uint64_t todo = __ballot(st == ST_DONE);
+        while (todo) {
+            const int lead = __ffsll((long long)todo) - 1;
+            const int i = __builtin_amdgcn_readlane(inst, lead);
+            const bool mine = inst == i;
+            todo &= ~__ballot(mine);
+            if (!__ballot(mine && st != ST_DONE && st != ST_IDLE)) {
+                unsigned long long c = mine ? cnt : 0u;
+#pragma unroll
+                for (int off = 32; off > 0; off >>= 1) c += shfl_xor_u64(c, off);
+                if (mine) cnt = 0;
+                if (lane == lead) {
+                    if (c) atomicAdd(&p.cnt[grp * p.gstride + i], c);
+                    atomicSub(&p.pend[grp * p.gstride + i], 1u);
+                }
+            }
+        }
+        if (st == ST_DONE) st = ST_IDLE;
+    };
+
+    // idle lanes get up to `most` queue items, of ring 0 first and of the
+    // wave's own group first
+    auto take_items = [&](int most, Item &it, bool &have) {
+        const KParams &p = params_again();
+#pragma unroll 1
+        for (int t = 0; t < 2 * kGroups && most > 0; ++t) {
+            const int r = t / kGroups;
+            const unsigned x = (grp + t) & (kGroups - 1);
+            if (((r ? empty1 : empty0) >> x) & 1u) continue;
+            unsigned long long *c = p.q_ctl + kQHead + r * kQRing + x * kLine;
+            const unsigned long long lim = p.q_ctl[kQTail + r * kQRing + 1];
+            const uint64_t need = __ballot(st == ST_IDLE && !have);
+            const int n = min(__popcll(need), most);
+            if (n <= 0) break;
+            const int leader = __ffsll((long long)need) - 1;
+            unsigned long long base = 0;
+            if (lane == leader) {
+                base = ld_agent(c);
+                if (base < lim) base = atomicAdd(c, (unsigned long long)n * kGroups);
+            }
+            base = shfl_u64(base, leader);
+            const int rank = __popcll(need & lanemask_lt());
+            const unsigned long long my = base + (unsigned long long)rank * kGroups;
+            const bool took = st == ST_IDLE && !have && rank < n && my < lim;
+            if (took) {
+                it = p.q[q_slot(p, r, my)];
+                have = true;
+                if (p.qpath)
+                    path_copy(p.qpath, (uint32_t)q_slot(p, r, my) * kPathWords, 1, p.c_ipath, (uint32_t)gl,
+                              (uint32_t)NL);
+            }
+            if (base + (unsigned long long)n * kGroups >= lim) (r ? empty1 : empty0) |= 1u << x;
+            // an item's pending unit becomes the wave's; more than one of an
+            // instance are one
+            uint64_t todo = __ballot(took);
+            most -= __popcll(todo);
+            while (todo) {
+                const int lead = __ffsll((long long)todo) - 1;
+                const int i = __builtin_amdgcn_readlane((int)it.inst, lead);
+                const uint64_t got = __ballot(took && (int)it.inst == i);
+                const uint64_t had = __ballot(!took && (have ? (int)it.inst == i : st != ST_IDLE && inst == i));
+                todo &= ~got;
+                const unsigned drop = (unsigned)__popcll(got) - (had ? 0u : 1u);
+                if (drop && lane == lead) atomicSub(&p.pend[grp * p.gstride + i], drop);
+            }
+        }
+    };
+
+    // Inside the wave: each idle lane takes the shallowest open node of one
+    // busy lane, by lane exchange (15-puzzle) or from its board in LDS.
+    auto share = [&](uint64_t idle_mask) {
+        const KParams &p = params_again();
+        const int lev = give_level(kGiveLevels);
+        const uint64_t donors = __ballot(lev < 255);
+        if (!donors) return;
+        const int n = min(__popcll(donors), __popcll(idle_mask));
+        const uint64_t giving = smallest(donors, lev < 255 ? min(g - sp + lev, 255) : 255, n);
+        const bool give = (giving >> lane) & 1ull;
+        // the n-th giver hands to the n-th idle lane: givers push their lane
+        // number to lane n, from where the takers read it
+        const int grank = __popcll(giving & lanemask_lt()), trank = __popcll(idle_mask & lanemask_lt());
+        const int slot = give ? grank : 63 - __popcll(~giving & lanemask_lt());
+        const int at_rank = __builtin_amdgcn_ds_permute(slot << 2, lane);
+        const int src = __shfl(at_rank, trank & 63);
+        const bool take = ((idle_mask >> lane) & 1ull) && trank < n;
+        // a giver goes back to its level and into the child it gives
+        int d2 = 0;
+        Here here;
+        if (give) {
+            save_pos(here);
+            go_back(lev);
+            const uint32_t e = stk[lev * sstride];
+            const uint32_t R = SE::rest(e);
+            d2 = __builtin_ctz(R);
+            stk[lev * sstride] = SE::make(SE::dir(e), R & (R - 1), SE::vals(e));
+            void_siblings(lev);
+            (void)step_down(d2);
+        }
+        // the takers' copies.  The boards are read across lanes of the wave:
+        // its LDS accesses complete in order, only the compiler must keep
+        // them so
+        const uint32_t m = meta_pack(s.cell(), give ? g - sp + lev + 1 : 0, s.hs.h, d2);
+        const uint32_t m2 = (uint32_t)__shfl((int)m, src);
+        const int i2 = __shfl(inst, src), L2 = __shfl(L, src);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if constexpr (W == 4) {
+            const unsigned long long b2 = shfl_u64(s.bd.b, src);
+            if (take) s.bd.b = b2;
+        } else {
+            const uint32_t *from = (const uint32_t *)(s.bd.p + (src - lane) * kLdsBoardBytes);
+            uint32_t w7[kLdsBoardBytes / 4];
+#pragma unroll
+            for (int k = 0; k < kLdsBoardBytes / 4; ++k) w7[k] = from[k];
+            if (take) {
+#pragma unroll
+                for (int k = 0; k < kLdsBoardBytes / 4; ++k) ((uint32_t *)s.bd.p)[k] = w7[k];
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int gsp = __shfl(g - sp, src), lev2 = __shfl(lev, src);
+        if (take) {
+            relabel(i2);
+            L = L2;
+            g = meta_g(m2);
+            prev = meta_prev(m2);
+            s.set_cell(meta_blank(m2));
+            sp = 0;
+            goal_seen = false;
+            st = ST_FRESH;
+            const int gsrc = gl + src - lane;
+            if (p.want_load) p.c_origin[gl] = p.c_origin[gsrc];
+            if (p.qpath) {
+                // the giver's item path, its moves down to the level, the child
+                path_copy(p.c_ipath, (uint32_t)gsrc, (uint32_t)NL, p.c_ipath, (uint32_t)gl, (uint32_t)NL);
+                for (int k = 0; k < lev2; ++k)
+                    path_put(p.c_ipath, (uint32_t)gl, (uint32_t)NL, gsp + k, SE::dir(stk[k * sstride + src - lane]));
+                path_put(p.c_ipath, (uint32_t)gl, (uint32_t)NL, gsp + lev2, prev);
+            }
+            s.hs.h = meta_h(m2);
+            init = true;
+        }
+        // the giver returns to where it stood
+        if (give) load_pos(here);
+    };
+
+    // Between waves: a wave without work puts itself on its group's list and
+    // waits at its own mailbox, a line nobody else polls; a wave with work
+    // that sees somebody waiting takes one wave off the list and writes it
+    // half of what it could give, the shallowest open nodes, one a lane.  So
+    // the waiting cost no atomics but their entry and exit.  A mail is known
+    // by the list position it answers; what a wave finds at its next round's
+    // start was sent while it was leaving.
+    unsigned ticket = (unsigned)uniform(p.ticket[wave_id]); // list position + 1 waited at, 0: none
+    auto read_mail = [&](unsigned n, Item &it, bool &have) {
+        const KParams &p = params_again();
+        if ((unsigned)lane < n) {
+            const unsigned long long *w = (const unsigned long long *)&p.mail[(size_t)wave_id * 64 + lane];
+            const unsigned long long a = ld_agent(w), b = W == 5 ? ld_agent(w + 1) : 0ull;
+            const unsigned long long m = ld_agent(w + 2), o = ld_agent(w + 3);
+            it.b[0] = (uint32_t)a;
+            it.b[1] = (uint32_t)(a >> 32);
+            it.b[2] = (uint32_t)b;
+            it.b[3] = (uint32_t)(b >> 32);
+            it.meta = (uint32_t)m;
+            it.inst = (uint32_t)(m >> 32);
+            it.x0 = 0;
+            it.x1 = (uint32_t)(o >> 32);
+            have = true;
+            if (p.qpath)
+#pragma unroll 1
+                for (uint32_t k = 0; k < (uint32_t)kPathWords; ++k)
+                    p.c_ipath[(size_t)k * NL + gl] = ld_agent(&p.mail_path[((size_t)wave_id * 64 + lane) * kPathWords + k]);
+        }
+        ticket = 0;
+    };
+    // items of the mail that comes; 0: the round ends
+    auto wait_for_mail = [&]() -> unsigned {
+        const KParams &p = params_again();
+        const unsigned x = list_of(blockIdx.x);
+        unsigned long long *list = p.q_ctl + kQList + x * kLine;
+        unsigned long long old = 0;
+        if (lane == 0) old = atomicAdd(list, 1ull << 32);
+        old = uniform(old);
+        const unsigned pos = (unsigned)(old >> 32);
+        ticket = pos + 1;
+        if (lane == 0)
+            st_agent(&p.list[(size_t)x * (p.list_mask + 1) + (pos & p.list_mask)],
+                     ((unsigned long long)ticket << 32) | (unsigned)wave_id);
+        // the last wave of the last list to run out of work ends the round
+        if (waiting(old) + 1 == list_waves(p, x) && idle_waves(p) == (unsigned)NL >> 6) {
+            if (lane == 0) st_agent(p.stop, 1u);
+            return 0;
+        }
+#pragma unroll 1
+        for (int nap = 0; nap < kMaxNaps; ++nap) {
+            const unsigned long long h = uniform(ld_agent(&p.mail_head[(size_t)wave_id * kLine]));
+            if ((unsigned)(h >> 32) == ticket) return (unsigned)h;
+            if (uniform(ld_agent(p.stop))) return 0;
+            // workgroups that have not started yet need the place
+            if ((nap & 15) == 15 && started_waves(p) != (unsigned)NL >> 6) return 0;
+            if (p.round_ticks && (unsigned long long)(wall_clock64() - t_start) >= p.round_ticks) return 0;
+            for (int k = 0; k <= (nap < 3 ? nap : 3); ++k) __builtin_amdgcn_s_sleep(32);
+        }
+        return 0;
+    };
+    // for a waiting wave of list x
+    auto feed = [&](unsigned x, uint32_t rnd) {
+        const KParams &p = params_again();
+        unsigned long long *list = p.q_ctl + kQList + x * kLine;
+        unsigned long long w = uniform(ld_agent(list));
+        const unsigned idle = waiting(w);
+        if (idle == 0) return;
+        // about as many tries in a look's time as waves waiting
+        const unsigned all = list_waves(p, x), donors = all > idle ? all - idle : 1u;
+        if (__umulhi(rnd, donors) >= idle) return;
+        const int lev = give_level(kFeedLevels);
+        const uint64_t can = __ballot(lev < 255 && !ahead_ring(p, inst));
+        const int n = (__popcll(can) + 1) / 2;
+        if (n == 0) return;
+        bool got = false;
+        if (lane == 0) {
+            const unsigned long long seen = atomicCAS(list, w, w + 1);
+            got = seen == w;
+        }
+        if (!__ballot(got)) return;
+        const unsigned pos = (unsigned)w;
+        unsigned long long e = 0;
+        for (int spin = 0; spin < kWriteSpins; ++spin) {
+            e = uniform(ld_agent(&p.list[(size_t)x * (p.list_mask + 1) + (pos & p.list_mask)]));
+            if ((unsigned)(e >> 32) == pos + 1) break;
+            __builtin_amdgcn_s_sleep(8);
+        }
+        if ((unsigned)(e >> 32) != pos + 1) {
+            if (lane == 0) atomicOr(&p.ctl[3], 2u);
+            return;
+        }
+        const unsigned to = (unsigned)e;
+        const uint64_t chosen = smallest(can, lev < 255 ? min(g - sp + lev, 255) : 255, n);
+        const bool give = (chosen >> lane) & 1ull;
+        // the receiving wave's pending unit of each instance
+        uint64_t todo = chosen;
+        while (todo) {
+            const int lead = __ffsll((long long)todo) - 1;
+            const int i = __builtin_amdgcn_readlane(inst, lead);
+            todo &= ~__ballot(inst == i);
+            if (lane == lead) atomicAdd(&p.pend[grp * p.gstride + i], 1u);
+        }
+        if (give) {
+            const size_t slot = (size_t)to * 64 + (size_t)__popcll(chosen & lanemask_lt());
+            const uint32_t e2 = stk[lev * sstride];
+            const uint32_t R = SE::rest(e2);
+            const int d2 = __builtin_ctz(R);
+            if (p.qpath) {
+                uint32_t *to_path = &p.mail_path[slot * kPathWords];
+                for (uint32_t k = 0; k < (uint32_t)kPathWords; ++k)
+                    st_agent(&to_path[k], p.c_ipath[(size_t)k * NL + gl]);
+                for (int k = 0; k <= lev; ++k)
+                    path_put_agent(to_path, g - sp + k, k < lev ? SE::dir(stk[k * sstride]) : d2);
+            }
+            Here here;
+            save_pos(here);
+            go_back(lev);
+            stk[lev * sstride] = SE::make(SE::dir(e2), R & (R - 1), SE::vals(e2));
+            void_siblings(lev);
+            (void)step_down(d2);
+            uint32_t b[4];
+            s.bd.pack(b);
+            unsigned long long *m = (unsigned long long *)&p.mail[slot];
+            st_agent(m, ((unsigned long long)b[1] << 32) | b[0]);
+            if constexpr (W == 5) st_agent(m + 1, ((unsigned long long)b[3] << 32) | b[2]);
+            st_agent(m + 2, ((unsigned long long)(uint32_t)inst << 32) | meta_pack(s.cell(), g - sp + lev + 1, s.hs.h, d2));
+            st_agent(m + 3, p.want_load ? (unsigned long long)p.c_origin[gl] << 32 : 0ull);
+            load_pos(here);
+        }
+        arrival_fence();
+        if (lane == 0) {
+            st_agent(&p.mail_head[(size_t)to * kLine], ((unsigned long long)(pos + 1) << 32) | (unsigned)n);
+            atomicAdd(&p.q_ctl[kQList + list_of(blockIdx.x) * kLine + 1], (unsigned long long)n); // statistics
+        }
     };
 
     uint32_t pf_idle = 0, pf_exp = 0, pf_pop = 0, pf_steps = 0;
@@ -327,344 +870,318 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, cons
     // wait tracking does not carry its loads into every iteration (where it
     // would wait on a move's table reads before issuing the f-test's)
     __builtin_amdgcn_s_waitcnt(0);
-    for (int step = 0; step < budget; ++step) {
-        // a round with a time limit ends between two steps once it is up
-        // (the clock is a scalar read, wave-uniform)
-        if (p.round_ticks && (step & 3) == 3 && (unsigned long long)(wall_clock64() - t_start) >= p.round_ticks)
-            break;
-        // ---- idle lanes take queue items: one atomic per wave and ring,
-        // ring 0 first, none on a ring the wave has seen empty ----
-        {
-            uint64_t need = __ballot(st == ST_IDLE);
-            if (need) {
-                int n = __popcll(need);
-                int leader = __ffsll((long long)need) - 1;
-                unsigned long long base = 0;
-                if (!q0_empty) {
-                    if (lane == leader) base = atomicAdd(&p.q_ctl[0], (unsigned long long)n);
-                    base = shfl_u64(base, leader);
-                    const unsigned long long my = base + __popcll(need & lanemask_lt());
-                    if (st == ST_IDLE && my < limit) {
-                        start_item(p.q[q_slot(p, 0, my)]);
-                        if (p.qpath)
-                            path_copy(p.qpath, (uint32_t)q_slot(p, 0, my) * kPathWords, 1, p.c_ipath, (uint32_t)gl,
-                                      (uint32_t)NL);
+    const long long t_work = wall_clock64();
+    bool left = false; // the wave ran out of work
+    for (int blk = 0;; ++blk) {
+        const KParams &p = params_again();
+        settle();
+        uint64_t idle_mask = __ballot(st == ST_IDLE);
+        if (idle_mask == ~0ull || (take_most == 64 && __popcll(idle_mask) >= kShareMin)) {
+            Item it;
+            bool have = false;
+            unsigned mail = 0;
+            if (blk == 0 && ticket) {
+                // sent while the wave was leaving the last round
+                const unsigned long long h = uniform(p.mail_head[(size_t)wave_id * kLine]);
+                if ((unsigned)(h >> 32) == ticket) mail = (unsigned)h;
+                ticket = 0;
+            }
+            if (!mail) {
+                take_items(take_most, it, have);
+                if (idle_mask == ~0ull && !__ballot(have)) {
+                    mail = wait_for_mail();
+                    if (!mail) {
+                        left = true;
+                        break;
                     }
-                    q0_empty = base + (unsigned long long)n >= limit;
                 }
-                // lanes ring 0 could not serve try the lookahead ring
-                const uint64_t need1 = q1_empty ? 0ull : __ballot(st == ST_IDLE);
-                if (need1) {
-                    const int n1 = __popcll(need1);
-                    const int leader1 = __ffsll((long long)need1) - 1;
-                    unsigned long long base1 = 0;
-                    if (lane == leader1) base1 = atomicAdd(&p.q_ctl[kQCtl], (unsigned long long)n1);
-                    base1 = shfl_u64(base1, leader1);
-                    const unsigned long long my = base1 + __popcll(need1 & lanemask_lt());
-                    if (st == ST_IDLE && my < limit1) {
-                        start_item(p.q[q_slot(p, 1, my)]);
-                        if (p.qpath)
-                            path_copy(p.qpath, (uint32_t)q_slot(p, 1, my) * kPathWords, 1, p.c_ipath, (uint32_t)gl,
-                                      (uint32_t)NL);
-                    }
-                    q1_empty = base1 + (unsigned long long)n1 >= limit1;
-                }
-                if (st == ST_IDLE) st = ST_DRAINED;
+            }
+            if (mail) read_mail(mail, it, have);
+            if (have) start_item(it);
+            idle_mask = __ballot(st == ST_IDLE);
+        }
+        if (__popcll(idle_mask) >= kShareMin) share(idle_mask);
+        if (init) {
+            init_heur<W, HEUR>(s, P, meta_pack(0, 0, s.hs.h, 0));
+            init = false;
+        }
+        // the time limit, the round's end as some wave saw it, and, every few
+        // blocks, whether the waves without work have waited long enough
+        // (never before a wave's first block: every round makes progress)
+        if (blk >= least) {
+            const long long now = wall_clock64();
+            bool stop = steps_left <= 0 || (p.round_ticks && (unsigned long long)(now - t_start) >= p.round_ticks);
+            const bool over = uniform(ld_agent(p.stop)) != 0;
+            if (!stop && !over && threadIdx.x < 64 && (blk & 7) == 0)
+                stop = (unsigned long long)(now - t_work) * idle_waves(p) >= p.turn_ticks * n_waves;
+            if (stop && !over && lane == 0) st_agent(p.stop, 1u);
+            if (stop || over) break;
+            if (((blk + wave_id) & 1) == 0) {
+                // every other look at any list, not the wave's own
+                uint32_t rnd = ((uint32_t)now ^ (uint32_t)wave_id * 0x9e3779b9u) * 0x85ebca6bu;
+                rnd = (rnd ^ (rnd >> 15)) * 0xc2b2ae35u;
+                feed(blk & 2 ? (rnd >> 7) & (kLists - 1) : list_of(blockIdx.x), rnd ^ (rnd << 13));
             }
         }
-        if (!__ballot(st == ST_FRESH || st == ST_POP || st == ST_DESC)) break;
-
-        // ---- pop: undo up to kPops moves, until a level with a passing
-        // child not visited yet ----
-        bool finish = false;
-        int down = -1;      // child entered this step (-1: none)
-        int slot = 0;       // its stack level
-        uint32_t R = 0;     // passing children still to visit at that level
-        bool known = false; // its lookup values are known (PDB)
-        uint32_t kv = 0;
+        if (mode == 1 && searching(st) && ld_agent(&p.found[inst]) != kNoGoal)
+            sp = 0, st = ST_POP; // first-solution: the rest of the item is not wanted
+        const int block = max(1, min(steps_left, kShareSteps));
+        steps_left -= block;
+        for (int step = 0; step < block; ++step) {
+            if (!__ballot(searching(st))) break;
+            // ---- pop: undo up to kPops moves, until a level with a passing
+            // child not visited yet ----
+            int down = -1;      // child entered this step (-1: none)
+            int slot = 0;       // its stack level
+            uint32_t R = 0;     // passing children still to visit at that level
+            bool known = false; // its lookup values are known (PDB)
+            uint32_t kv = 0;
 #pragma unroll 1
-        for (int pk = 0; pk < kPops && st == ST_POP; ++pk) {
-            if (sp == 0) {
-                finish = true;
-                break;
+            for (int pk = 0; pk < kPops && st == ST_POP; ++pk) {
+                if (sp == 0) {
+                    st = ST_DONE;
+                    break;
+                }
+                uint32_t e = stk[(sp - 1) * sstride];
+                int d = SE::dir(e);
+                uint32_t Re = SE::rest(e);
+                if constexpr (HEUR == 1)
+                    do_move_known<W>(s, 3 - d, P, SE::vals(e));
+                else
+                    unmove_md(s, d, SE::vals(e));
+                --g;
+                if (Re) {
+                    down = __builtin_ctz(Re);
+                    R = Re & (Re - 1);
+                    slot = sp - 1;
+                    st = ST_FRESH;
+                    if constexpr (HEUR == 1) {
+                        uint32_t &c = sibc[(slot % kSibLevels) * blockDim.x];
+                        const uint32_t cv = c;
+                        if ((cv >> 24) == (uint32_t)slot) {
+                            known = true;
+                            kv = (cv & 63u) | (((cv >> 6) & 63u) << 8);
+                            c = (cv & 0xff000000u) | ((cv >> 12) & 0xfffu); // the sibling after it moves up
+                        }
+                    }
+                } else {
+                    --sp;
+                }
             }
-            uint32_t e = stk[(sp - 1) * sstride];
-            int d = SE::dir(e);
-            uint32_t Re = SE::rest(e);
-            if constexpr (HEUR == 1)
-                do_move_known<W>(s, 3 - d, P, SE::vals(e));
-            else
-                unmove_md(s, d, SE::vals(e));
-            --g;
-            if (Re) {
-                down = __builtin_ctz(Re);
-                R = Re & (Re - 1);
-                slot = sp - 1;
-                st = ST_FRESH;
+            // ---- or enter the first passing child of last step's expansion ----
+            if (st == ST_DESC) {
+                down = __builtin_ctz(dpass);
+                R = dpass & (dpass - 1);
+                slot = sp;
+                known = true;
+                kv = (((down >= 2) ? dval2 : dval) >> (16 * (down & 1))) & 0xffffu;
                 if constexpr (HEUR == 1) {
-                    uint32_t &c = sibc[(slot % kSibLevels) * blockDim.x];
-                    const uint32_t cv = c;
-                    if ((cv >> 24) == (uint32_t)slot) {
-                        known = true;
-                        kv = (cv & 63u) | (((cv >> 6) & 63u) << 8);
-                        c = (cv & 0xff000000u) | ((cv >> 12) & 0xfffu); // the sibling after it moves up
-                    }
-                }
-            } else {
-                --sp;
-            }
-        }
-        // ---- or enter the first passing child of last step's expansion ----
-        if (st == ST_DESC) {
-            down = __builtin_ctz(dpass);
-            R = dpass & (dpass - 1);
-            slot = sp;
-            known = true;
-            kv = (((down >= 2) ? dval2 : dval) >> (16 * (down & 1))) & 0xffffu;
-            if constexpr (HEUR == 1) {
-                if (R) {
-                    // values of the next two passing children, 6 + 6 bits
-                    // each.  An entry holds two siblings: a node with three
-                    // more (an item rooted at an instance's root, all four
-                    // moves passing) voids its level's entry instead, so
-                    // that none of them takes values left by an older node
-                    // of this depth, or the zeros shifted in after two
-                    uint32_t ent = 0xffffffffu;
-                    if (__builtin_popcount(R) <= 2) {
-                        const int s1 = __builtin_ctz(R);
-                        const uint32_t R2 = R & (R - 1);
-                        const int s2 = R2 ? __builtin_ctz(R2) : s1;
-                        const uint32_t v1 = (((s1 >= 2) ? dval2 : dval) >> (16 * (s1 & 1))) & 0xffffu;
-                        const uint32_t v2 = (((s2 >= 2) ? dval2 : dval) >> (16 * (s2 & 1))) & 0xffffu;
-                        const uint32_t p1 = (v1 & 63u) | (((v1 >> 8) & 63u) << 6);
-                        const uint32_t p2 = (v2 & 63u) | (((v2 >> 8) & 63u) << 6);
-                        ent = ((uint32_t)slot << 24) | p1 | (p2 << 12);
-                    }
-                    sibc[(slot % kSibLevels) * blockDim.x] = ent;
-                }
-            }
-        }
-        // ---- one move down per lane and step, both cases on one path.  For
-        // the PDB the move's values are applied after the f-test's table
-        // reads are issued, so both sets of reads are in flight together ----
-        PendMove pm;
-        bool pmv = false;
-        if (down >= 0) {
-            if constexpr (HEUR == 1) {
-                uint32_t ov;
-                if (p.prof) pf_sib += known ? 0u : 1u;
-                pm = move_pdb_begin<W>(s, down, P, known, kv, ov);
-                pmv = true;
-                stk[slot * sstride] = SE::make(down, R, ov);
-                sp = slot + 1;
-                ++g;
-                prev = down;
-                st = ST_FRESH;
-            } else {
-                enter_child(down, R, slot, known, kv);
-            }
-        }
-
-        // ---- expand, first half (PDB): the children's lookup indices and
-        // table reads; they need the node's indices, not its values ----
-        uint32_t gen = 0;
-        // per child slot: lookups kr/kf, the index of the second lookup, the
-        // first and second values read, the direction
-        int ckr[4], ckf[4], cv1[4], cv2[4], cdir[4];
-        uint32_t cidx2[4];
-        int ng = 0;
-        bool regfirst = true; // read the regular lookup first (else the reflected)
-        if (st == ST_FRESH) {
-            gen = legal_moves(s) & ~(prev < 4 ? (1u << (3 - prev)) : 0u);
-            if constexpr (HEUR == 1) {
-                // lane-slot j reads the lane's j-th generated child, so the
-                // wave runs as many slots as its largest family (3 below the
-                // root), not one per direction.  Only one lookup per child
-                // is read here: that of the partition whose sum is larger at
-                // the node (before a pending move's values: a heuristic
-                // choice); the other is read only for children the first
-                // does not already cut off (the reference's early cut,
-                // src_horie/idas_pdb.cu:228-231, regular sum first).
-                ng = __builtin_popcount(gen);
-                regfirst = s.hs.A >= s.hs.B;
-                const int bl = s.cell();
-                const PdbGeo &G = *P.geo;
-                uint32_t rem = gen;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    ckr[j] = ckf[j] = cv1[j] = cv2[j] = cdir[j] = 0;
-                    cidx2[j] = 0;
-                    if (!__ballot(j < ng)) continue;
-                    if (j < ng) {
-                        const int d = __builtin_ctz(rem);
-                        rem &= rem - 1;
-                        const int from = bl + dir_cell<W>(d);
-                        const int t = s.bd.tile(from);
-                        const uint2 wa = G.w[t][from], wb = G.w[t][bl];
-                        const int kr = (int)(wa.x >> 28), kf = (int)(wa.y >> 28);
-                        const uint32_t ir = sel4(s.hs.i0, s.hs.i1, s.hs.i2, s.hs.i3, kr) + (wb.x - wa.x);
-                        const uint32_t iff = sel4(s.hs.j0, s.hs.j1, s.hs.j2, s.hs.j3, kf) + (wb.y - wa.y);
-                        cdir[j] = d;
-                        ckr[j] = kr;
-                        ckf[j] = kf;
-                        cv1[j] = pdb_read(P, regfirst ? ir : iff);
-                        cidx2[j] = regfirst ? iff : ir;
-                    }
-                }
-            }
-        }
-        if constexpr (HEUR == 1) {
-            if (pmv) move_pdb_finish(s.hs, pm);
-        }
-
-        // ---- expand, second half: goal test, count, f-tests ----
-        bool expanded = false;
-        if (st == ST_FRESH) {
-            const int h = s.hs.h;
-            bool xp = true;
-            if (h == 0) {
-                atomicMin(&p.found[inst], g);
-                if (p.lookahead) kill_newer(p, inst);
-                // the first goal of the slot's iteration records its path
-                // (the first iteration with a goal has threshold = optimum,
-                // and every goal it finds has that depth)
-                if (p.sol && g <= kPathMax && atomicCAS(&p.sol_len[inst], -1, g) == -1) {
-                    const uint32_t so = (uint32_t)inst * kPathWords;
-                    path_copy(p.c_ipath, (uint32_t)gl, (uint32_t)NL, p.sol, so, 1);
-                    const int gr = meta_g(rmeta);
-                    for (int k = 0; k < sp; ++k) path_put(p.sol, so, 1, gr + k, SE::dir(stk[k * sstride]));
-                }
-                if (mode == 1) {
-                    st = ST_POP;
-                    xp = false;
-                }
-            }
-            if (xp) {
-                expanded = true;
-                cnt += (uint32_t)__builtin_popcount(gen);
-                uint32_t pass = gen;
-                uint32_t cvals = 0, cvals2 = 0; // PDB values of children 0,1 / 2,3 (16 bits each)
-                if constexpr (HEUR == 0) {
-                    // Manhattan is consistent: h changes by exactly +-1 per
-                    // move and f keeps the threshold's parity, so with slack
-                    // >= 2 every child fits and with slack 0 only children
-                    // with h-1 do.
-                    const int slack = L - g - h;
-                    if (slack <= 2) {
-                        const uint32_t near = nearer_moves<W>(s.bd, s.cell());
-                        if (slack < 2) pass = gen & near;
-                        // A child at slack 0 (slack 0 and nearer, or slack 2
-                        // and farther) whose own children all fail the
-                        // f-test is a leaf: its children are counted here
-                        // and it is not entered.  Its children's tiles are
-                        // all on the current board (entering it would only
-                        // move the blank there).  With h >= 2 no such child
-                        // is a goal, and a leaf has no goal child (one would
-                        // be nearer, and pass).  One child per expansion is
-                        // tested, the first such: a wave would run the test
-                        // as often as its lane with the most.
-                        const uint32_t cand = h < 2 ? 0u : (slack < 2 ? pass : gen & ~near);
-                        if (cand) {
-                            const int d = __builtin_ctz(cand);
-                            const int cc = s.cell() + dir_cell<W>(d);
-                            const uint32_t cgen = legal_cell<W>(cc) & ~(1u << (3 - d));
-                            if (!(cgen & nearer_moves<W>(s.bd, cc))) {
-                                cnt += (uint32_t)__builtin_popcount(cgen);
-                                pass &= ~(1u << d);
-                            }
+                    if (R) {
+                        // values of the next two passing children, 6 + 6 bits
+                        // each.  An entry holds two siblings: a node with three
+                        // more (an item rooted at an instance's root, all four
+                        // moves passing) voids its level's entry instead, so
+                        // that none of them takes values left by an older node
+                        // of this depth, or the zeros shifted in after two
+                        uint32_t ent = 0xffffffffu;
+                        if (__builtin_popcount(R) <= 2) {
+                            const int s1 = __builtin_ctz(R);
+                            const uint32_t R2 = R & (R - 1);
+                            const int s2 = R2 ? __builtin_ctz(R2) : s1;
+                            const uint32_t v1 = (((s1 >= 2) ? dval2 : dval) >> (16 * (s1 & 1))) & 0xffffu;
+                            const uint32_t v2 = (((s2 >= 2) ? dval2 : dval) >> (16 * (s2 & 1))) & 0xffffu;
+                            const uint32_t p1 = (v1 & 63u) | (((v1 >> 8) & 63u) << 6);
+                            const uint32_t p2 = (v2 & 63u) | (((v2 >> 8) & 63u) << 6);
+                            ent = ((uint32_t)slot << 24) | p1 | (p2 << 12);
                         }
+                        sibc[(slot % kSibLevels) * blockDim.x] = ent;
                     }
+                }
+            }
+            // ---- one move down per lane and step, both cases on one path.  For
+            // the PDB the move's values are applied after the f-test's table
+            // reads are issued, so both sets of reads are in flight together ----
+            PendMove pm;
+            bool pmv = false;
+            if (down >= 0) {
+                if constexpr (HEUR == 1) {
+                    uint32_t ov;
+                    if constexpr (PROF) pf_sib += known ? 0u : 1u;
+                    pm = move_pdb_begin<W>(s, down, P, known, kv, ov);
+                    pmv = true;
+                    stk[slot * sstride] = SE::make(down, R, ov);
+                    sp = slot + 1;
+                    ++g;
+                    prev = down;
+                    st = ST_FRESH;
                 } else {
-                    // the PDB max is not consistent (lookups take the minimum
-                    // over blank cells): h may jump by 3, so every generated
-                    // child gets its own f-test
-                    pass = 0;
-                    const HState<1> &hs = s.hs;
-                    // the first partition's sum of each child; the second
-                    // lookup is read only where that sum fits
-                    uint32_t need = 0;
+                    enter_child(down, R, slot, known, kv);
+                }
+            }
+
+            // ---- expand, first half (PDB): the children's lookup indices and
+            // table reads; they need the node's indices, not its values ----
+            uint32_t gen = 0;
+            // per child slot: lookups kr/kf, the index of the second lookup, the
+            // first and second values read, the direction
+            int ckr[4], ckf[4], cv1[4], cv2[4], cdir[4];
+            uint32_t cidx2[4];
+            int ng = 0;
+            bool regfirst = true; // read the regular lookup first (else the reflected)
+            if (st == ST_FRESH) {
+                gen = legal_moves(s) & ~(prev < 4 ? (1u << (3 - prev)) : 0u);
+                if constexpr (HEUR == 1) {
+                    // lane-slot j reads the lane's j-th generated child, so the
+                    // wave runs as many slots as its largest family (3 below the
+                    // root), not one per direction.  Only one lookup per child
+                    // is read here: that of the partition whose sum is larger at
+                    // the node (before a pending move's values: a heuristic
+                    // choice); the other is read only for children the first
+                    // does not already cut off (the reference's early cut,
+                    // src_horie/idas_pdb.cu:228-231, regular sum first).
+                    ng = __builtin_popcount(gen);
+                    regfirst = s.hs.A >= s.hs.B;
+                    const int bl = s.cell();
+                    const PdbGeo &G = *P.geo;
+                    uint32_t rem = gen;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
+                        ckr[j] = ckf[j] = cv1[j] = cv2[j] = cdir[j] = 0;
+                        cidx2[j] = 0;
+                        if (!__ballot(j < ng)) continue;
                         if (j < ng) {
-                            const int s1 = regfirst ? hs.A - byte_of(hs.v0, ckr[j]) + cv1[j]
-                                                    : hs.B - byte_of(hs.v1, ckf[j]) + cv1[j];
-                            if (g + 1 + s1 <= L) {
-                                need |= 1u << j;
-                                cv2[j] = pdb_read(P, cidx2[j]);
-                            }
-                            if (p.prof) {
-                                pf_rd1 += 1u;
-                                pf_rd2 += (g + 1 + s1 <= L) ? 1u : 0u;
-                            }
+                            const int d = __builtin_ctz(rem);
+                            rem &= rem - 1;
+                            const int from = bl + dir_cell<W>(d);
+                            const int t = s.bd.tile(from);
+                            const uint2 wa = G.w[t][from], wb = G.w[t][bl];
+                            const int kr = (int)(wa.x >> 28), kf = (int)(wa.y >> 28);
+                            const uint32_t ir = sel4(s.hs.i0, s.hs.i1, s.hs.i2, s.hs.i3, kr) + (wb.x - wa.x);
+                            const uint32_t iff = sel4(s.hs.j0, s.hs.j1, s.hs.j2, s.hs.j3, kf) + (wb.y - wa.y);
+                            cdir[j] = d;
+                            ckr[j] = kr;
+                            ckf[j] = kf;
+                            cv1[j] = pdb_read(P, regfirst ? ir : iff);
+                            cidx2[j] = regfirst ? iff : ir;
                         }
                     }
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        if ((need >> j) & 1u) {
-                            const int d = cdir[j];
-                            const int vr = regfirst ? cv1[j] : cv2[j];
-                            const int vf = regfirst ? cv2[j] : cv1[j];
-                            const int A = hs.A - byte_of(hs.v0, ckr[j]) + vr;
-                            const int B = hs.B - byte_of(hs.v1, ckf[j]) + vf;
-                            const int hc = A > B ? A : B;
-                            pass |= (g + 1 + hc <= L) ? (1u << d) : 0u;
-                            const uint32_t v = ((uint32_t)vr | ((uint32_t)vf << 8)) << (16u * (uint32_t)(d & 1));
-                            if (d < 2)
-                                cvals |= v;
-                            else
-                                cvals2 |= v;
-                        }
-                    }
-                }
-                if (!pass) {
-                    st = ST_POP;
-                } else if (sp < MAXD) {
-                    // enter the first passing child next step
-                    st = ST_DESC;
-                    dpass = pass;
-                    dval = cvals;
-                    dval2 = cvals2;
-                } else {
-                    // stack full: the passing children become queue items
-                    int k = __builtin_popcount(pass);
-                    atomicAdd(&p.pend[inst], (unsigned)k);
-                    const int r = ahead_ring(p, inst);
-                    unsigned long long pos = q_reserve(p, r, (unsigned long long)k);
-                    atomicAdd(&p.ctl[8], (unsigned)k);
-                    while (pass) {
-                        int d = __builtin_ctz(pass);
-                        pass &= pass - 1;
-                        if (p.qpath) item_path(r, pos, sp, d);
-                        Pos<W, HEUR> c = reg_pos(s);
-                        if constexpr (HEUR == 1)
-                            move_board_only(c, d); // the item's lane recomputes its lookups
-                        else
-                            do_move<W, HEUR>(c, d, P);
-                        put_item<W, HEUR>(p, r, pos++, c, g + 1, d, inst, origin);
-                    }
-                    st = ST_POP;
                 }
             }
-        }
+            if constexpr (HEUR == 1) {
+                if (pmv) move_pdb_finish(s.hs, pm);
+            }
 
-        // ---- items whose subtree is done (after the expansion, so that its
-        // fence does not wait on the step's table reads) ----
-        if (finish) {
-            if (cnt) {
-                atomicAdd(&p.cnt[inst], (unsigned long long)cnt);
-                atomicAdd(&p.load[(size_t)(inst >> 1) * p.capl + origin], (unsigned long long)cnt);
+            // ---- expand, second half: goal test, count, f-tests ----
+            bool expanded = false;
+            if (st == ST_FRESH) {
+                const int h = s.hs.h;
+                bool xp = true;
+                if (h == 0) {
+                    // recorded between two blocks of steps, then expanded
+                    xp = goal_seen;
+                    if (!goal_seen) st = ST_GOAL;
+                    goal_seen = false;
+                }
+                if (xp) {
+                    expanded = true;
+                    cnt += (uint32_t)__builtin_popcount(gen);
+                    uint32_t pass = gen;
+                    uint32_t cvals = 0, cvals2 = 0; // PDB values of children 0,1 / 2,3 (16 bits each)
+                    if constexpr (HEUR == 0) {
+                        // Manhattan is consistent: h changes by exactly +-1 per
+                        // move and f keeps the threshold's parity, so with slack
+                        // >= 2 every child fits and with slack 0 only children
+                        // with h-1 do.
+                        const int slack = L - g - h;
+                        if (slack <= 2) {
+                            const uint32_t near = nearer_moves<W>(s.bd, s.cell());
+                            if (slack < 2) pass = gen & near;
+                            // A child at slack 0 (slack 0 and nearer, or slack 2
+                            // and farther) whose own children all fail the
+                            // f-test is a leaf: its children are counted here
+                            // and it is not entered.  Its children's tiles are
+                            // all on the current board (entering it would only
+                            // move the blank there).  With h >= 2 no such child
+                            // is a goal, and a leaf has no goal child (one would
+                            // be nearer, and pass).  One child per expansion is
+                            // tested, the first such: a wave would run the test
+                            // as often as its lane with the most.
+                            const uint32_t cand = h < 2 ? 0u : (slack < 2 ? pass : gen & ~near);
+                            if (cand) {
+                                const int d = __builtin_ctz(cand);
+                                const int cc = s.cell() + dir_cell<W>(d);
+                                const uint32_t cgen = legal_cell<W>(cc) & ~(1u << (3 - d));
+                                if (!(cgen & nearer_moves<W>(s.bd, cc))) {
+                                    cnt += (uint32_t)__builtin_popcount(cgen);
+                                    pass &= ~(1u << d);
+                                }
+                            }
+                        }
+                    } else {
+                        // the PDB max is not consistent (lookups take the minimum
+                        // over blank cells): h may jump by 3, so every generated
+                        // child gets its own f-test
+                        pass = 0;
+                        const HState<1> &hs = s.hs;
+                        // the first partition's sum of each child; the second
+                        // lookup is read only where that sum fits
+                        uint32_t need = 0;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            if (j < ng) {
+                                const int s1 = regfirst ? hs.A - byte_of(hs.v0, ckr[j]) + cv1[j]
+                                                        : hs.B - byte_of(hs.v1, ckf[j]) + cv1[j];
+                                if (g + 1 + s1 <= L) {
+                                    need |= 1u << j;
+                                    cv2[j] = pdb_read(P, cidx2[j]);
+                                }
+                                if constexpr (PROF) {
+                                    pf_rd1 += 1u;
+                                    pf_rd2 += (g + 1 + s1 <= L) ? 1u : 0u;
+                                }
+                            }
+                        }
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            if ((need >> j) & 1u) {
+                                const int d = cdir[j];
+                                const int vr = regfirst ? cv1[j] : cv2[j];
+                                const int vf = regfirst ? cv2[j] : cv1[j];
+                                const int A = hs.A - byte_of(hs.v0, ckr[j]) + vr;
+                                const int B = hs.B - byte_of(hs.v1, ckf[j]) + vf;
+                                const int hc = A > B ? A : B;
+                                pass |= (g + 1 + hc <= L) ? (1u << d) : 0u;
+                                const uint32_t v = ((uint32_t)vr | ((uint32_t)vf << 8)) << (16u * (uint32_t)(d & 1));
+                                if (d < 2)
+                                    cvals |= v;
+                                else
+                                    cvals2 |= v;
+                            }
+                        }
+                    }
+                    if (!pass) {
+                        st = ST_POP;
+                    } else if (sp < MAXD) {
+                        // enter the first passing child next step
+                        st = ST_DESC;
+                        dpass = pass;
+                        dval = cvals;
+                        dval2 = cvals2;
+                    } else {
+                        // stack full: the passing children become queue items
+                        // between two blocks of steps
+                        st = ST_FULL;
+                        dpass = pass;
+                    }
+                }
             }
-            __threadfence();
-            unsigned old = atomicSub(&p.pend[inst], 1u);
-            if (old == 1u) iteration_drained(p, inst);
-            cnt = 0;
-            st = ST_IDLE;
-        }
-        if (p.prof) {
-            pf_steps += 1;
-            pf_idle += (st == ST_IDLE || st == ST_DRAINED) ? 1u : 0u;
-            pf_exp += expanded ? 1u : 0u;
-            pf_pop += (!expanded && (st == ST_POP || st == ST_DESC)) ? 1u : 0u;
+
+            if constexpr (PROF) {
+                pf_steps += 1;
+                pf_idle += (!expanded && (st == ST_IDLE || st >= ST_DONE)) ? 1u : 0u;
+                pf_exp += expanded ? 1u : 0u;
+                pf_pop += (!expanded && (st == ST_POP || st == ST_DESC)) ? 1u : 0u;
+            }
         }
     }
 
@@ -674,102 +1191,25 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, cons
         enter_child(dn, dpass & (dpass - 1), sp, true, (((dn >= 2) ? dval2 : dval) >> (16 * (dn & 1))) & 0xffffu);
     }
 
-    // ---- round end: donate shallow open nodes, then save the context ----
     const bool busy = (st == ST_FRESH || st == ST_POP);
-    // lanes on lookahead iterations donate into ring 1, under their own quota
-    const int ring = busy ? ahead_ring(p, inst) : 0;
-    const int per_lane = (int)(ring ? p.ctl[19] : p.ctl[4]);
-    int want = 0;
-    if (busy && per_lane > 0) {
-        int avail = 0;
-        for (int k = 0; k < sp && avail < per_lane; ++k) avail += __builtin_popcount(SE::rest(stk[k * sstride]));
-        want = avail < per_lane ? avail : per_lane;
-    }
-    if (__ballot(want > 0)) {
-        // per ring: wave prefix sum of `want`, one queue reservation per wave
-        unsigned long long pos = 0;
-        for (int r = 0; r < 2; ++r) {
-            const int wr = ring == r ? want : 0;
-            if (!__ballot(wr > 0)) continue;
-            int incl = wr;
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) {
-                int v = __shfl_up(incl, off);
-                if (lane >= off) incl += v;
-            }
-            int total = __shfl(incl, 63);
-            unsigned long long base = 0;
-            if (lane == 0) {
-                base = q_reserve(p, r, (unsigned long long)total);
-                atomicAdd(&p.ctl[7], (unsigned)total);
-            }
-            base = shfl_u64(base, 0);
-            if (wr > 0) pos = base + (unsigned long long)(incl - wr);
-        }
-        if (want > 0) {
-            atomicAdd(&p.pend[inst], (unsigned)want);
-            if (p.qpath) {
-                // the donated items' paths first, in the order of the pass
-                // below (a pass of its own keeps the replayed positions out
-                // of its registers)
-                unsigned long long pp = pos;
-                int emitted = 0;
-                for (int k = 0; k < sp && emitted < want; ++k) {
-                    uint32_t R = SE::rest(stk[k * sstride]);
-                    while (R && emitted < want) {
-                        const int d2 = __builtin_ctz(R);
-                        R &= R - 1;
-                        item_path(ring, pp++, k, d2);
-                        ++emitted;
-                    }
-                }
-            }
-            // replay from the item root along the taken moves (for the PDB the
-            // board alone: the lane that takes an item recomputes its lookups)
-            Pos<W, HEUR> c;
-            if constexpr (HEUR == 1) {
-                c.bd.unpack(root);
-                c.set_cell(meta_blank(rmeta));
-                c.hs.h = 0;
-            } else {
-                pos_from_item<W, HEUR>(c, root, rmeta, P);
-            }
-            int cg = meta_g(rmeta);
-            int emitted = 0;
-            for (int k = 0; k < sp && emitted < want; ++k) {
-                uint32_t e = stk[k * sstride];
-                int d = SE::dir(e);
-                uint32_t R = SE::rest(e);
-                while (R && emitted < want) {
-                    int d2 = __builtin_ctz(R);
-                    R &= R - 1;
-                    Pos<W, HEUR> x = c;
-                    if constexpr (HEUR == 1)
-                        move_board_only(x, d2);
-                    else
-                        do_move<W, HEUR>(x, d2, P);
-                    put_item<W, HEUR>(p, ring, pos++, x, cg + 1, d2, inst, origin);
-                    ++emitted;
-                }
-                stk[k * sstride] = SE::make(d, R, SE::vals(e));
-                if (emitted < want) {
-                    if constexpr (HEUR == 1)
-                        move_board_only(c, d);
-                    else
-                        do_move<W, HEUR>(c, d, P);
-                    ++cg;
-                }
-            }
-        }
-    }
+    if (lane == 0) p.ticket[wave_id] = left ? ticket : 0u;
 
-    // keep the per-lane u32 count far from wrapping on long-lived items
-    if (busy && cnt >= (1u << 30)) {
-        atomicAdd(&p.cnt[inst], (unsigned long long)cnt);
-        atomicAdd(&p.load[(size_t)(inst >> 1) * p.capl + origin], (unsigned long long)cnt);
-        cnt = 0;
+    // node counts of idle lanes, and of lanes far on the way to wrapping
+    uint64_t todo = __ballot(cnt != 0 && (!busy || cnt >= (1u << 30)));
+    while (todo) {
+        const int lead = __ffsll((long long)todo) - 1;
+        const int i = __builtin_amdgcn_readlane(inst, lead);
+        const bool mine = cnt != 0 && (!busy || cnt >= (1u << 30)) && inst == i;
+        todo &= ~__ballot(mine);
+        if (mine && p.want_load)
+            atomicAdd(&p.load[(size_t)(inst >> 1) * p.capl + p.c_origin[gl]], (unsigned long long)cnt);
+        unsigned long long c = mine ? cnt : 0u;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) c += shfl_xor_u64(c, off);
+        if (mine) cnt = 0;
+        if (lane == lead) atomicAdd(&p.cnt[grp * p.gstride + i], c);
     }
-    if (p.prof) {
+    if constexpr (PROF) {
         // wave sums of this round's lane-step states
         for (int off = 32; off > 0; off >>= 1) {
             pf_idle += __shfl_xor(pf_idle, off);
@@ -780,13 +1220,14 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, cons
             pf_rd2 += __shfl_xor(pf_rd2, off);
         }
         if (lane == 0) {
-            atomicAdd(&p.prof[0], (unsigned long long)pf_idle);
-            atomicAdd(&p.prof[1], (unsigned long long)pf_exp);
-            atomicAdd(&p.prof[2], (unsigned long long)pf_pop);
-            atomicAdd(&p.prof[3], (unsigned long long)pf_steps);
-            atomicAdd(&p.prof[4], (unsigned long long)pf_sib);
-            atomicAdd(&p.prof[5], (unsigned long long)pf_rd1);
-            atomicAdd(&p.prof[6], (unsigned long long)pf_rd2);
+            unsigned long long *w = p.prof + (size_t)wave_id * 8; // the wave's own: one address for all would be a queue
+            w[0] += pf_idle;
+            w[1] += pf_exp;
+            w[2] += pf_pop;
+            w[3] += pf_steps;
+            w[4] += pf_sib;
+            w[5] += pf_rd1;
+            w[6] += pf_rd2;
         }
     }
     if (p.wtime && lane == 0 && p.ctl[6] == p.wtime_round) {
@@ -794,23 +1235,15 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 1)) k_round(KParams p, cons
         p.wtime[2 * wg] = (unsigned long long)t_start;
         p.wtime[2 * wg + 1] = (unsigned long long)wall_clock64();
     }
-    uint64_t busy_mask = __ballot(busy);
-    if (lane == 0 && busy_mask) atomicAdd(&p.ctl[2], (unsigned)__popcll(busy_mask));
-    const uint64_t ahead_mask = p.lookahead ? __ballot(busy && ring == 1) : 0ull;
-    if (lane == 0 && ahead_mask) atomicAdd(&p.ctl[34], (unsigned)__popcll(ahead_mask));
     if (busy) {
-        p.c_st[gl] = (uint32_t)st | ((uint32_t)sp << 8);
+        p.c_st[gl] = (uint32_t)(goal_seen && st == ST_FRESH ? ST_GOAL : st) | ((uint32_t)sp << 8);
         uint32_t b[4];
         s.bd.pack(b);
 #pragma unroll
         for (int k = 0; k < 4; ++k) p.c_rows[k * NL + gl] = b[k];
-#pragma unroll
-        for (int k = 0; k < 4; ++k) p.c_root[k * NL + gl] = root[k];
         p.c_meta[gl] = meta_pack(s.cell(), g, s.hs.h, prev);
-        p.c_rmeta[gl] = rmeta;
         p.c_inst[gl] = (uint32_t)inst;
         p.c_cnt[gl] = cnt;
-        p.c_origin[gl] = origin;
         if constexpr (HEUR == 1) {
             p.c_pdb[0 * NL + gl] = s.hs.i0;
             p.c_pdb[1 * NL + gl] = s.hs.i1;
@@ -836,8 +1269,8 @@ __device__ __forceinline__ int path_f(const Item &it) {
 }
 
 // ---------------------------------------------------------------------------
-// k_restart: between rounds, one block per instance on the restart list (a
-// slot of it drained, it is new, or lookahead was asked for).  Thread 0
+// k_restart: between rounds, one block per instance; it acts where the current
+// iteration has ended, none runs yet, or lookahead was asked for.  Thread 0
 // resolves the instance's iterations in order: while the current iteration
 // has drained, its count is recorded and it ends the instance (goal found,
 // or iteration limit) or the next one becomes current -- already running if
@@ -948,7 +1381,7 @@ __device__ int resolve_instance(const KParams &p, int inst) {
             }
             return -1;
         }
-        p.iter_counts[(size_t)inst * p.max_iters + cur] = p.cnt[isc];
+        p.iter_counts[(size_t)inst * p.max_iters + cur] = slot_count(p, isc);
         if (p.found[isc] != kNoGoal || cur + 1 >= p.max_iters) {
             p.opt[inst] = p.found[isc] != kNoGoal ? p.found[isc] : -1;
             p.done[inst] = 1;
@@ -971,9 +1404,19 @@ __global__ void __launch_bounds__(256) k_restart(KParams p, const PdbGeo *geo_g)
     __shared__ float s_est;
     __shared__ unsigned s_nfit;
     __shared__ PdbGeo geo_s;
-    const unsigned n_list = p.ctl[0];
-    if (blockIdx.x >= n_list) return;
-    const int inst = p.restart_list[blockIdx.x];
+    const int inst = (int)blockIdx.x;
+    if (threadIdx.x == 0) {
+        // nothing to do while the current iteration runs and no lookahead is
+        // asked for
+        const int live = p.nlive[inst], at = inst * 2 + (p.it[inst] & 1);
+        const bool ended = live > 0 && slot_pend(p, at) == 0;
+        s_j = !p.done[inst] && (live == 0 || ended || p.want_next[inst]) ? 1 : 0;
+        if (live > 0) p.drained[at] = ended;
+        if (live > 1) p.drained[at ^ 1] = slot_pend(p, at ^ 1) == 0;
+    }
+    __syncthreads();
+    if (!s_j) return;
+    __syncthreads();
     const unsigned nf = min(p.nfront[inst], (unsigned)p.capl);
     const Item *F = p.frontier + (size_t)inst * p.capl;
     unsigned long long *load = p.load + (size_t)inst * p.capl;
@@ -1077,8 +1520,10 @@ __global__ void __launch_bounds__(256) k_restart(KParams p, const PdbGeo *geo_g)
             p.L[isl] = L;
             p.itn[isl] = it;
             p.found[isl] = p.top_goal[inst] <= L ? p.top_goal[inst] : kNoGoal;
-            p.cnt[isl] = s_cnt;
-            p.pend[isl] = off;
+            for (int x = 0; x < kGroups; ++x) {
+                p.cnt[x * p.gstride + isl] = x ? 0ull : s_cnt;
+                p.pend[x * p.gstride + isl] = x ? 0u : off;
+            }
             p.drained[isl] = off == 0 ? 1 : 0;
             p.dead[isl] = 0;
         }
@@ -1128,30 +1573,36 @@ __global__ void __launch_bounds__(256) k_restart(KParams p, const PdbGeo *geo_g)
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        p.want_next[inst] = 0;
-        p.listed[inst] = 0;
-    }
+    if (threadIdx.x == 0) p.want_next[inst] = 0;
 }
 
-// k_spec (lookahead): after a round, while idle lanes outnumber the queued
-// items by more than 1/32 of the lanes, put instances that run a single
-// iteration (no goal yet, and a previous iteration, if any, of at least one
-// node per lane) on the restart list with lookahead asked for, until their
-// frontiers would fill the idle lanes.  Instances are taken from a
-// start that rotates with the round number.  Only the schedule changes: each
-// iteration's count is its own, and the result is resolved in order.
+// k_spec (lookahead): after a round, while the waves without work outnumber
+// the queued items by more than 1/32 of the lanes, ask for lookahead for
+// instances that run a single iteration (no goal yet, and a previous
+// iteration, if any, of at least one node per lane), until their frontiers
+// would fill them.  Instances are taken from a start that rotates with the
+// round number.  Only the schedule changes: each iteration's count is its own,
+// and the result is resolved in order.
+// items of ring r not taken yet
+__device__ __forceinline__ unsigned long long q_waiting(const KParams &p, int r) {
+    const unsigned long long tail = p.q_ctl[kQTail + r * kQRing];
+    unsigned long long n = 0;
+    for (int x = 0; x < kGroups; ++x) {
+        const unsigned long long h = p.q_ctl[kQHead + r * kQRing + x * kLine];
+        if (h < tail) n += (tail - h + kGroups - 1) / kGroups;
+    }
+    return n;
+}
+
 __global__ void __launch_bounds__(256) k_spec(KParams p) {
     __shared__ unsigned long long s_room, s_used;
+    const unsigned idle = idle_waves(p);
     if (threadIdx.x == 0) {
         unsigned long long qlen = 0;
-        for (int r = 0; r < 2; ++r) {
-            const unsigned long long *c = p.q_ctl + kQCtl * r;
-            const unsigned long long head = c[0], lim = c[1], tail = c[2];
-            qlen += tail - (head < lim ? head : lim);
-        }
-        const unsigned long long lanes = (unsigned long long)p.n_lanes, busy = p.ctl[2];
-        const unsigned long long taken = busy + qlen;
+        for (int r = 0; r < 2; ++r) qlen += q_waiting(p, r);
+        // a queued item feeds a wave
+        const unsigned long long lanes = (unsigned long long)p.n_lanes;
+        const unsigned long long taken = lanes - 64ull * idle + 64ull * qlen;
         s_room = (taken < lanes && lanes - taken >= lanes / 32) ? lanes - taken : 0ull;
         s_used = 0;
     }
@@ -1162,70 +1613,67 @@ __global__ void __launch_bounds__(256) k_spec(KParams p) {
     for (int k = threadIdx.x; k < n; k += blockDim.x) {
         int inst = start + k;
         if (inst >= n) inst -= n;
-        if (p.done[inst] || p.nlive[inst] != 1 || p.listed[inst]) continue;
+        if (p.done[inst] || p.nlive[inst] != 1) continue;
         const int cur = p.it[inst];
         const int isc = inst * 2 + (cur & 1);
-        if (cur + 1 >= p.max_iters || p.found[isc] != kNoGoal || p.drained[isc]) continue;
+        if (cur + 1 >= p.max_iters || p.found[isc] != kNoGoal || slot_pend(p, isc) == 0) continue;
         // an instance whose last finished iteration counted fewer nodes than
         // there are lanes has iterations that end within a round or two:
         // lookahead would mostly run work that its goal then drops (100
         // 40-move 15-puzzles: 3200 instances/s with it, 5300 without)
         if (cur > 0 && p.iter_counts[(size_t)inst * p.max_iters + cur - 1] < (unsigned long long)p.n_lanes) continue;
         const unsigned long long est = min(p.nfront[inst], (unsigned)p.capl);
-        if (atomicAdd(&s_used, est) >= s_room) continue;
-        if (atomicExch(&p.listed[inst], 1) == 0) {
-            p.want_next[inst] = 1;
-            const unsigned k2 = atomicAdd(&p.ctl[0], 1u);
-            p.restart_list[k2] = inst;
-        }
+        if (atomicAdd(&s_used, 8ull * est) >= s_room) continue;
+        p.want_next[inst] = 1;
     }
 }
 
 // k_control: between rounds.  Publishes the items appended to both rings
-// during the last round, sizes the donation quotas from the number of idle
-// lanes, and picks the next round's step budget.  ctl[9] = budget used when
-// the queue can keep every lane busy, ctl[10] = budget while it cannot.
-// Lanes on current iterations (ctl[4]) donate to fill the idle lanes not
-// covered by ring 0; lanes on lookahead iterations (ctl[19]) only where both
-// rings together fall short, at most kAheadDonate nodes per lane and round,
-// and their items wait behind ring 0's.  A lookahead iteration's work is
-// dropped when the current one ends the search; spread wide it also holds
-// lanes, round after round, that the current iteration's tail needs (one
-// random 15-puzzle per launch: caps of 1 / 2 / 4 / 8 / 32 gave 43.0 / 44.7 /
-// 44.1 / 42.7 / 42.3 instances/s, and no donation at all 38.7).
-constexpr unsigned kAheadDonate = 2;
-__device__ __forceinline__ unsigned donate_quota(const KParams &p, unsigned long long idle,
-                                                 unsigned long long queued, unsigned long long donors) {
-    if (queued >= idle || donors == 0) return 0;
-    unsigned long long per = (idle - queued + donors - 1) / donors;
-    // donations of one round stay below a quarter of a ring
-    const unsigned long long cap = ((p.qmask + 1ull) / 4ull) / donors;
-    if (per > cap) per = cap;
-    return (unsigned)(per > 32ull ? 32ull : per);
-}
-
-__global__ void k_control(KParams p) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    unsigned long long qlen[2];
-    for (int r = 0; r < 2; ++r) {
-        unsigned long long *c = p.q_ctl + kQCtl * r;
-        unsigned long long head = c[0], limit = c[1], tail = c[2];
-        if (head > limit) head = limit;
-        c[0] = head;
-        c[1] = tail;
-        qlen[r] = tail - head;
+// during the last round, sets how many a wave takes at once (an even share of
+// the queue, so that few items reach many waves), and clears the round's
+// words: whoever still waits on a list waits no more.  One wave, a word a lane.
+__global__ void __launch_bounds__(64) k_control(KParams p) {
+    const int lane = threadIdx.x;
+    unsigned long long items = 0;
+    if (lane < 2 * kGroups) {
+        const int r = lane / kGroups, x = lane % kGroups;
+        unsigned long long *head = p.q_ctl + kQHead + r * kQRing + x * kLine;
+        const unsigned long long limit = p.q_ctl[kQTail + r * kQRing + 1], tail = p.q_ctl[kQTail + r * kQRing];
+        unsigned long long h = *head;
+        // a head past the limit goes back to the group's first position there
+        if (h >= limit + kGroups) h = limit + ((unsigned)(x - (int)(limit % kGroups)) & (kGroups - 1));
+        *head = h;
+        if (h < tail) items = (tail - h + kGroups - 1) / kGroups;
+    } else if (lane < 3 * kGroups) {
+        p.q_ctl[kQStart + (lane - 2 * kGroups) * kLine] = 0;
     }
-    const unsigned busy = p.ctl[2], busy1 = p.ctl[34];
-    p.ctl[2] = 0;
-    p.ctl[34] = 0;
-    p.ctl[12] = busy; // lanes busy at the end of the last round, for the host
-    p.ctl[0] = 0;     // restart list consumed
-    const unsigned long long lanes = (unsigned long long)p.n_lanes;
-    const unsigned long long idle = lanes > busy ? lanes - busy : 0ull;
-    p.ctl[4] = donate_quota(p, idle, qlen[0], busy - busy1);
-    p.ctl[19] = min(donate_quota(p, idle, qlen[0] + qlen[1], busy1), kAheadDonate);
-    p.ctl[5] = (qlen[0] + qlen[1] + busy >= lanes / 2) ? p.ctl[9] : p.ctl[10];
-    p.ctl[6] += 1;
+    static_assert(kLists == 64, "a list a lane");
+    unsigned long long *list = p.q_ctl + kQList + lane * kLine;
+    const unsigned long long w = list[0];
+    unsigned idle = waiting(w);
+    unsigned long long given = list[1];
+    list[0] = (w & 0xffffffff00000000ull) | (w >> 32);
+    list[1] = 0;
+    for (int off = 32; off > 0; off >>= 1) {
+        items += shfl_xor_u64(items, off);
+        given += shfl_xor_u64(given, off);
+        idle += __shfl_xor(idle, off);
+    }
+    __syncthreads(); // the limits are read
+    if (lane < 2) {
+        unsigned long long *c = p.q_ctl + kQTail + lane * kQRing;
+        c[1] = c[0];
+    }
+    if (lane == 0) {
+        const unsigned n_waves = (unsigned)p.n_lanes >> 6;
+        *p.stop = 0;
+        p.ctl[7] += (unsigned)given;
+        p.ctl[12] = n_waves - idle;  // waves with work at the round's end, for the host
+        p.ctl[20] = items > 0xffffffffull ? 0xffffffffu : (unsigned)items;
+        const unsigned long long share = (items + n_waves - 1) / n_waves;
+        p.ctl[4] = share < 1 ? 1u : share > 64 ? 64u : (unsigned)share;
+        p.ctl[6] += 1;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1414,11 +1862,11 @@ template <int W, int HEUR>
 static hipError_t launch_round_t(const KParams &p, const PdbGeo *geo, int wg, hipStream_t s, hipEvent_t t0,
                                  hipEvent_t t1) {
     size_t lds = round_lds_bytes(W, p.maxd, wg, HEUR);
+    auto *const k = p.prof ? &k_round<W, HEUR, true> : &k_round<W, HEUR, false>;
     if (t0 && t1)
-        hipExtLaunchKernelGGL((k_round<W, HEUR>), dim3(p.n_lanes / wg), dim3(wg), (uint32_t)lds, s, t0, t1, 0u, p,
-                              geo);
+        hipExtLaunchKernelGGL(k, dim3(p.n_lanes / wg), dim3(wg), (uint32_t)lds, s, t0, t1, 0u, p, geo);
     else
-        hipLaunchKernelGGL((k_round<W, HEUR>), dim3(p.n_lanes / wg), dim3(wg), lds, s, p, geo);
+        hipLaunchKernelGGL(k, dim3(p.n_lanes / wg), dim3(wg), lds, s, p, geo);
     return hipGetLastError();
 }
 
@@ -1437,9 +1885,9 @@ size_t round_lds_bytes(int width, int maxd, int wg, int heur) {
 }
 
 const void *round_kernel_ptr(int width, int heur) {
-    if (width == 4) return (const void *)&k_round<4, 0>;
-    if (heur == 0) return (const void *)&k_round<5, 0>;
-    return (const void *)&k_round<5, 1>;
+    if (width == 4) return (const void *)&k_round<4, 0, false>;
+    if (heur == 0) return (const void *)&k_round<5, 0, false>;
+    return (const void *)&k_round<5, 1, false>;
 }
 
 hipError_t launch_restart(int width, int heur, const KParams &p, const PdbGeo *geo, hipStream_t s) {
