@@ -35,8 +35,7 @@ hipError_t launch_eval_h(int width, int heur, const KParams &p, const PdbGeo *ge
 hipError_t launch_scatter_roots(const Item *roots, Item *lvl, int capl, int n, hipStream_t s);
 hipError_t launch_eval_h_bytes(int width, int heur, const uint8_t *bytes, int n, const PdbGeo *geo,
                                const uint8_t *pdb, int *h, hipStream_t s);
-hipError_t pdb_bfs_build(int pat, uint8_t *compact, uint32_t *work, unsigned long long *d_cnt, hipStream_t s,
-                         int *levels_out);
+hipError_t pdb_bfs_build(int pat, uint8_t *compact, uint32_t *work, unsigned *d_any, hipStream_t s, int *levels_out);
 hipError_t pdb_spread(const uint8_t *compact, uint8_t *direct, hipStream_t s);
 hipError_t launch_gather_probe(const uint8_t *t, uint64_t span, int blocks, int per_thread, uint64_t seed, uint32_t *out,
                                hipStream_t s);
@@ -673,7 +672,7 @@ int spz_build_pdb(spz_ctx *ctx, const char *cache_path) try {
     }
     DBuf work, cntb;
     hipError_t e = work.ensure(3ull * kPlacementsHost * 4);
-    if (e == hipSuccess) e = cntb.ensure(8);
+    if (e == hipSuccess) e = cntb.ensure(256 * 4);
     if (e != hipSuccess) {
         work.release();
         cntb.release();
@@ -682,8 +681,8 @@ int spz_build_pdb(spz_ctx *ctx, const char *cache_path) try {
     auto t0 = std::chrono::steady_clock::now();
     for (int t = 0; t < 2; ++t) {
         int levels = 0;
-        e = pdb_bfs_build(t, ctx->pdb_compact[t].as<uint8_t>(), work.as<uint32_t>(),
-                          cntb.as<unsigned long long>(), ctx->stream, &levels);
+        e = pdb_bfs_build(t, ctx->pdb_compact[t].as<uint8_t>(), work.as<uint32_t>(), cntb.as<unsigned>(), ctx->stream,
+                          &levels);
         if (e != hipSuccess) break;
         ctx->stats[4 + t] = levels;
     }

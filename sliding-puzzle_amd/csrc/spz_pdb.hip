@@ -9,9 +9,9 @@
 //   Level 0 is the goal (pattern tiles home, blank at cell 0) closed under
 //   0-cost moves; a table entry is the first level that reaches any blank
 //   cell of that placement, i.e. the minimum over blank cells.
-// Per placement the BFS keeps three 25-bit masks of blank cells (seen, in
-// the current level, reached for the next level), indexed by the placement's
-// rank in the reference's file order (25!/19! = 127,512,000 placements).
+// Per placement the BFS keeps three 25-bit masks of blank cells (seen, and
+// reached for this and for the next level), indexed by the placement's rank in
+// the reference's file order (25!/19! = 127,512,000 placements).
 // The finished compact table is then spread into direct 25^6 addressing so
 // that the search updates an index with one multiply-add per move.
 #include "spz_board.h"
@@ -98,6 +98,20 @@ uint32_t pdb_goal_rank(int t) {
     return rank;
 }
 
+// the n-th set bit of a mask of 25 bits, by halving
+__device__ __forceinline__ int nth_bit(uint32_t m, int n) {
+    int at = 0;
+#pragma unroll
+    for (int w = 16; w > 0; w >>= 1) {
+        const int c = __builtin_popcount((m >> at) & ((1u << w) - 1u));
+        if (n >= c) {
+            n -= c;
+            at += w;
+        }
+    }
+    return at;
+}
+
 __device__ __forceinline__ void pl_unrank(uint32_t rank, int (&s)[6]) {
     int dig[6];
 #pragma unroll
@@ -108,9 +122,7 @@ __device__ __forceinline__ void pl_unrank(uint32_t rank, int (&s)[6]) {
     uint32_t used = 0;
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
-        uint32_t free_ = ~used & kFull25;
-        for (int k = 0; k < dig[i]; ++k) free_ &= free_ - 1u;
-        s[i] = __builtin_ctz(free_);
+        s[i] = nth_bit(~used & kFull25, dig[i]);
         used |= 1u << s[i];
     }
 }
@@ -129,84 +141,58 @@ __device__ __forceinline__ uint32_t flood5(uint32_t seed, uint32_t free_) {
     }
 }
 
-__device__ __forceinline__ int nb5(int cell, int d) {
-    int r = cell / 5, c = cell - r * 5;
-    if (d == DIR_UP) return r > 0 ? cell - 5 : -1;
-    if (d == DIR_RIGHT) return c < 4 ? cell + 1 : -1;
-    if (d == DIR_LEFT) return c > 0 ? cell - 1 : -1;
-    return r < 4 ? cell + 5 : -1;
-}
-
-// level d -> candidates of level d+1
-__global__ void __launch_bounds__(256) k_bfs_expand(const uint32_t *__restrict__ cur, const uint32_t *__restrict__ seen,
-                                                    uint32_t *nxt) {
-    uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
+// One level: every placement's candidates of the level are closed under
+// 0-cost blank moves, what is new recorded, and its pattern moves made
+// candidates of the next level.  A candidate set whose placement is closed
+// later in the same launch is masked then, so the two halves need no launch
+// of their own and no array of the current level between them: per level the
+// launch reads one mask a placement (510 MB) and touches the rest only where
+// the level has something.  any: set if the level had something new (a plain
+// store of the same value, once seen unset: counting the waves with an atomic
+// on one address took 5.5 ms a level).  Measured on MI355X, both tables: 539
+// ms as two launches a level with the count, 74 ms so.
+__global__ void __launch_bounds__(256) k_bfs_level(uint32_t *__restrict__ cand, uint32_t *seen, uint32_t *next,
+                                                   uint8_t *val, int level, unsigned *any) {
+    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= kPlacements) return;
-    uint32_t m = cur[p];
+    uint32_t m = cand[p];
     if (!m) return;
+    cand[p] = 0;
     int s[6];
     pl_unrank(p, s);
     uint32_t occ = 0;
 #pragma unroll
     for (int j = 0; j < 6; ++j) occ |= 1u << s[j];
-    while (m) {
-        int b = __builtin_ctz(m);
-        m &= m - 1u;
+    const uint32_t old = seen[p];
+    m = flood5(m, kFull25 & ~occ) & ~old;
+    if (!m) return;
+    if (val[p] == 0xffu) val[p] = (uint8_t)level;
+    seen[p] = old | m;
+    if (*(volatile unsigned *)any == 0u) *(volatile unsigned *)any = 1u;
+    // a pattern tile beside a new blank cell steps into it; the blank is then
+    // where the tile was
 #pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            int q = nb5(b, d);
-            if (q < 0 || !(occ & (1u << q))) continue;
+    for (int j = 0; j < 6; ++j) {
+        const int q = s[j];
+        const uint32_t beside = dilate5(1u << q) & m;
+#pragma unroll 1
+        for (uint32_t b = beside; b; b &= b - 1u) {
             int s2[6];
 #pragma unroll
-            for (int j = 0; j < 6; ++j) s2[j] = (s[j] == q) ? b : s[j]; // the tile steps into the blank
-            uint32_t p2 = pl_rank(s2);
-            uint32_t bit = 1u << q; // the blank is where the tile was
-            if (!(seen[p2] & bit)) atomicOr(&nxt[p2], bit);
+            for (int i = 0; i < 6; ++i) s2[i] = i == j ? __builtin_ctz(b) : s[i];
+            const uint32_t p2 = pl_rank(s2);
+            if (!(seen[p2] & (1u << q))) atomicOr(&next[p2], 1u << q);
         }
     }
 }
 
-// close the candidates under 0-cost blank moves; record first levels
-__global__ void __launch_bounds__(256) k_bfs_close(uint32_t *cur, uint32_t *seen, uint32_t *nxt, uint8_t *val,
-                                                   int level, unsigned long long *n_new) {
-    uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    uint32_t hit = 0;
-    if (p < kPlacements) {
-        uint32_t m = nxt[p];
-        if (m) {
-            nxt[p] = 0;
-            int s[6];
-            pl_unrank(p, s);
-            uint32_t occ = 0;
-#pragma unroll
-            for (int j = 0; j < 6; ++j) occ |= 1u << s[j];
-            m = flood5(m, kFull25 & ~occ) & ~seen[p];
-            if (m) {
-                if (val[p] == 0xffu) val[p] = (uint8_t)level;
-                seen[p] |= m;
-                hit = 1;
-            }
-        }
-        cur[p] = m;
-    }
-    uint64_t b = __ballot(hit);
-    if ((threadIdx.x & 63) == 0 && b) atomicAdd(n_new, (unsigned long long)__popcll(b));
-}
-
-__global__ void k_bfs_seed(uint32_t *cur, uint32_t *seen, uint8_t *val, int pat) {
+// level 0: the goal placement's candidates
+__global__ void k_bfs_seed(uint32_t *cand, int pat) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     int s[6];
     const int A[6] = {1, 2, 5, 6, 7, 12}, B[6] = {3, 4, 8, 9, 13, 14};
-    uint32_t occ = 0;
-    for (int j = 0; j < 6; ++j) {
-        s[j] = pat == 0 ? A[j] : B[j];
-        occ |= 1u << s[j];
-    }
-    uint32_t p = pl_rank(s);
-    uint32_t m = flood5(1u, kFull25 & ~occ); // blank at cell 0, closed under 0-cost moves
-    cur[p] = m;
-    seen[p] = m;
-    val[p] = 0;
+    for (int j = 0; j < 6; ++j) s[j] = pat == 0 ? A[j] : B[j];
+    cand[pl_rank(s)] = 1u; // blank at cell 0
 }
 
 // compact (file order) -> direct 25^6 addressing; invalid tuples get 0
@@ -261,26 +247,36 @@ hipError_t launch_gather_probe(const uint8_t *t, uint64_t span, int blocks, int 
 
 // ---------------------------------------------------------------------------
 // Host driver: builds canonical table `pat` (0 or 1) into `compact` (device,
-// kPlacements bytes).  Scratch: 3 x kPlacements u32.  Returns levels run.
-hipError_t pdb_bfs_build(int pat, uint8_t *compact, uint32_t *work, unsigned long long *d_cnt, hipStream_t s,
-                         int *levels_out) {
-    uint32_t *seen = work, *cur = work + kPlacements, *nxt = work + 2ull * kPlacements;
+// kPlacements bytes).  Scratch: 3 x kPlacements u32 and d_any, 256 u32.
+// levels_out: levels run, the last of them empty.
+hipError_t pdb_bfs_build(int pat, uint8_t *compact, uint32_t *work, unsigned *d_any, hipStream_t s, int *levels_out) {
+    uint32_t *seen = work, *a = work + kPlacements, *b = work + 2ull * kPlacements;
     hipError_t e;
     if ((e = hipMemsetAsync(work, 0, 3ull * kPlacements * 4, s)) != hipSuccess) return e;
     if ((e = hipMemsetAsync(compact, 0xff, kPlacements, s)) != hipSuccess) return e;
-    hipLaunchKernelGGL(k_bfs_seed, dim3(1), dim3(64), 0, s, cur, seen, compact, pat);
-    dim3 grid((kPlacements + 255) / 256);
-    int level = 0;
-    for (; level < 254; ++level) {
-        hipLaunchKernelGGL(k_bfs_expand, grid, dim3(256), 0, s, cur, seen, nxt);
-        if ((e = hipMemsetAsync(d_cnt, 0, 8, s)) != hipSuccess) return e;
-        hipLaunchKernelGGL(k_bfs_close, grid, dim3(256), 0, s, cur, seen, nxt, compact, level + 1, d_cnt);
-        unsigned long long h = 0;
-        if ((e = hipMemcpyAsync(&h, d_cnt, 8, hipMemcpyDeviceToHost, s)) != hipSuccess) return e;
+    if ((e = hipMemsetAsync(d_any, 0, 256 * 4, s)) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_bfs_seed, dim3(1), dim3(64), 0, s, a, pat);
+    const dim3 grid((kPlacements + 255) / 256);
+    // the host looks after every few levels; a level after the last is a scan
+    // of empty masks
+    constexpr int kLook = 6;
+    unsigned any[256];
+    int level = 0, last = -1;
+    while (level < 255 && last < 0) {
+        const int from = level;
+        for (; level < 255 && level < from + kLook; ++level) {
+            hipLaunchKernelGGL(k_bfs_level, grid, dim3(256), 0, s, a, seen, b, compact, level, d_any + level);
+            uint32_t *t = a;
+            a = b;
+            b = t;
+        }
+        if ((e = hipMemcpyAsync(any + from, d_any + from, (size_t)(level - from) * 4, hipMemcpyDeviceToHost, s)) != hipSuccess)
+            return e;
         if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
-        if (h == 0) break;
+        for (int l = from; l < level && last < 0; ++l)
+            if (!any[l]) last = l;
     }
-    if (levels_out) *levels_out = level + 1;
+    if (levels_out) *levels_out = last < 0 ? 255 : last;
     return hipGetLastError();
 }
 
