@@ -268,10 +268,11 @@ int spz_get_paths(spz_ctx *ctx, uint8_t *moves, int32_t max_len, int32_t *lens);
  *                                                  without work
  *  3 lanes                 4,5 PDB BFS levels     6 PDB build ms
  *  7 stack-overflow items  8 round-kernel ms (sum, when time_kernels)
- *  9 round launches timed  10 split ms            11 instances
+ *  9 round launches timed  10 split ms (enqueue)  11 instances
  *  12 nodes (all instances, all iterations)
- *  13 setup ms (upload, root split, first restart)  14 rounds wall ms
- *  15 1 if the rounds ran from a hipGraph
+ *  13 setup ms (to the first restart's enqueue)  14 rounds wall ms (with
+ *     what of the setup still ran)
+ *  15 1 if the rounds ran from a hipGraph (all but the first poll period)
  *  16-19 with env SPZ_PROFILE=1: lane-steps idle, expanding, only popping,
  *        and wave-steps (x64 = lane-steps) of the search rounds;
  *  20-22 with SPZ_PROFILE=1 (PDB): moves into a sibling (2 table reads each),

@@ -26,13 +26,14 @@ hipError_t launch_restart(int width, int heur, const KParams &p, const PdbGeo *g
 hipError_t launch_spec(const KParams &p, hipStream_t s);
 hipError_t launch_control(const KParams &p, hipStream_t s);
 hipError_t launch_split_level(int width, int heur, const KParams &p, const PdbGeo *geo, const Item *lvl_in,
-                              const unsigned *n_in, Item *lvl_out, unsigned *n_out, unsigned *nfront,
-                              unsigned *topgen, int *top_goal, int *frozen, int depth, int max_depth,
-                              unsigned target, const unsigned long long *lp_in, unsigned long long *lp_out,
-                              unsigned long long *fp_out, hipStream_t s);
+                              const unsigned *n_in, Item *lvl_out, unsigned *n_out, int *frozen, int depth,
+                              int max_depth, unsigned target, const unsigned long long *lp_in,
+                              unsigned long long *lp_out, hipStream_t s);
+hipError_t launch_begin(int width, int heur, const KParams &p, const PdbGeo *geo, Item *lvl0, Item *lvl1,
+                        unsigned *nlvl0, int *frozen, int max_depth, unsigned target, unsigned long long *lp0,
+                        unsigned long long *lp1, bool split, unsigned n_list, hipStream_t s);
 hipError_t launch_eval_h(int width, int heur, const KParams &p, const PdbGeo *geo, Item *items, int n,
                          hipStream_t s);
-hipError_t launch_scatter_roots(const Item *roots, Item *lvl, int capl, int n, hipStream_t s);
 hipError_t launch_eval_h_bytes(int width, int heur, const uint8_t *bytes, int n, const PdbGeo *geo,
                                const uint8_t *pdb, int *h, hipStream_t s);
 hipError_t pdb_bfs_build(int pat, uint8_t *compact, uint32_t *work, unsigned *d_any, hipStream_t s, int *levels_out);
@@ -125,6 +126,10 @@ static hipError_t scratch_for_device(int dev, void **out) {
     return hipSuccess;
 }
 
+// layout of a context's head buffer: 64 control words, kQCtlWords queue-control
+// words on lines of their own, the roots
+constexpr size_t kHeadQCtl = 256, kHeadRoots = kHeadQCtl + (size_t)kQCtlWords * 8;
+
 struct spz_ctx {
     spz_config cfg;
     hipStream_t stream = nullptr;
@@ -147,12 +152,15 @@ struct spz_ctx {
     // lane contexts
     DBuf c_st, c_rows, c_meta, c_inst, c_cnt, c_pdb, c_stack;
     // queue and control
-    DBuf q, q_ctl, ctl;
+    DBuf q;
+    DBuf head;    // control words, queue-control words, then the roots: one upload
+    DBuf results; // per instance: optimum, last iteration, h0, then the counts: one download
+    HBuf stage;   // pinned staging of both, and of the control words polled
     DBuf list, mail, mail_head, ticket, mail_path; // waves without work
     size_t qcap = 0;
     // per instance
-    DBuf roots, L, it, cnt, pend, found, done, opt, iter_counts;
-    DBuf itn, drained, dead, nlive, Lbase, want_next; // iteration slots (lookahead)
+    DBuf L, cnt, pend, found, done;
+    DBuf itn, drained, dead, nlive, want_next; // iteration slots (lookahead)
     DBuf frontier, nfront, topgen, top_goal, frozen, lvl[2], nlvl[2];
     // load balancing
     DBuf c_origin, load, samples, nsamp, pred;
@@ -276,6 +284,11 @@ constexpr int kLanesPerCuPdb = 768;
 // 524288 5.4; 250 mixed ones, 16 each: 131072 lanes 1513 ms, 256000 1040,
 // 524288 1030).
 constexpr size_t kLanesPerItem = 64;
+// largest root-split target that a workgroup per instance splits (k_begin)
+constexpr unsigned kOneBlockSplit = 16384;
+// largest upload or download through pinned staging; larger ones stream from
+// and to pageable memory
+constexpr size_t kMaxStage = 16u << 20;
 // A round ends early once the waves that ran out of work have waited, summed
 // over them and divided by all waves, this long: about what it costs to end a
 // round, save and restore the lanes, start iterations and feed the waves again.
@@ -398,7 +411,7 @@ int spz_create(spz_ctx **out, const spz_config *cfg) try {
         pdb_geo_build(&ctx->geo_h);
         if ((e = ctx->geo_d.ensure(sizeof(PdbGeo))) != hipSuccess ||
             (e = hipMemcpy(ctx->geo_d.p, &ctx->geo_h, sizeof(PdbGeo), hipMemcpyHostToDevice)) != hipSuccess ||
-            (e = ctx->q_ctl.ensure(kQCtlWords * 8)) != hipSuccess || (e = ctx->ctl.ensure(64 * 4)) != hipSuccess) {
+            (e = ctx->head.ensure(kHeadRoots)) != hipSuccess) {
             rc = fail(ctx, SPZ_E_HIP, "context allocation: %s", hipGetErrorString(e));
             break;
         }
@@ -534,25 +547,21 @@ const char *spz_last_error(spz_ctx *ctx) { return ctx ? ctx->err.c_str() : "null
 
 void spz_destroy(spz_ctx *ctx) {
     if (!ctx) return;
-    DBuf *all[] = {&ctx->geo_d,       &ctx->pdb_compact[0], &ctx->pdb_compact[1], &ctx->pdb_direct,
-                   &ctx->c_st,         &ctx->c_rows,
-                   &ctx->c_meta,      &ctx->c_inst,         &ctx->c_cnt,
-                   &ctx->c_pdb,       &ctx->c_stack,        &ctx->q,              &ctx->q_ctl,
-                   &ctx->ctl,         &ctx->roots,          &ctx->L,              &ctx->it,
-                   &ctx->cnt,         &ctx->pend,           &ctx->found,          &ctx->done,
-                   &ctx->opt,         &ctx->iter_counts,    &ctx->frontier,
-                   &ctx->nfront,      &ctx->topgen,         &ctx->top_goal,       &ctx->frozen,
-                   &ctx->lvl[0],      &ctx->lvl[1],         &ctx->nlvl[0],        &ctx->nlvl[1],
-                   &ctx->c_origin,    &ctx->load,           &ctx->samples,        &ctx->nsamp,
-                   &ctx->pred,        &ctx->qpath,          &ctx->c_ipath,        &ctx->fpath,
-                   &ctx->lpath[0],    &ctx->lpath[1],       &ctx->sol,            &ctx->sol_len,
-                   &ctx->itn,         &ctx->drained,        &ctx->nlive,          &ctx->Lbase,
-                   &ctx->list,        &ctx->mail,           &ctx->mail_head,      &ctx->ticket,
-                   &ctx->mail_path,   &ctx->want_next,      &ctx->dead,           &ctx->prof,
-                   &ctx->wtime};
+    DBuf *all[] = {&ctx->geo_d,   &ctx->pdb_compact[0], &ctx->pdb_compact[1], &ctx->pdb_direct, &ctx->c_st,
+                   &ctx->c_rows,  &ctx->c_meta,         &ctx->c_inst,         &ctx->c_cnt,      &ctx->c_pdb,
+                   &ctx->c_stack, &ctx->q,              &ctx->head,           &ctx->results,    &ctx->L,
+                   &ctx->cnt,     &ctx->pend,           &ctx->found,          &ctx->done,       &ctx->frontier,
+                   &ctx->nfront,  &ctx->topgen,         &ctx->top_goal,       &ctx->frozen,     &ctx->lvl[0],
+                   &ctx->lvl[1],  &ctx->nlvl[0],        &ctx->nlvl[1],        &ctx->c_origin,   &ctx->load,
+                   &ctx->samples, &ctx->nsamp,          &ctx->pred,           &ctx->qpath,      &ctx->c_ipath,
+                   &ctx->fpath,   &ctx->lpath[0],       &ctx->lpath[1],       &ctx->sol,        &ctx->sol_len,
+                   &ctx->itn,     &ctx->drained,        &ctx->nlive,          &ctx->list,       &ctx->mail,
+                   &ctx->mail_head, &ctx->ticket,       &ctx->mail_path,      &ctx->want_next,  &ctx->dead,
+                   &ctx->prof,    &ctx->wtime};
     for (DBuf *b : all) b->release();
     ctx->dd_items.release();
     ctx->dd_paths.release();
+    ctx->stage.release();
     if (ctx->mlp_alloced) mlp_free(ctx->mlp);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -765,32 +774,35 @@ static BoardKey board_key(int width, const Item &it) {
 static hipError_t dedup_level(spz_ctx *ctx, int n, int capl, int width, int cur, bool paths,
                               std::vector<SeenBoards> &seen, hipStream_t s);
 
+// offset of the per-iteration counts in the results buffer
+static size_t results_counts(size_t n) { return (3 * n * 4 + 7) / 8 * 8; }
+
 static KParams base_params(spz_ctx *ctx, int n, int max_iters, int capl) {
     KParams p;
     memset(&p, 0, sizeof p);
     p.q = ctx->q.as<Item>();
     p.qmask = ctx->qcap - 1;
-    p.q_ctl = ctx->q_ctl.as<unsigned long long>();
+    p.ctl = ctx->head.as<unsigned>();
+    p.q_ctl = (unsigned long long *)(ctx->head.as<uint8_t>() + kHeadQCtl);
     p.stop = (unsigned *)(p.q_ctl + kQStop);
     p.n_inst = n;
     p.max_iters = max_iters;
     p.mode = ctx->cfg.mode;
-    p.roots = ctx->roots.as<Item>();
+    p.roots = (Item *)(ctx->head.as<uint8_t>() + kHeadRoots);
     p.L = ctx->L.as<int>();
-    p.it = ctx->it.as<int>();
     p.itn = ctx->itn.as<int>();
     p.drained = ctx->drained.as<int>();
     p.dead = ctx->dead.as<int>();
     p.nlive = ctx->nlive.as<int>();
-    p.Lbase = ctx->Lbase.as<int>();
     p.want_next = ctx->want_next.as<int>();
     p.cnt = ctx->cnt.as<unsigned long long>();
     p.pend = ctx->pend.as<unsigned>();
     p.found = ctx->found.as<int>();
     p.done = ctx->done.as<int>();
-    p.opt = ctx->opt.as<int>();
-    p.iter_counts = ctx->iter_counts.as<unsigned long long>();
-    p.ctl = ctx->ctl.as<unsigned>();
+    p.opt = ctx->results.as<int>();
+    p.it = p.opt + n;
+    p.Lbase = p.it + n;
+    p.iter_counts = (unsigned long long *)(ctx->results.as<uint8_t>() + results_counts((size_t)n));
     p.frontier = ctx->frontier.as<Item>();
     p.nfront = ctx->nfront.as<unsigned>();
     p.topgen = ctx->topgen.as<unsigned>();
@@ -910,7 +922,16 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     ctx->qcap = qcap;
 
     HIPCHK(ctx->q.ensure(2 * qcap * sizeof(Item))); // ring 0: current iterations, ring 1: lookahead
-    HIPCHK(ctx->roots.ensure(N * sizeof(Item)));
+    HIPCHK(ctx->head.ensure(kHeadRoots + N * sizeof(Item)));
+    const size_t results_n = results_counts(N) + N * (size_t)max_iters * 8;
+    HIPCHK(ctx->results.ensure(results_n));
+    // pinned staging: control words polled (first 256 bytes), then the upload
+    // and later the results, where they are not too large to pin
+    const size_t head_n = kHeadRoots + N * sizeof(Item);
+    const bool pinned = std::max(head_n, results_n) <= kMaxStage;
+    HIPCHK(ctx->stage.ensure(256 + (pinned ? std::max(head_n, results_n) : 0)));
+    std::vector<uint8_t> pageable(pinned ? 0 : std::max(head_n, results_n));
+    uint8_t *const stage = pinned ? (uint8_t *)ctx->stage.p + 256 : pageable.data();
     HIPCHK(ctx->L.ensure(2 * N * 4));
     HIPCHK(ctx->itn.ensure(2 * N * 4));
     const size_t gstride = (2 * N + 31) / 32 * 32; // each group's part on lines of its own
@@ -926,13 +947,9 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     HIPCHK(ctx->found.ensure(2 * N * 4));
     HIPCHK(ctx->drained.ensure(2 * N * 4));
     HIPCHK(ctx->dead.ensure(2 * N * 4));
-    HIPCHK(ctx->it.ensure(N * 4));
     HIPCHK(ctx->nlive.ensure(N * 4));
-    HIPCHK(ctx->Lbase.ensure(N * 4));
     HIPCHK(ctx->want_next.ensure(N * 4));
     HIPCHK(ctx->done.ensure(N * 4));
-    HIPCHK(ctx->opt.ensure(N * 4));
-    HIPCHK(ctx->iter_counts.ensure(N * (size_t)max_iters * 8));
     HIPCHK(ctx->frontier.ensure(front_items * sizeof(Item)));
     HIPCHK(ctx->nfront.ensure(N * 4));
     HIPCHK(ctx->topgen.ensure(N * kFBins * 4));
@@ -983,9 +1000,6 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
         for (int k = 0; k < 2; ++k) HIPCHK(ctx->lpath[k].ensure(front_items * 8));
         HIPCHK(ctx->sol.ensure(2 * N * kPathWords * 4)); // per iteration slot
         HIPCHK(ctx->sol_len.ensure(2 * N * 4));
-        HIPCHK(hipMemsetAsync(ctx->lpath[0].p, 0, front_items * 8, s)); // the roots' empty paths
-        HIPCHK(hipMemsetAsync(ctx->sol.p, 0, 2 * N * kPathWords * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->sol_len.p, 0xff, 2 * N * 4, s)); // -1: none yet
         p.qpath = ctx->qpath.as<uint32_t>();
         p.c_ipath = ctx->c_ipath.as<uint32_t>();
         p.fpath = ctx->fpath.as<unsigned long long>();
@@ -993,45 +1007,48 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
         p.sol_len = ctx->sol_len.as<int>();
     }
 
-    // roots and their heuristic
-    std::vector<Item> roots(N);
+    // upload: control words, the queue's, the roots
+    unsigned *ctl = (unsigned *)stage;
+    memset(stage, 0, kHeadRoots);
+    ctl[1] = (unsigned)n; // active instances
+    ctl[5] = (unsigned)(ctx->cfg.round_budget > 0 ? ctx->cfg.round_budget : kRoundSteps);
+    unsigned long long *qc = (unsigned long long *)(stage + kHeadQCtl);
+    for (int r = 0; r < 2; ++r)
+        for (int x = 0; x < kGroups; ++x) qc[kQHead + r * kQRing + x * kLine] = (unsigned long long)x;
+    Item *roots = (Item *)(stage + kHeadRoots);
     for (int i = 0; i < n; ++i) pack_root(w, boards + (size_t)i * w * w, i, &roots[i]);
-    HIPCHK(hipMemcpyAsync(ctx->roots.p, roots.data(), N * sizeof(Item), hipMemcpyHostToDevice, s));
-    HIPCHK(launch_eval_h(w, heur, p, ctx->geo_d.as<PdbGeo>(), ctx->roots.as<Item>(), n, s));
-    HIPCHK(hipMemcpyAsync(roots.data(), ctx->roots.p, N * sizeof(Item), hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(ctx->head.p, stage, head_n, hipMemcpyHostToDevice, s));
 
-    // root split: level 0 holds the root of each instance at slot 0
-    HIPCHK(hipMemsetAsync(ctx->topgen.p, 0, N * kFBins * 4, s));
-    HIPCHK(hipMemsetAsync(ctx->frozen.p, 0, N * 4, s));
-    HIPCHK(hipMemsetAsync(ctx->nfront.p, 0, N * 4, s));
-    HIPCHK(hipStreamSynchronize(s));
-    {
-        std::vector<int> tg(N, kNoGoal);
-        HIPCHK(hipMemcpyAsync(ctx->top_goal.p, tg.data(), N * 4, hipMemcpyHostToDevice, s));
-        std::vector<unsigned> ones(N, 1u);
-        HIPCHK(hipMemcpyAsync(ctx->nlvl[0].p, ones.data(), N * 4, hipMemcpyHostToDevice, s));
-        HIPCHK(launch_scatter_roots(ctx->roots.as<Item>(), ctx->lvl[0].as<Item>(), capl, n, s));
-        HIPCHK(hipStreamSynchronize(s));
-    }
+    // state and root split; duplicate pruning works on the host between the
+    // split's levels, and a very large frontier is split by the whole device
     const int max_depth = ctx->cfg.max_split_depth;
+    const bool one_block = !ctx->cfg.dedup && target <= kOneBlockSplit;
     auto t_split = std::chrono::steady_clock::now();
-    int cur = 0;
-    std::vector<SeenBoards> seen(ctx->cfg.dedup ? N : 0);
-    // the closed list starts with the root (src_horie/idas_smem.cu:1068)
-    for (size_t i = 0; i < seen.size(); ++i)
-        seen[i].emplace_back(board_key(w, roots[i]), meta_h(roots[i].meta));
-    for (int depth = 0; depth <= max_depth; ++depth) {
-        if (ctx->cfg.dedup && depth > 0) HIPCHK(dedup_level(ctx, n, capl, w, cur, paths, seen, s));
-        HIPCHK(hipMemsetAsync(ctx->nlvl[cur ^ 1].p, 0, N * 4, s));
-        HIPCHK(launch_split_level(w, heur, p, ctx->geo_d.as<PdbGeo>(), ctx->lvl[cur].as<Item>(),
-                                  ctx->nlvl[cur].as<unsigned>(), ctx->lvl[cur ^ 1].as<Item>(),
-                                  ctx->nlvl[cur ^ 1].as<unsigned>(), ctx->nfront.as<unsigned>(),
-                                  ctx->topgen.as<unsigned>(), ctx->top_goal.as<int>(), ctx->frozen.as<int>(),
-                                  depth, max_depth, target,
-                                  paths ? ctx->lpath[cur].as<unsigned long long>() : nullptr,
-                                  paths ? ctx->lpath[cur ^ 1].as<unsigned long long>() : nullptr,
-                                  paths ? ctx->fpath.as<unsigned long long>() : nullptr, s));
-        cur ^= 1;
+    HIPCHK(launch_begin(w, heur, p, ctx->geo_d.as<PdbGeo>(), ctx->lvl[0].as<Item>(), ctx->lvl[1].as<Item>(),
+                        ctx->nlvl[0].as<unsigned>(), ctx->frozen.as<int>(), max_depth, target,
+                        paths ? ctx->lpath[0].as<unsigned long long>() : nullptr,
+                        paths ? ctx->lpath[1].as<unsigned long long>() : nullptr, one_block,
+                        (unsigned)(kLists * list_n), s));
+    if (!one_block) {
+        std::vector<SeenBoards> seen(ctx->cfg.dedup ? N : 0);
+        if (ctx->cfg.dedup) {
+            // the closed list starts with the root (src_horie/idas_smem.cu:1068)
+            std::vector<int> h0(N);
+            HIPCHK(hipMemcpyAsync(h0.data(), p.Lbase, N * 4, hipMemcpyDeviceToHost, s));
+            HIPCHK(hipStreamSynchronize(s));
+            for (size_t i = 0; i < N; ++i) seen[i].emplace_back(board_key(w, roots[i]), h0[i]);
+        }
+        int cur = 0;
+        for (int depth = 0; depth <= max_depth; ++depth) {
+            if (ctx->cfg.dedup && depth > 0) HIPCHK(dedup_level(ctx, n, capl, w, cur, paths, seen, s));
+            HIPCHK(hipMemsetAsync(ctx->nlvl[cur ^ 1].p, 0, N * 4, s));
+            HIPCHK(launch_split_level(w, heur, p, ctx->geo_d.as<PdbGeo>(), ctx->lvl[cur].as<Item>(),
+                                      ctx->nlvl[cur].as<unsigned>(), ctx->lvl[cur ^ 1].as<Item>(),
+                                      ctx->nlvl[cur ^ 1].as<unsigned>(), ctx->frozen.as<int>(), depth, max_depth,
+                                      target, paths ? ctx->lpath[cur].as<unsigned long long>() : nullptr,
+                                      paths ? ctx->lpath[cur ^ 1].as<unsigned long long>() : nullptr, s));
+            cur ^= 1;
+        }
     }
 
     if (getenv("SPZ_PROFILE") && atoi(getenv("SPZ_PROFILE")) > 0) {
@@ -1046,58 +1063,18 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
             p.wtime_round = (unsigned)atoi(getenv("SPZ_WAVE_TIMES"));
         }
     }
-    HIPCHK(hipMemsetAsync(ctx->load.p, 0, front_items * 8, s));
     HIPCHK(hipMemsetAsync(ctx->nsamp.p, 0, 64, s));
     if (ctx->cfg.lb_policy == SPZ_LB_LEARNED)
         HIPCHK(mlp_predict_frontier(ctx->mlp, w, ctx->frontier.as<Item>(), ctx->nfront.as<unsigned>(),
-                                    ctx->roots.as<Item>(), n, capl, ctx->pred.as<float>(), s));
-    HIPCHK(hipStreamSynchronize(s));
+                                    p.roots, n, capl, ctx->pred.as<float>(), s));
     ctx->stats[10] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_split).count();
 
-    // per-instance iteration state: every instance with no iteration
-    // started (k_restart starts iteration 0)
-    {
-        std::vector<int> Lh(N), nog(2 * N, kNoGoal), neg(N, -1);
-        for (int i = 0; i < n; ++i) {
-            Lh[i] = meta_h(roots[i].meta);
-        }
-        HIPCHK(hipMemcpyAsync(ctx->Lbase.p, Lh.data(), N * 4, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemsetAsync(ctx->L.p, 0, 2 * N * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->itn.p, 0, 2 * N * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->cnt.p, 0, kGroups * gstride * 8, s));
-        HIPCHK(hipMemsetAsync(ctx->pend.p, 0, kGroups * gstride * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->list.p, 0, kLists * list_n * 8, s));
-        HIPCHK(hipMemsetAsync(ctx->mail_head.p, 0, waves * kLine * 8, s));
-        HIPCHK(hipMemsetAsync(ctx->ticket.p, 0, waves * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->drained.p, 0, 2 * N * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->dead.p, 0, 2 * N * 4, s));
-        HIPCHK(hipMemcpyAsync(ctx->found.p, nog.data(), 2 * N * 4, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemsetAsync(ctx->it.p, 0, N * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->nlive.p, 0, N * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->want_next.p, 0, N * 4, s));
-        HIPCHK(hipMemsetAsync(ctx->done.p, 0, N * 4, s));
-        HIPCHK(hipMemcpyAsync(ctx->opt.p, neg.data(), N * 4, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemsetAsync(ctx->iter_counts.p, 0, N * (size_t)max_iters * 8, s));
-        unsigned ctl[64];
-        memset(ctl, 0, sizeof ctl);
-        ctl[1] = (unsigned)n; // active instances
-        const int budget = ctx->cfg.round_budget > 0 ? ctx->cfg.round_budget : kRoundSteps;
-        // a round ends after its step budget or its time limit, whichever
-        // comes first
-        const int rt = ctx->cfg.round_time_us == 0 ? kRoundTimeUs : ctx->cfg.round_time_us;
-        p.round_ticks = (rt > 0 && ctx->wall_ticks_per_us > 0)
-                            ? (unsigned long long)(rt * ctx->wall_ticks_per_us) : 0ull;
-        p.turn_ticks = ctx->wall_ticks_per_us > 0 ? (unsigned long long)(kTurnUs * ctx->wall_ticks_per_us) : 1ull << 40;
-        ctl[5] = (unsigned)budget;
-        HIPCHK(hipMemcpyAsync(ctx->ctl.p, ctl, sizeof ctl, hipMemcpyHostToDevice, s));
-        unsigned long long qc[kQCtlWords];
-        memset(qc, 0, sizeof qc);
-        for (int r = 0; r < 2; ++r)
-            for (int x = 0; x < kGroups; ++x) qc[kQHead + r * kQRing + x * kLine] = (unsigned long long)x;
-        HIPCHK(hipMemcpyAsync(ctx->q_ctl.p, qc, sizeof qc, hipMemcpyHostToDevice, s));
-        HIPCHK(hipMemsetAsync(ctx->c_st.p, 0, lanes * 4, s));
-        HIPCHK(hipStreamSynchronize(s));
-    }
+    // a round ends after its step budget or its time limit, whichever comes
+    // first
+    const int rt = ctx->cfg.round_time_us == 0 ? kRoundTimeUs : ctx->cfg.round_time_us;
+    p.round_ticks =
+        (rt > 0 && ctx->wall_ticks_per_us > 0) ? (unsigned long long)(rt * ctx->wall_ticks_per_us) : 0ull;
+    p.turn_ticks = ctx->wall_ticks_per_us > 0 ? (unsigned long long)(kTurnUs * ctx->wall_ticks_per_us) : 1ull << 40;
 
     HIPCHK(launch_restart(w, heur, p, ctx->geo_d.as<PdbGeo>(), s));
     HIPCHK(launch_control(p, s));
@@ -1117,8 +1094,7 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
         for (auto &x : ev) HIPCHK(hipEventCreate(&x));
     double round_ms = 0;
     long timed = 0;
-    unsigned *h_ctl = nullptr; // pinned: 64 control words
-    HIPCHK(hipHostMalloc((void **)&h_ctl, 64 * 4, hipHostMallocDefault));
+    unsigned *const h_ctl = (unsigned *)ctx->stage.p; // pinned: 64 control words
     int rc = SPZ_OK;
     long rounds = 0;
 
@@ -1134,7 +1110,7 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
             if (e == hipSuccess) e = launch_restart(w, heur, p, ctx->geo_d.as<PdbGeo>(), s);
             if (e == hipSuccess) e = launch_control(p, s);
         }
-        if (e == hipSuccess) e = hipMemcpyAsync(h_ctl, ctx->ctl.p, 64 * 4, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipMemcpyAsync(h_ctl, ctx->head.p, 64 * 4, hipMemcpyDeviceToHost, s);
         return e;
     };
     // hipGraph: the period is captured once and replayed; the kernels read
@@ -1144,7 +1120,7 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     // kernel timing runs the rounds eagerly: HIP events recorded by a captured
     // graph cannot be timed against each other
     bool use_graph = ctx->cfg.use_graph != 0 && !timing;
-    if (use_graph) {
+    auto make_graph = [&]() {
         hipError_t e = hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed);
         hipError_t e2 = e == hipSuccess ? enqueue_period() : e;
         hipError_t e3 = e == hipSuccess ? hipStreamEndCapture(s, &graph) : e;
@@ -1158,10 +1134,12 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
             use_graph = false;
             (void)hipGetLastError();
         }
-    }
-    ctx->stats[15] = use_graph ? 1.0 : 0.0;
-    for (;;) {
-        hipError_t e = use_graph ? hipGraphLaunch(gexec, s) : enqueue_period();
+    };
+    for (long period = 0;; ++period) {
+        // the first period is launched kernel by kernel: a short search is
+        // over sooner than the graph is made
+        if (period == 1 && use_graph) make_graph();
+        hipError_t e = period > 0 && use_graph ? hipGraphLaunch(gexec, s) : enqueue_period();
         rounds += per_poll;
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (timing && e == hipSuccess) {
@@ -1209,10 +1187,8 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     if (graph) (void)hipGraphDestroy(graph);
     if (timing)
         for (auto &x : ev) (void)hipEventDestroy(x);
-    if (rc != SPZ_OK) {
-        (void)hipHostFree(h_ctl);
-        return rc;
-    }
+    if (rc != SPZ_OK) return rc;
+    ctx->stats[15] = use_graph ? 1.0 : 0.0;
     ctx->stats[14] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_rounds).count();
     ctx->stats[8] = round_ms;
     ctx->stats[9] = (double)timed;
@@ -1223,20 +1199,17 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     ctx->stats[23] = (double)h_ctl[13];
     ctx->stats[24] = (double)h_ctl[14];
     ctx->stats[25] = (double)h_ctl[15];
-    (void)hipHostFree(h_ctl);
 
-    std::vector<int> opt(N), its(N);
-    std::vector<unsigned long long> ic(N * (size_t)max_iters);
-    HIPCHK(hipMemcpyAsync(opt.data(), ctx->opt.p, N * 4, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(its.data(), ctx->it.p, N * 4, hipMemcpyDeviceToHost, s));
-    HIPCHK(hipMemcpyAsync(ic.data(), ctx->iter_counts.p, ic.size() * 8, hipMemcpyDeviceToHost, s));
+    HIPCHK(hipMemcpyAsync(stage, ctx->results.p, results_n, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
+    const int *opt = (const int *)stage, *its = opt + N, *h0 = its + N;
+    const unsigned long long *ic = (const unsigned long long *)(stage + results_counts(N));
     ctx->stats[1] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
     double all_nodes = 0;
     for (int i = 0; i < n; ++i) {
         spz_result &r = out[i];
         r.opt_len = opt[i];
-        r.h0 = meta_h(roots[i].meta);
+        r.h0 = h0[i];
         r.n_iters = its[i] + 1;
         r.status = opt[i] >= 0 ? SPZ_ST_SOLVED : SPZ_ST_ITER_LIMIT;
         uint64_t tot = 0;

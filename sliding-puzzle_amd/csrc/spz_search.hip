@@ -172,11 +172,12 @@ __device__ __forceinline__ void put_item(const KParams &p, int r, unsigned long 
 // more than the ring's capacity past the oldest item not taken would
 // overwrite it, so that sets the error word (ctl[3]) and the host fails the
 // solve with SPZ_E_CAPACITY rather than return counts from a corrupt queue.
+template <int Unroll>
 __device__ __forceinline__ unsigned long long q_reserve(const KParams &p, int r, unsigned long long k) {
     unsigned long long *c = p.q_ctl + kQTail + r * kQRing;
     const unsigned long long pos = atomicAdd(&c[0], k);
     unsigned long long oldest = c[1]; // the limit: taken positions end there
-#pragma unroll 1
+#pragma unroll Unroll
     for (int x = 0; x < kGroups; ++x) {
         const unsigned long long h = ld_agent(&p.q_ctl[kQHead + r * kQRing + x * kLine]);
         oldest = h < oldest ? h : oldest;
@@ -263,6 +264,7 @@ __device__ __forceinline__ const KParams &params_again() {
 // at 3 waves per SIMD.  PROF: with the lane-state counters (SPZ_PROFILE).
 template <int W, int HEUR, bool PROF>
 __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, const PdbGeo *geo_g) {
+    if (p.ctl[1] == 0) return; // every instance is done: a round enqueued in advance
     // every wave of the grid starts within microseconds of the others
     const long long t_start = wall_clock64();
     const int MAXD = p.maxd;
@@ -562,7 +564,7 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
             atomicAdd(&p.pend[grp * p.gstride + inst], (unsigned)k);
             atomicAdd(&p.ctl[8], (unsigned)k);
             const int r = ahead_ring(p, inst);
-            unsigned long long pos = q_reserve(p, r, (unsigned long long)k);
+            unsigned long long pos = q_reserve<1>(p, r, (unsigned long long)k);
 #pragma unroll 1
             for (uint32_t pass = dpass; pass; pass &= pass - 1) {
                 const int d = __builtin_ctz(pass);
@@ -1395,14 +1397,19 @@ __device__ int resolve_instance(const KParams &p, int inst) {
     }
 }
 
+// threads of a restart block: four passes over the instance's frontier, its
+// items' loads waited for in each (one instance, 2048 nodes: 18 us with 256
+// threads, 16 us with 1024)
+constexpr int kRestartThreads = 1024;
+
 template <int W, int HEUR>
-__global__ void __launch_bounds__(256) k_restart(KParams p, const PdbGeo *geo_g) {
+__global__ void __launch_bounds__(kRestartThreads) k_restart(KParams p, const PdbGeo *geo_g) {
     __shared__ unsigned long long s_cnt;
     __shared__ unsigned s_bucket[64];
     __shared__ unsigned long long s_base;
     __shared__ int s_j, s_ring;
     __shared__ float s_est;
-    __shared__ unsigned s_nfit;
+    __shared__ unsigned s_nfit, s_items;
     __shared__ PdbGeo geo_s;
     const int inst = (int)blockIdx.x;
     if (threadIdx.x == 0) {
@@ -1509,14 +1516,22 @@ __global__ void __launch_bounds__(256) k_restart(KParams p, const PdbGeo *geo_g)
             atomicAdd(&s_cnt, (unsigned long long)gn);
         }
         __syncthreads();
-        if (threadIdx.x == 0) {
-            unsigned off = 0;
-            for (int b = 63; b >= 0; --b) { // largest keys first
-                unsigned n = s_bucket[b];
-                s_bucket[b] = off;
-                off += n;
+        static_assert(kRestartThreads >= 64, "a wave scans the buckets");
+        if (threadIdx.x < 64) { // largest keys first
+            const int b = 63 - (int)threadIdx.x;
+            const unsigned n = s_bucket[b];
+            unsigned upto = n;
+            for (int o = 1; o < 64; o <<= 1) {
+                const unsigned v = __shfl_up(upto, o);
+                if ((int)threadIdx.x >= o) upto += v;
             }
-            s_base = off ? q_reserve(p, s_ring, (unsigned long long)off) : 0ull;
+            s_bucket[b] = upto - n;
+            if (threadIdx.x == 63) s_items = upto;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const unsigned off = s_items;
+            s_base = off ? q_reserve<kGroups>(p, s_ring, (unsigned long long)off) : 0ull;
             p.L[isl] = L;
             p.itn[isl] = it;
             p.found[isl] = p.top_goal[inst] <= L ? p.top_goal[inst] : kNoGoal;
@@ -1677,72 +1692,36 @@ __global__ void __launch_bounds__(64) k_control(KParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// k_split_level: one level of the root split, all instances at once.  A level
-// that already holds >= target nodes (or is at max depth) becomes the
-// instance's frontier; otherwise every node is expanded without pruning:
-// its generated children are counted into the top-tree histogram under the
-// node's f, and the children form the next level.
-template <int W, int HEUR>
-__global__ void __launch_bounds__(256) k_split_level(KParams p, const PdbGeo *geo_g, const Item *lvl_in,
-                                                     const unsigned *n_in, Item *lvl_out, unsigned *n_out,
-                                                     unsigned *nfront, unsigned *topgen, int *top_goal,
-                                                     int *frozen, int depth, int max_depth, unsigned target,
-                                                     const unsigned long long *lp_in, unsigned long long *lp_out,
-                                                     unsigned long long *fp_out) {
-    __shared__ PdbGeo geo_s;
-    PdbCtx P{&geo_s, p.pdb};
-    if constexpr (HEUR == 1) {
-        const uint32_t *src = (const uint32_t *)geo_g;
-        uint32_t *dst = (uint32_t *)&geo_s;
-        for (int i = threadIdx.x; i < (int)(sizeof(PdbGeo) / 4); i += blockDim.x) dst[i] = src[i];
-        __syncthreads();
-    }
-    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int inst = (int)(gid / (size_t)p.capl);
-    const unsigned j = (unsigned)(gid % (size_t)p.capl);
-    if (inst >= p.n_inst) return;
-    // frozen[inst] = 1 + the depth at which the instance froze; it is written
-    // during that launch, so this launch only honours earlier freezes
-    const int fz = frozen[inst];
-    if (fz != 0 && fz - 1 < depth) return;
-    const unsigned n = min(n_in[inst], (unsigned)p.capl);
-    const bool freeze = (n >= target) || (depth >= max_depth);
-    if (freeze) {
-        if (j < n) {
-            ((Item *)p.frontier)[(size_t)inst * p.capl + j] = lvl_in[(size_t)inst * p.capl + j];
-            if (fp_out) fp_out[(size_t)inst * p.capl + j] = lp_in[(size_t)inst * p.capl + j];
-        }
-        if (j == 0) {
-            nfront[inst] = n;
-            frozen[inst] = depth + 1;
-        }
-        return;
-    }
-    if (j >= n) return;
-    Item it = lvl_in[(size_t)inst * p.capl + j];
+// Root split: one node of a level.  It is expanded without pruning: its
+// generated children are counted under its f (hist), and they form the next
+// level, from position reserve(children) of `out` on.  lp_in/lp_out: the
+// levels' paths, or null.  F = largest f on the path from the root (x0 carries
+// the parent's F): the node is expanded in iteration L iff F <= L, heuristic
+// consistent or not.
+template <int W, int HEUR, class Reserve, class Hist, class Goal>
+__device__ __forceinline__ void split_expand(const KParams &p, const PdbCtx &P, int inst, const Item &it, Item *out,
+                                             const unsigned long long *lp_in, unsigned long long *lp_out,
+                                             Reserve &&reserve, Hist &&hist, Goal &&goal) {
     Pos<W, HEUR> s;
     pos_from_item<W, HEUR>(s, it.b, it.meta, P);
-    int g = meta_g(it.meta), prev = meta_prev(it.meta);
-    // F = largest f on the path from the root (x0 carries the parent's F):
-    // the node is expanded in iteration L iff F <= L, heuristic consistent
-    // or not
+    const int g = meta_g(it.meta), prev = meta_prev(it.meta);
     int f = g + s.hs.h;
     if ((int)it.x0 > f) f = (int)it.x0;
     if (s.hs.h == 0) {
-        atomicMin(&top_goal[inst], f);
+        goal(f);
         // levels run in depth order, so the first goal recorded is a
         // shallowest one; it goes to both iteration slots (the iteration that
         // ends the instance, in either slot, finds no shallower goal)
         if (p.sol)
             for (int sl = inst * 2; sl < inst * 2 + 2; ++sl)
-                if (atomicCAS(&p.sol_len[sl], -1, g) == -1)
-                    path_from_u64(lp_in[(size_t)inst * p.capl + j], p.sol, (uint32_t)sl * kPathWords);
+                if (atomicCAS(&p.sol_len[sl], -1, g) == -1) path_from_u64(*lp_in, p.sol, (uint32_t)sl * kPathWords);
     }
     uint32_t gen = legal_moves(s) & ~(prev < 4 ? (1u << (3 - prev)) : 0u);
-    atomicAdd(&topgen[(size_t)inst * kFBins + (f < kFBins ? f : kFBins - 1)], (unsigned)__builtin_popcount(gen));
-    unsigned k = atomicAdd(&n_out[inst], (unsigned)__builtin_popcount(gen));
+    const unsigned n = (unsigned)__builtin_popcount(gen);
+    hist(f < kFBins ? f : kFBins - 1, n);
+    unsigned k = reserve(n);
     while (gen) {
-        int d = __builtin_ctz(gen);
+        const int d = __builtin_ctz(gen);
         gen &= gen - 1;
         Pos<W, HEUR> c = s;
         do_move<W, HEUR>(c, d, P);
@@ -1753,12 +1732,171 @@ __global__ void __launch_bounds__(256) k_split_level(KParams p, const PdbGeo *ge
         ci.x0 = (uint32_t)f;
         ci.x1 = 0;
         if (k < (unsigned)p.capl) {
-            lvl_out[(size_t)inst * p.capl + k] = ci;
+            out[k] = ci;
             // split depth <= 32 when paths are recorded: move g fits the u64
-            if (lp_out) lp_out[(size_t)inst * p.capl + k] = lp_in[(size_t)inst * p.capl + j] | ((unsigned long long)d << (2 * g));
+            if (lp_out) lp_out[k] = *lp_in | ((unsigned long long)d << (2 * g));
         }
         ++k;
     }
+}
+
+template <int HEUR> __device__ __forceinline__ void load_geo(PdbGeo &geo_s, const PdbGeo *geo_g) {
+    if constexpr (HEUR == 1) {
+        const uint32_t *src = (const uint32_t *)geo_g;
+        uint32_t *dst = (uint32_t *)&geo_s;
+        for (int i = threadIdx.x; i < (int)(sizeof(PdbGeo) / 4); i += blockDim.x) dst[i] = src[i];
+        __syncthreads();
+    }
+}
+
+// k_split_level: one level of the root split, all instances at once.  A level
+// that already holds >= target nodes (or is at max depth) becomes the
+// instance's frontier; otherwise every node is expanded.
+template <int W, int HEUR>
+__global__ void __launch_bounds__(256) k_split_level(KParams p, const PdbGeo *geo_g, const Item *lvl_in,
+                                                     const unsigned *n_in, Item *lvl_out, unsigned *n_out,
+                                                     int *frozen, int depth, int max_depth, unsigned target,
+                                                     const unsigned long long *lp_in, unsigned long long *lp_out) {
+    __shared__ PdbGeo geo_s;
+    PdbCtx P{&geo_s, p.pdb};
+    load_geo<HEUR>(geo_s, geo_g);
+    const size_t gid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int inst = (int)(gid / (size_t)p.capl);
+    const unsigned j = (unsigned)(gid % (size_t)p.capl);
+    if (inst >= p.n_inst) return;
+    // frozen[inst] = 1 + the depth at which the instance froze; it is written
+    // during that launch, so this launch only honours earlier freezes
+    const int fz = frozen[inst];
+    if (fz != 0 && fz - 1 < depth) return;
+    const unsigned n = min(n_in[inst], (unsigned)p.capl);
+    const bool freeze = (n >= target) || (depth >= max_depth);
+    const size_t at = (size_t)inst * p.capl;
+    if (freeze) {
+        if (j < n) {
+            ((Item *)p.frontier)[at + j] = lvl_in[at + j];
+            if (lp_in) ((unsigned long long *)p.fpath)[at + j] = lp_in[at + j];
+        }
+        if (j == 0) {
+            ((unsigned *)p.nfront)[inst] = n;
+            frozen[inst] = depth + 1;
+        }
+        return;
+    }
+    if (j >= n) return;
+    split_expand<W, HEUR>(
+        p, P, inst, lvl_in[at + j], lvl_out + at, lp_in ? lp_in + at + j : nullptr, lp_out ? lp_out + at : nullptr,
+        [&](unsigned k) { return atomicAdd(&n_out[inst], k); },
+        [&](int f, unsigned k) { atomicAdd((unsigned *)&p.topgen[(size_t)inst * kFBins + f], k); },
+        [&](int f) { atomicMin((int *)&p.top_goal[inst], f); });
+}
+
+// k_begin: one workgroup per instance starts it: the root's heuristic, the
+// per-instance state, and (split) the whole root split, level by level in the
+// instance's region of the two level buffers, sizes and f-histogram in LDS.
+// A launch a level over all instances' regions costs 4 us a level however
+// small, and where there are many instances mostly looks at empty slots (100
+// instances, 2048 nodes each: 25 launches, 2.1 ms; so 0.05 ms).  One workgroup
+// falls behind the grid on a very large frontier (kOneBlockSplit).
+constexpr int kBeginThreads = 1024;
+template <int W, int HEUR>
+__global__ void __launch_bounds__(kBeginThreads) k_begin(KParams p, const PdbGeo *geo_g, Item *lvl0, Item *lvl1,
+                                                         unsigned *nlvl0, int *frozen, int max_depth, unsigned target,
+                                                         unsigned long long *lp0, unsigned long long *lp1, int split) {
+    __shared__ PdbGeo geo_s;
+    __shared__ unsigned s_n[2], s_hist[kFBins];
+    __shared__ int s_goal, s_h;
+    PdbCtx P{&geo_s, p.pdb};
+    load_geo<HEUR>(geo_s, geo_g);
+    const int inst = (int)blockIdx.x, t = threadIdx.x;
+    const size_t at = (size_t)inst * p.capl;
+    if (t == 0) {
+        Item it = p.roots[inst];
+        Board<W> bd;
+        bd.unpack(it.b);
+        int h = 0;
+        if constexpr (HEUR == 0) {
+            for (int c = 0; c < W * W; ++c) {
+                const int x = bd.tile(c);
+                if (x) h += abs(c / W - trow<W>(x)) + abs(c % W - tcol<W>(x));
+            }
+        } else {
+            HState<1> hs;
+            pdb_init(P, hs, bd);
+            h = hs.h;
+        }
+        it.meta = (it.meta & 0xff00ffffu) | ((uint32_t)h << 16);
+        ((Item *)p.roots)[inst] = it;
+        lvl0[at] = it;
+        if (lp0) lp0[at] = 0ull; // the root's empty path
+        s_n[0] = 1;
+        s_n[1] = 0;
+        s_goal = kNoGoal;
+        s_h = h;
+        p.it[inst] = 0;
+        p.nlive[inst] = 0;
+        p.want_next[inst] = 0;
+        p.done[inst] = 0;
+        p.opt[inst] = -1;
+        ((int *)p.Lbase)[inst] = h;
+        if (!split) {
+            nlvl0[inst] = 1;
+            frozen[inst] = 0;
+            ((int *)p.top_goal)[inst] = kNoGoal;
+        }
+    }
+    if (t < 2) {
+        const int isl = inst * 2 + t;
+        p.L[isl] = 0;
+        p.itn[isl] = 0;
+        p.found[isl] = kNoGoal;
+        p.drained[isl] = 0;
+        p.dead[isl] = 0;
+        if (p.sol_len) p.sol_len[isl] = -1; // none yet
+    }
+    for (int i = t; i < p.max_iters; i += kBeginThreads) p.iter_counts[(size_t)inst * p.max_iters + i] = 0;
+    for (int f = t; f < kFBins; f += kBeginThreads) {
+        s_hist[f] = 0;
+        if (!split) ((unsigned *)p.topgen)[(size_t)inst * kFBins + f] = 0;
+    }
+    if (!split) return;
+    for (int depth = 0;; ++depth) {
+        __syncthreads();
+        const int a = depth & 1;
+        const unsigned n = min(s_n[a], (unsigned)p.capl);
+        const Item *in = (a ? lvl1 : lvl0) + at;
+        Item *out = (a ? lvl0 : lvl1) + at;
+        unsigned long long *li = a ? lp1 : lp0, *lo = a ? lp0 : lp1;
+        __syncthreads(); // s_n is read
+        if (t == 0) s_n[a] = 0;
+        if (n >= target || depth >= max_depth) {
+            for (unsigned j = t; j < n; j += kBeginThreads) {
+                ((Item *)p.frontier)[at + j] = in[j];
+                if (li) ((unsigned long long *)p.fpath)[at + j] = li[at + j];
+            }
+            if (t == 0) {
+                ((unsigned *)p.nfront)[inst] = n;
+                ((int *)p.top_goal)[inst] = s_goal;
+            }
+            for (int f = t; f < kFBins; f += kBeginThreads) ((unsigned *)p.topgen)[(size_t)inst * kFBins + f] = s_hist[f];
+            return;
+        }
+        for (unsigned j = t; j < n; j += kBeginThreads)
+            split_expand<W, HEUR>(
+                p, P, inst, in[j], out, li ? li + at + j : nullptr, lo ? lo + at : nullptr,
+                [&](unsigned k) { return atomicAdd(&s_n[a ^ 1], k); },
+                [&](int f, unsigned k) { atomicAdd(&s_hist[f], k); }, [&](int f) { atomicMin(&s_goal, f); });
+    }
+}
+
+// The words of a solve's waves: no lane has a context, no wave waits.
+__global__ void __launch_bounds__(256) k_clear_waves(KParams p, unsigned n_list) {
+    const unsigned i = blockIdx.x * 256u + threadIdx.x;
+    if (i < (unsigned)p.n_lanes) p.c_st[i] = ST_IDLE;
+    if (i < (unsigned)p.n_lanes >> 6) {
+        p.ticket[i] = 0;
+        p.mail_head[(size_t)i * kLine] = 0;
+    }
+    if (i < n_list) p.list[i] = 0;
 }
 
 // heuristic of packed items (spz_eval_h and the root h0)
@@ -1846,12 +1984,6 @@ hipError_t launch_eval_h_bytes(int width, int heur, const uint8_t *bytes, int n,
     return hipGetLastError();
 }
 
-// roots -> slot 0 of each instance's level-0 region
-__global__ void k_scatter_roots(const Item *roots, Item *lvl, int capl, int n) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) lvl[(size_t)i * capl] = roots[i];
-}
-
 // ---------------------------------------------------------------------------
 // host-side launchers
 size_t round_lds_bytes(int width, int maxd, int wg, int heur);
@@ -1892,11 +2024,11 @@ const void *round_kernel_ptr(int width, int heur) {
 
 hipError_t launch_restart(int width, int heur, const KParams &p, const PdbGeo *geo, hipStream_t s) {
     if (width == 4)
-        hipLaunchKernelGGL((k_restart<4, 0>), dim3(p.n_inst), dim3(256), 0, s, p, geo);
+        hipLaunchKernelGGL((k_restart<4, 0>), dim3(p.n_inst), dim3(kRestartThreads), 0, s, p, geo);
     else if (heur == 0)
-        hipLaunchKernelGGL((k_restart<5, 0>), dim3(p.n_inst), dim3(256), 0, s, p, geo);
+        hipLaunchKernelGGL((k_restart<5, 0>), dim3(p.n_inst), dim3(kRestartThreads), 0, s, p, geo);
     else
-        hipLaunchKernelGGL((k_restart<5, 1>), dim3(p.n_inst), dim3(256), 0, s, p, geo);
+        hipLaunchKernelGGL((k_restart<5, 1>), dim3(p.n_inst), dim3(kRestartThreads), 0, s, p, geo);
     return hipGetLastError();
 }
 
@@ -1911,26 +2043,24 @@ hipError_t launch_control(const KParams &p, hipStream_t s) {
 }
 
 hipError_t launch_split_level(int width, int heur, const KParams &p, const PdbGeo *geo, const Item *lvl_in,
-                              const unsigned *n_in, Item *lvl_out, unsigned *n_out, unsigned *nfront,
-                              unsigned *topgen, int *top_goal, int *frozen, int depth, int max_depth,
-                              unsigned target, const unsigned long long *lp_in, unsigned long long *lp_out,
-                              unsigned long long *fp_out, hipStream_t s) {
-    size_t total = (size_t)p.n_inst * p.capl;
-    dim3 grid((unsigned)((total + 255) / 256));
-    if (width == 4)
-        hipLaunchKernelGGL((k_split_level<4, 0>), grid, dim3(256), 0, s, p, geo, lvl_in, n_in, lvl_out, n_out, nfront,
-                           topgen, top_goal, frozen, depth, max_depth, target, lp_in, lp_out, fp_out);
-    else if (heur == 0)
-        hipLaunchKernelGGL((k_split_level<5, 0>), grid, dim3(256), 0, s, p, geo, lvl_in, n_in, lvl_out, n_out, nfront,
-                           topgen, top_goal, frozen, depth, max_depth, target, lp_in, lp_out, fp_out);
-    else
-        hipLaunchKernelGGL((k_split_level<5, 1>), grid, dim3(256), 0, s, p, geo, lvl_in, n_in, lvl_out, n_out, nfront,
-                           topgen, top_goal, frozen, depth, max_depth, target, lp_in, lp_out, fp_out);
+                              const unsigned *n_in, Item *lvl_out, unsigned *n_out, int *frozen, int depth,
+                              int max_depth, unsigned target, const unsigned long long *lp_in,
+                              unsigned long long *lp_out, hipStream_t s) {
+    const size_t total = (size_t)p.n_inst * p.capl;
+    auto *const k = width == 4 ? &k_split_level<4, 0> : heur == 0 ? &k_split_level<5, 0> : &k_split_level<5, 1>;
+    hipLaunchKernelGGL(k, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, p, geo, lvl_in, n_in, lvl_out, n_out,
+                       frozen, depth, max_depth, target, lp_in, lp_out);
     return hipGetLastError();
 }
 
-hipError_t launch_scatter_roots(const Item *roots, Item *lvl, int capl, int n, hipStream_t s) {
-    hipLaunchKernelGGL(k_scatter_roots, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, roots, lvl, capl, n);
+hipError_t launch_begin(int width, int heur, const KParams &p, const PdbGeo *geo, Item *lvl0, Item *lvl1,
+                        unsigned *nlvl0, int *frozen, int max_depth, unsigned target, unsigned long long *lp0,
+                        unsigned long long *lp1, bool split, unsigned n_list, hipStream_t s) {
+    const unsigned most = (unsigned)p.n_lanes > n_list ? (unsigned)p.n_lanes : n_list;
+    hipLaunchKernelGGL(k_clear_waves, dim3((most + 255) / 256), dim3(256), 0, s, p, n_list);
+    auto *const k = width == 4 ? &k_begin<4, 0> : heur == 0 ? &k_begin<5, 0> : &k_begin<5, 1>;
+    hipLaunchKernelGGL(k, dim3(p.n_inst), dim3(kBeginThreads), 0, s, p, geo, lvl0, lvl1, nlvl0, frozen, max_depth,
+                       target, lp0, lp1, split ? 1 : 0);
     return hipGetLastError();
 }
 
