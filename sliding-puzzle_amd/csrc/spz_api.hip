@@ -32,10 +32,9 @@ hipError_t launch_split_level(int width, int heur, const KParams &p, const PdbGe
 hipError_t launch_begin(int width, int heur, const KParams &p, const PdbGeo *geo, Item *lvl0, Item *lvl1,
                         unsigned *nlvl0, int *frozen, int max_depth, unsigned target, unsigned long long *lp0,
                         unsigned long long *lp1, bool split, unsigned n_list, hipStream_t s);
-hipError_t launch_eval_h(int width, int heur, const KParams &p, const PdbGeo *geo, Item *items, int n,
-                         hipStream_t s);
-hipError_t launch_eval_h_bytes(int width, int heur, const uint8_t *bytes, int n, const PdbGeo *geo,
-                               const uint8_t *pdb, int *h, hipStream_t s);
+hipError_t launch_boards(int width, int heur, const uint8_t *bytes, int n, const PdbGeo *geo, const uint8_t *pdb,
+                         const int *thr, const float *tgt, Item *items, int *thr_d, float *tgt_d, int *h,
+                         unsigned *bad, hipStream_t s);
 hipError_t pdb_bfs_build(int pat, uint8_t *compact, uint32_t *work, unsigned *d_any, hipStream_t s, int *levels_out);
 hipError_t pdb_spread(const uint8_t *compact, uint8_t *direct, hipStream_t s);
 hipError_t launch_gather_probe(const uint8_t *t, uint64_t span, int blocks, int per_thread, uint64_t seed, uint32_t *out,
@@ -156,6 +155,8 @@ struct spz_ctx {
     DBuf head;    // control words, queue-control words, then the roots: one upload
     DBuf results; // per instance: optimum, last iteration, h0, then the counts: one download
     HBuf stage;   // pinned staging of both, and of the control words polled
+    HBuf fetch;   // pinned staging of what an evaluation returns
+    DBuf rows_items, rows_thr, rows_tgt, rows_y; // boards of the predictor's entry points
     DBuf list, mail, mail_head, ticket, mail_path; // waves without work
     size_t qcap = 0;
     // per instance
@@ -211,15 +212,14 @@ static int host_failure(spz_ctx *c, const char *what) noexcept {
     } while (0)
 
 static bool is_solvable(int w, const uint8_t *b) {
-    int n2 = w * w;
-    bool seen[25] = {false};
-    int inv = 0, blank = -1;
+    const int n2 = w * w;
+    uint32_t seen = 0;
+    int inv = 0, blank = 0;
     for (int i = 0; i < n2; ++i) {
-        if (b[i] >= n2 || seen[b[i]]) return false;
-        seen[b[i]] = true;
+        if (b[i] >= n2 || ((seen >> b[i]) & 1u)) return false;
+        inv += __builtin_popcount(seen >> b[i]); // the greater ones before it
+        seen |= 1u << b[i];
         if (b[i] == 0) blank = i;
-        for (int j = i + 1; j < n2; ++j)
-            if (b[i] > b[j]) ++inv;
     }
     // every move flips both the permutation parity and the blank's row+col parity
     return (inv & 1) == ((blank / w + blank % w) & 1);
@@ -289,6 +289,16 @@ constexpr unsigned kOneBlockSplit = 16384;
 // largest upload or download through pinned staging; larger ones stream from
 // and to pageable memory
 constexpr size_t kMaxStage = 16u << 20;
+// the staging's first words: the control words polled, or the bad-board flag
+constexpr size_t kStageHead = 256;
+// Boards a launch of k_boards checks: the host copies the next ones to the
+// staging meanwhile.  A launch costs the host more than the overlap gives on
+// small pieces (40,003 boards: 4096 a launch 138 us, 8192 89, 16384 73, all in
+// one 65).
+constexpr int kBoardsPiece = 65536;
+// boards spz_eval_h_noalloc checks on the host: waiting for the device's
+// verdict before the values are copied costs 8 us, a board's check 45 ns
+constexpr int kHostCheck = 256;
 // A round ends early once the waves that ran out of work have waited, summed
 // over them and divided by all waves, this long: about what it costs to end a
 // round, save and restore the lanes, start iterations and feed the waves again.
@@ -411,7 +421,7 @@ int spz_create(spz_ctx **out, const spz_config *cfg) try {
         pdb_geo_build(&ctx->geo_h);
         if ((e = ctx->geo_d.ensure(sizeof(PdbGeo))) != hipSuccess ||
             (e = hipMemcpy(ctx->geo_d.p, &ctx->geo_h, sizeof(PdbGeo), hipMemcpyHostToDevice)) != hipSuccess ||
-            (e = ctx->head.ensure(kHeadRoots)) != hipSuccess) {
+            (e = ctx->head.ensure(kHeadRoots)) != hipSuccess || (e = ctx->stage.ensure(kStageHead)) != hipSuccess) {
             rc = fail(ctx, SPZ_E_HIP, "context allocation: %s", hipGetErrorString(e));
             break;
         }
@@ -557,11 +567,13 @@ void spz_destroy(spz_ctx *ctx) {
                    &ctx->fpath,   &ctx->lpath[0],       &ctx->lpath[1],       &ctx->sol,        &ctx->sol_len,
                    &ctx->itn,     &ctx->drained,        &ctx->nlive,          &ctx->list,       &ctx->mail,
                    &ctx->mail_head, &ctx->ticket,       &ctx->mail_path,      &ctx->want_next,  &ctx->dead,
-                   &ctx->prof,    &ctx->wtime};
+                   &ctx->prof,    &ctx->wtime,          &ctx->rows_items,     &ctx->rows_thr,   &ctx->rows_tgt,
+                   &ctx->rows_y};
     for (DBuf *b : all) b->release();
     ctx->dd_items.release();
     ctx->dd_paths.release();
     ctx->stage.release();
+    ctx->fetch.release();
     if (ctx->mlp_alloced) mlp_free(ctx->mlp);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -836,29 +848,79 @@ static size_t next_pow2(size_t x) {
     return p;
 }
 
-int spz_eval_h(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t *h) try {
-    if (!ctx || !boards || !h || n < 0) return SPZ_E_ARG;
-    if (n == 0) return SPZ_OK;
-    const int w = ctx->cfg.width, heur = ctx->cfg.heuristic;
-    if (heur == SPZ_H_PDB666 && !ctx->have_pdb) return fail(ctx, SPZ_E_NOPDB, "call spz_build_pdb first");
+// a k_boards launch found a bad board: which one
+static int bad_board(spz_ctx *ctx, const uint8_t *boards, int n) {
+    const int w = ctx->cfg.width;
     for (int i = 0; i < n; ++i)
         if (!is_solvable(w, boards + (size_t)i * w * w))
             return fail(ctx, SPZ_E_ARG, "board %d is not a solvable permutation", i);
-    HIPCHK(hipSetDevice(ctx->cfg.device));
-    std::vector<Item> items((size_t)n);
-    for (int i = 0; i < n; ++i) pack_root(w, boards + (size_t)i * w * w, i, &items[i]);
-    DBuf d;
-    HIPCHK(d.ensure(sizeof(Item) * (size_t)n));
-    KParams p = base_params(ctx, 0, 1, 1);
-    hipError_t e = hipMemcpyAsync(d.p, items.data(), sizeof(Item) * n, hipMemcpyHostToDevice, ctx->stream);
-    if (e == hipSuccess) e = launch_eval_h(w, heur, p, ctx->geo_d.as<PdbGeo>(), d.as<Item>(), n, ctx->stream);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(items.data(), d.p, sizeof(Item) * n, hipMemcpyDeviceToHost, ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    d.release();
-    if (e != hipSuccess) return fail(ctx, SPZ_E_HIP, "eval_h: %s", hipGetErrorString(e));
-    for (int i = 0; i < n; ++i) h[i] = meta_h(items[i].meta);
+    return fail(ctx, SPZ_E_HIP, "boards changed while they were read");
+}
+
+static unsigned *bad_flag(spz_ctx *ctx) { return (unsigned *)ctx->stage.p; }
+
+// Boards (and thresholds, targets) through the pinned staging to k_boards,
+// which leaves their heuristics in h_d or packed boards in items_d.  The
+// caller waits for the stream, and fails with bad_board if *bad_flag is set.
+static int load_boards(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int n, int *h_d,
+                       Item *items_d, int *thr_d, float *tgt_d) {
+    const int w = ctx->cfg.width, n2 = w * w;
+    if (ctx->cfg.heuristic == SPZ_H_PDB666 && !ctx->have_pdb) return fail(ctx, SPZ_E_NOPDB, "call spz_build_pdb first");
+    // a piece's boards, thresholds and targets, 16-byte aligned each
+    const size_t piece_n = ((size_t)std::min(n, kBoardsPiece) + 15) & ~(size_t)15;
+    const size_t per = piece_n * (size_t)(n2 + (thr ? 4 : 0) + (tgt ? 4 : 0));
+    const size_t pieces = ((size_t)n + kBoardsPiece - 1) / kBoardsPiece;
+    const size_t held = std::min(pieces, std::max<size_t>(1, kMaxStage / per));
+    HIPCHK(ctx->stage.ensure(kStageHead + held * per));
+    *bad_flag(ctx) = 0;
+    for (size_t k = 0; k < pieces; ++k) {
+        const size_t i0 = k * kBoardsPiece, m = std::min<size_t>((size_t)n - i0, kBoardsPiece);
+        if (k && k % held == 0) HIPCHK(hipStreamSynchronize(ctx->stream)); // the staging is read
+        uint8_t *b = (uint8_t *)ctx->stage.p + kStageHead + (k % held) * per, *t = b + piece_n * n2;
+        uint8_t *g = t + (thr ? piece_n * 4 : 0);
+        memcpy(b, boards + i0 * n2, m * n2);
+        if (thr) memcpy(t, thr + i0, m * 4);
+        if (tgt) memcpy(g, tgt + i0, m * 4);
+        HIPCHK(launch_boards(w, ctx->cfg.heuristic, b, (int)m, ctx->geo_d.as<PdbGeo>(), ctx->pdb_direct.as<uint8_t>(),
+                             thr ? (const int *)t : nullptr, tgt ? (const float *)g : nullptr,
+                             items_d ? items_d + i0 : nullptr, thr ? thr_d + i0 : nullptr,
+                             tgt ? tgt_d + i0 : nullptr, h_d ? h_d + i0 : nullptr, bad_flag(ctx), ctx->stream));
+    }
     return SPZ_OK;
+}
+
+// What the stream leaves at src, to dst, once the boards turn out good:
+// through pinned staging up to kMaxStage bytes (src may be that staging).
+static int fetch_checked(spz_ctx *ctx, const uint8_t *boards, int n, void *dst, const void *src, size_t bytes) {
+    const bool pinned = bytes <= kMaxStage;
+    if (pinned && src != ctx->fetch.p) {
+        HIPCHK(ctx->fetch.ensure(bytes));
+        HIPCHK(hipMemcpyAsync(ctx->fetch.p, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+    }
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (*bad_flag(ctx)) return bad_board(ctx, boards, n);
+    if (pinned)
+        memcpy(dst, ctx->fetch.p, bytes);
+    else
+        HIPCHK(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
+    return SPZ_OK;
+}
+
+int spz_eval_h(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t *h) try {
+    if (!ctx || !boards || !h || n < 0) return SPZ_E_ARG;
+    if (n == 0) return SPZ_OK;
+    HIPCHK(hipSetDevice(ctx->cfg.device));
+    // the values go straight to pinned memory where there are not too many
+    const size_t bytes = (size_t)n * 4;
+    DBuf d;
+    if (bytes <= kMaxStage)
+        HIPCHK(ctx->fetch.ensure(bytes));
+    else
+        HIPCHK(d.ensure(bytes));
+    int *const h_d = (int *)(bytes <= kMaxStage ? ctx->fetch.p : d.p);
+    const int rc = load_boards(ctx, boards, nullptr, nullptr, n, h_d, nullptr, nullptr, nullptr);
+    if (rc) return rc;
+    return fetch_checked(ctx, boards, n, h, h_d, bytes);
 } SPZ_CATCH(ctx)
 
 // spz_eval_h without any allocation: boards and values pass through the
@@ -872,15 +934,20 @@ int spz_eval_h_noalloc(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t *
     if (!ctx->scratch_d) return fail(ctx, SPZ_E_HIP, "no scratch on this device");
     const int w = ctx->cfg.width, heur = ctx->cfg.heuristic, n2 = w * w;
     if (heur == SPZ_H_PDB666 && !ctx->have_pdb) return fail(ctx, SPZ_E_NOPDB, "call spz_build_pdb first");
-    for (int i = 0; i < n; ++i)
+    for (int i = 0; n <= kHostCheck && i < n; ++i)
         if (!is_solvable(w, boards + (size_t)i * n2))
             return fail(ctx, SPZ_E_ARG, "board %d is not a solvable permutation", i);
     HIPCHK(hipSetDevice(ctx->cfg.device));
     hipStream_t s = ctx->stream;
     int *hd = (int *)(ctx->scratch_d + kNoAllocHOff);
+    *bad_flag(ctx) = 0;
     HIPCHK(hipMemcpyAsync(ctx->scratch_d, boards, (size_t)n * n2, hipMemcpyHostToDevice, s));
-    HIPCHK(launch_eval_h_bytes(w, heur, ctx->scratch_d, n, ctx->geo_d.as<PdbGeo>(), ctx->pdb_direct.as<uint8_t>(),
-                               hd, s));
+    HIPCHK(launch_boards(w, heur, ctx->scratch_d, n, ctx->geo_d.as<PdbGeo>(), ctx->pdb_direct.as<uint8_t>(), nullptr,
+                         nullptr, nullptr, nullptr, nullptr, hd, bad_flag(ctx), s));
+    if (n > kHostCheck) {
+        HIPCHK(hipStreamSynchronize(s));
+        if (*bad_flag(ctx)) return bad_board(ctx, boards, n);
+    }
     HIPCHK(hipMemcpyAsync(h, hd, (size_t)n * 4, hipMemcpyDeviceToHost, s));
     HIPCHK(hipStreamSynchronize(s));
     return SPZ_OK;
@@ -929,9 +996,9 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     // and later the results, where they are not too large to pin
     const size_t head_n = kHeadRoots + N * sizeof(Item);
     const bool pinned = std::max(head_n, results_n) <= kMaxStage;
-    HIPCHK(ctx->stage.ensure(256 + (pinned ? std::max(head_n, results_n) : 0)));
+    HIPCHK(ctx->stage.ensure(kStageHead + (pinned ? std::max(head_n, results_n) : 0)));
     std::vector<uint8_t> pageable(pinned ? 0 : std::max(head_n, results_n));
-    uint8_t *const stage = pinned ? (uint8_t *)ctx->stage.p + 256 : pageable.data();
+    uint8_t *const stage = pinned ? (uint8_t *)ctx->stage.p + kStageHead : pageable.data();
     HIPCHK(ctx->L.ensure(2 * N * 4));
     HIPCHK(ctx->itn.ensure(2 * N * 4));
     const size_t gstride = (2 * N + 31) / 32 * 32; // each group's part on lines of its own
@@ -1386,24 +1453,22 @@ int spz_mlp_get_params(spz_ctx *ctx, float *params) try {
     return SPZ_OK;
 } SPZ_CATCH(ctx)
 
-// boards -> Items with the context's heuristic in meta -> feature rows
-static int mlp_load_rows(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, int32_t n, DBuf &items,
-                         DBuf &thr_d) {
-    const int w = ctx->cfg.width;
-    if (ctx->cfg.heuristic == SPZ_H_PDB666 && !ctx->have_pdb) return fail(ctx, SPZ_E_NOPDB, "call spz_build_pdb first");
-    for (int i = 0; i < n; ++i)
-        if (!is_solvable(w, boards + (size_t)i * w * w))
-            return fail(ctx, SPZ_E_ARG, "board %d is not a solvable permutation", i);
-    std::vector<Item> it((size_t)n);
-    for (int i = 0; i < n; ++i) pack_root(w, boards + (size_t)i * w * w, i, &it[i]);
-    HIPCHK(items.ensure((size_t)n * sizeof(Item)));
-    HIPCHK(thr_d.ensure((size_t)n * 4));
-    HIPCHK(hipMemcpyAsync(items.p, it.data(), (size_t)n * sizeof(Item), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(hipMemcpyAsync(thr_d.p, thr, (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream));
-    KParams p = base_params(ctx, 0, 1, 1);
-    HIPCHK(launch_eval_h(w, ctx->cfg.heuristic, p, ctx->geo_d.as<PdbGeo>(), items.as<Item>(), n, ctx->stream));
+// boards, thresholds and targets of a predictor call to the device
+static int mlp_load_rows(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int32_t n) {
+    HIPCHK(ctx->rows_items.ensure((size_t)n * sizeof(Item)));
+    HIPCHK(ctx->rows_thr.ensure((size_t)n * 4));
+    if (tgt) HIPCHK(ctx->rows_tgt.ensure((size_t)n * 4));
+    return load_boards(ctx, boards, thr, tgt, n, nullptr, ctx->rows_items.as<Item>(), ctx->rows_thr.as<int>(),
+                       ctx->rows_tgt.as<float>());
+}
+
+// and the feature rows of them
+static int mlp_load_features(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int32_t n) {
+    const int rc = mlp_load_rows(ctx, boards, thr, tgt, n);
+    if (rc) return rc;
     HIPCHK(mlp_reserve(ctx->mlp, (size_t)n));
-    HIPCHK(mlp_features_items(ctx->mlp, w, items.as<Item>(), thr_d.as<int>(), n, ctx->stream));
+    HIPCHK(mlp_features_items(ctx->mlp, ctx->cfg.width, ctx->rows_items.as<Item>(), ctx->rows_thr.as<int>(), n,
+                              ctx->stream));
     return SPZ_OK;
 }
 
@@ -1411,13 +1476,10 @@ int spz_mlp_forward(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, int
     if (!ctx || !boards || !thr || !out || n <= 0) return SPZ_E_ARG;
     if (!ctx->mlp_alloced || !ctx->mlp.ready) return fail(ctx, SPZ_E_ARG, "no MLP parameters");
     HIPCHK(hipSetDevice(ctx->cfg.device));
-    DBuf items, thr_d;
-    int rc = mlp_load_rows(ctx, boards, thr, n, items, thr_d);
+    const int rc = mlp_load_features(ctx, boards, thr, nullptr, n);
     if (rc) return rc;
     HIPCHK(mlp_forward(ctx->mlp, n, ctx->stream));
-    HIPCHK(hipMemcpyAsync(out, ctx->mlp.y, (size_t)n * 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    return SPZ_OK;
+    return fetch_checked(ctx, boards, n, out, ctx->mlp.y, (size_t)n * 4);
 } SPZ_CATCH(ctx)
 
 static_assert(kPredK == kPredThr, "one prediction per threshold slot of the restart");
@@ -1426,15 +1488,12 @@ int spz_mlp_predict(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr0, in
     if (!ctx || !boards || !thr0 || !out || n <= 0) return SPZ_E_ARG;
     if (!ctx->mlp_alloced || !ctx->mlp.ready) return fail(ctx, SPZ_E_ARG, "no MLP parameters");
     HIPCHK(hipSetDevice(ctx->cfg.device));
-    DBuf items, thr_d, y;
-    int rc = mlp_load_rows(ctx, boards, thr0, n, items, thr_d);
+    const int rc = mlp_load_rows(ctx, boards, thr0, nullptr, n);
     if (rc) return rc;
-    HIPCHK(y.ensure((size_t)n * kPredThr * 4));
-    HIPCHK(mlp_predict_items(ctx->mlp, ctx->cfg.width, items.as<Item>(), thr_d.as<int>(), n, y.as<float>(),
-                             ctx->stream));
-    HIPCHK(hipMemcpyAsync(out, y.p, (size_t)n * kPredThr * 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    return SPZ_OK;
+    HIPCHK(ctx->rows_y.ensure((size_t)n * kPredThr * 4));
+    HIPCHK(mlp_predict_items(ctx->mlp, ctx->cfg.width, ctx->rows_items.as<Item>(), ctx->rows_thr.as<int>(), n,
+                             ctx->rows_y.as<float>(), ctx->stream));
+    return fetch_checked(ctx, boards, n, out, ctx->rows_y.p, (size_t)n * kPredThr * 4);
 } SPZ_CATCH(ctx)
 
 int spz_mlp_grad(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *target, int32_t n,
@@ -1442,16 +1501,17 @@ int spz_mlp_grad(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const 
     if (!ctx || !boards || !thr || !target || !loss || !grad || n <= 0) return SPZ_E_ARG;
     if (!ctx->mlp_alloced || !ctx->mlp.ready) return fail(ctx, SPZ_E_ARG, "no MLP parameters");
     HIPCHK(hipSetDevice(ctx->cfg.device));
-    DBuf items, thr_d, tgt;
-    int rc = mlp_load_rows(ctx, boards, thr, n, items, thr_d);
+    const int rc = mlp_load_features(ctx, boards, thr, target, n);
     if (rc) return rc;
-    HIPCHK(tgt.ensure((size_t)n * 4));
-    HIPCHK(hipMemcpyAsync(tgt.p, target, (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream));
     HIPCHK(mlp_forward(ctx->mlp, n, ctx->stream));
-    HIPCHK(mlp_backward(ctx->mlp, tgt.as<float>(), n, ctx->stream));
-    HIPCHK(hipMemcpyAsync(loss, ctx->mlp.loss, 4, hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(grad, ctx->mlp.grad, kMlpParams * 4, hipMemcpyDeviceToHost, ctx->stream));
+    HIPCHK(mlp_backward(ctx->mlp, ctx->rows_tgt.as<float>(), n, ctx->stream));
+    // the loss lies behind the gradient
+    HIPCHK(ctx->fetch.ensure((kMlpParams + 1) * 4));
+    HIPCHK(hipMemcpyAsync(ctx->fetch.p, ctx->mlp.grad, (kMlpParams + 1) * 4, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    if (*bad_flag(ctx)) return bad_board(ctx, boards, n);
+    memcpy(grad, ctx->fetch.p, kMlpParams * 4);
+    memcpy(loss, (const float *)ctx->fetch.p + kMlpParams, 4);
     return SPZ_OK;
 } SPZ_CATCH(ctx)
 
@@ -1465,12 +1525,6 @@ int spz_mlp_train(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const
     // all rows, thresholds and targets to the device once; each epoch uploads
     // one permutation and its batches are gathered on the device, so the
     // host waits once per epoch (for the epoch's summed batch losses)
-    std::vector<Item> it((size_t)n);
-    for (int i = 0; i < n; ++i) {
-        if (!is_solvable(w, boards + (size_t)i * w * w))
-            return fail(ctx, SPZ_E_ARG, "board %d is not a solvable permutation", i);
-        pack_root(w, boards + (size_t)i * w * w, i, &it[i]);
-    }
     DBuf items, thr_d, tgt_d, perm_d, btgt, eloss;
     HIPCHK(items.ensure((size_t)n * sizeof(Item)));
     HIPCHK(thr_d.ensure((size_t)n * 4));
@@ -1478,12 +1532,12 @@ int spz_mlp_train(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const
     HIPCHK(perm_d.ensure((size_t)n * 4));
     HIPCHK(btgt.ensure((size_t)batch * 4));
     HIPCHK(eloss.ensure((size_t)epochs * 4));
-    HIPCHK(hipMemcpyAsync(items.p, it.data(), (size_t)n * sizeof(Item), hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(thr_d.p, thr, (size_t)n * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(hipMemcpyAsync(tgt_d.p, target, (size_t)n * 4, hipMemcpyHostToDevice, s));
+    const int rc = load_boards(ctx, boards, thr, target, n, nullptr, items.as<Item>(), thr_d.as<int>(),
+                               tgt_d.as<float>());
+    HIPCHK(hipStreamSynchronize(s));
+    if (rc) return rc;
+    if (*bad_flag(ctx)) return bad_board(ctx, boards, n);
     HIPCHK(hipMemsetAsync(eloss.p, 0, (size_t)epochs * 4, s));
-    KParams p = base_params(ctx, 0, 1, 1);
-    HIPCHK(launch_eval_h(w, ctx->cfg.heuristic, p, ctx->geo_d.as<PdbGeo>(), items.as<Item>(), n, s));
     HIPCHK(mlp_reserve(ctx->mlp, (size_t)batch));
     std::vector<int> perm((size_t)n);
     for (int i = 0; i < n; ++i) perm[i] = i;

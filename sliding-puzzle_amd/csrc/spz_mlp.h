@@ -34,7 +34,7 @@ struct Item;
 struct MlpState {
     float *master = nullptr;    // fp32 parameters [kMlpParams]
     uint16_t *wbf = nullptr;    // bf16 copy of the parameters
-    float *grad = nullptr;      // fp32 gradient [kMlpParams]
+    float *grad = nullptr;      // fp32 gradient [kMlpParams], then the loss
     float *adam_m = nullptr, *adam_v = nullptr;
     int adam_t = 0;
     bool ready = false;         // parameters set
@@ -47,7 +47,7 @@ struct MlpState {
     float *dz = nullptr;        // [cap][256] scratch gradient
     uint16_t *dzb = nullptr;    // bf16 copy
     float *part = nullptr;      // [cap/64][256] partial column sums
-    float *loss = nullptr;      // [1]
+    float *loss = nullptr;      // grad + kMlpParams
     uint16_t *w2frag = nullptr; // W2 in MFMA B-fragment order (prediction)
 };
 

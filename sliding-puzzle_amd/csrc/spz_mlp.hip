@@ -219,10 +219,10 @@ hipError_t mlp_alloc(MlpState &m) {
     hipError_t e;
     if ((e = hipMalloc(&m.master, kMlpParams * 4)) != hipSuccess) return e;
     if ((e = hipMalloc(&m.wbf, kMlpParams * 2)) != hipSuccess) return e;
-    if ((e = hipMalloc(&m.grad, kMlpParams * 4)) != hipSuccess) return e;
+    if ((e = hipMalloc(&m.grad, (kMlpParams + 1) * 4)) != hipSuccess) return e;
     if ((e = hipMalloc(&m.adam_m, kMlpParams * 4)) != hipSuccess) return e;
     if ((e = hipMalloc(&m.adam_v, kMlpParams * 4)) != hipSuccess) return e;
-    if ((e = hipMalloc(&m.loss, 4)) != hipSuccess) return e;
+    m.loss = m.grad + kMlpParams;
     return hipSuccess;
 }
 
@@ -257,7 +257,6 @@ void mlp_free(MlpState &m) {
     fr(m.grad);
     fr(m.adam_m);
     fr(m.adam_v);
-    fr(m.loss);
     fr(m.w2frag);
     m = MlpState();
 }

@@ -1899,88 +1899,96 @@ __global__ void __launch_bounds__(256) k_clear_waves(KParams p, unsigned n_list)
     if (i < n_list) p.list[i] = 0;
 }
 
-// heuristic of packed items (spz_eval_h and the root h0)
+// Boards given as bytes (row-major, W*W per board, `bytes` 16-byte aligned and
+// readable up to a multiple of 16): each is checked -- a permutation, and one
+// that moves reach from the goal: its inversions and the blank's row + column
+// have the same parity -- and its heuristic goes to h[i], or the packed board
+// with it to items[i]; thr and tgt (null: none) are copied along.  A bad board
+// sets *bad and stands as the goal board.  The input may be host memory: a
+// block reads its bytes once, 16 at a time, into LDS.  Bound by that transfer
+// (40,003 boards, 1.0 MB: 20 us; the host's check and packing of them took
+// 3 ms).
 template <int W, int HEUR>
-__global__ void k_eval_h(KParams p, const PdbGeo *geo_g, Item *items, int n) {
+__global__ void __launch_bounds__(256) k_boards(const uint8_t *bytes, int n, const PdbGeo *geo_g, const uint8_t *pdb,
+                                                const int *thr, const float *tgt, Item *items, int *thr_d,
+                                                float *tgt_d, int *h, unsigned *bad) {
+    constexpr int N2 = W * W;
     __shared__ PdbGeo geo_s;
-    PdbCtx P{&geo_s, p.pdb};
-    if constexpr (HEUR == 1) {
-        const uint32_t *src = (const uint32_t *)geo_g;
-        uint32_t *dst = (uint32_t *)&geo_s;
-        for (int i = threadIdx.x; i < (int)(sizeof(PdbGeo) / 4); i += blockDim.x) dst[i] = src[i];
-        __syncthreads();
-    }
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    Item it = items[i];
-    Board<W> bd;
-    bd.unpack(it.b);
-    int h = 0;
-    if constexpr (HEUR == 0) {
-        for (int c = 0; c < W * W; ++c) {
-            int t = bd.tile(c);
-            if (t) h += abs(c / W - trow<W>(t)) + abs(c % W - tcol<W>(t));
-        }
-    } else {
-        HState<1> hs;
-        pdb_init(P, hs, bd);
-        h = hs.h;
-    }
-    it.meta = (it.meta & 0xff00ffffu) | ((uint32_t)h << 16);
-    items[i] = it;
-}
-
-// heuristic of n boards given as bytes (row-major, W*W per board) into
-// h[n]; the allocation-free evaluation entry point's kernel
-template <int W, int HEUR>
-__global__ void k_eval_h_bytes(const uint8_t *bytes, int n, const PdbGeo *geo_g, const uint8_t *pdb, int *h) {
-    __shared__ PdbGeo geo_s;
+    __shared__ uint4 raw[256 * N2 / 16];
     PdbCtx P{&geo_s, pdb};
-    if constexpr (HEUR == 1) {
-        const uint32_t *src = (const uint32_t *)geo_g;
-        uint32_t *dst = (uint32_t *)&geo_s;
-        for (int i = threadIdx.x; i < (int)(sizeof(PdbGeo) / 4); i += blockDim.x) dst[i] = src[i];
-        __syncthreads();
+    load_geo<HEUR>(geo_s, geo_g);
+    const int t = threadIdx.x, i = (int)blockIdx.x * 256 + t;
+    const int here = min(256, n - (int)blockIdx.x * 256);
+    const uint4 *src = (const uint4 *)(bytes + (size_t)blockIdx.x * (256 * N2));
+    for (int k = t; k < (here * N2 + 15) / 16; k += 256) raw[k] = src[k];
+    __syncthreads();
+    if (t >= here) return;
+    const uint8_t *b = (const uint8_t *)raw + t * N2;
+    uint32_t seen = 0;
+    int inv = 0, blank = 0;
+    bool ok = true;
+    uint64_t lo = 0, hi = 0; // cells 0-11 and 12-23 of width 5; width 4 in lo
+#pragma unroll
+    for (int c = 0; c < N2; ++c) {
+        const uint32_t v = b[c];
+        ok &= v < (uint32_t)N2 && !((seen >> (v & 31u)) & 1u);
+        inv += __popc(seen >> (v & 31u)); // the greater ones before it
+        seen |= 1u << (v & 31u);
+        blank = v ? blank : c;
+        if constexpr (W == 4)
+            lo |= (uint64_t)(v & 15u) << (4 * c);
+        else if (c < 24)
+            (c < 12 ? lo : hi) |= (uint64_t)(v & 31u) << (5 * (c % 12));
     }
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint8_t *b = bytes + (size_t)i * (W * W);
+    ok &= ((inv ^ (blank / W + blank % W)) & 1) == 0;
     Board<W> bd;
     if constexpr (W == 4) {
-        bd.b = 0;
-#pragma unroll
-        for (int c = 0; c < 16; ++c) bd.b |= (uint64_t)b[c] << (4 * c);
+        bd.b = lo;
     } else {
-        bd.lo = bd.hi = 0;
+        bd.lo = lo;
+        bd.hi = hi;
         bd.top = b[24];
-#pragma unroll
-        for (int c = 0; c < 12; ++c) bd.lo |= (uint64_t)b[c] << (5 * c);
-#pragma unroll
-        for (int c = 12; c < 24; ++c) bd.hi |= (uint64_t)b[c] << (5 * (c - 12));
+    }
+    if (!ok) {
+        *bad = 1u;
+        if constexpr (W == 4) {
+            bd.b = 0xfedcba9876543210ull;
+        } else {
+            bd.lo = bd.hi = 0;
+            bd.top = 24;
+            for (int c = 0; c < 24; ++c) (c < 12 ? bd.lo : bd.hi) |= (uint64_t)c << (5 * (c % 12));
+        }
+        blank = 0;
     }
     int v = 0;
     if constexpr (HEUR == 0) {
-        for (int c = 0; c < W * W; ++c) {
-            const int t = bd.tile(c);
-            if (t) v += abs(c / W - trow<W>(t)) + abs(c % W - tcol<W>(t));
+        for (int c = 0; c < N2; ++c) {
+            const int x = bd.tile(c);
+            if (x) v += abs(c / W - trow<W>(x)) + abs(c % W - tcol<W>(x));
         }
     } else {
         HState<1> hs;
         pdb_init(P, hs, bd);
         v = hs.h;
     }
-    h[i] = v;
+    if (h) h[i] = v;
+    if (items) {
+        Item it;
+        bd.pack(it.b);
+        it.meta = meta_pack(blank, 0, v, DIR_NONE);
+        it.inst = it.x0 = it.x1 = 0;
+        items[i] = it;
+    }
+    if (thr) thr_d[i] = thr[i];
+    if (tgt) tgt_d[i] = tgt[i];
 }
 
-hipError_t launch_eval_h_bytes(int width, int heur, const uint8_t *bytes, int n, const PdbGeo *geo,
-                               const uint8_t *pdb, int *h, hipStream_t s) {
-    dim3 grid((unsigned)((n + 255) / 256));
-    if (width == 4)
-        hipLaunchKernelGGL((k_eval_h_bytes<4, 0>), grid, dim3(256), 0, s, bytes, n, geo, pdb, h);
-    else if (heur == 0)
-        hipLaunchKernelGGL((k_eval_h_bytes<5, 0>), grid, dim3(256), 0, s, bytes, n, geo, pdb, h);
-    else
-        hipLaunchKernelGGL((k_eval_h_bytes<5, 1>), grid, dim3(256), 0, s, bytes, n, geo, pdb, h);
+hipError_t launch_boards(int width, int heur, const uint8_t *bytes, int n, const PdbGeo *geo, const uint8_t *pdb,
+                         const int *thr, const float *tgt, Item *items, int *thr_d, float *tgt_d, int *h,
+                         unsigned *bad, hipStream_t s) {
+    auto *const k = width == 4 ? &k_boards<4, 0> : heur == 0 ? &k_boards<5, 0> : &k_boards<5, 1>;
+    hipLaunchKernelGGL(k, dim3((unsigned)(((size_t)n + 255) / 256)), dim3(256), 0, s, bytes, n, geo, pdb, thr, tgt,
+                       items, thr_d, tgt_d, h, bad);
     return hipGetLastError();
 }
 
@@ -2061,18 +2069,6 @@ hipError_t launch_begin(int width, int heur, const KParams &p, const PdbGeo *geo
     auto *const k = width == 4 ? &k_begin<4, 0> : heur == 0 ? &k_begin<5, 0> : &k_begin<5, 1>;
     hipLaunchKernelGGL(k, dim3(p.n_inst), dim3(kBeginThreads), 0, s, p, geo, lvl0, lvl1, nlvl0, frozen, max_depth,
                        target, lp0, lp1, split ? 1 : 0);
-    return hipGetLastError();
-}
-
-hipError_t launch_eval_h(int width, int heur, const KParams &p, const PdbGeo *geo, Item *items, int n,
-                         hipStream_t s) {
-    dim3 grid((unsigned)((n + 255) / 256));
-    if (width == 4)
-        hipLaunchKernelGGL((k_eval_h<4, 0>), grid, dim3(256), 0, s, p, geo, items, n);
-    else if (heur == 0)
-        hipLaunchKernelGGL((k_eval_h<5, 0>), grid, dim3(256), 0, s, p, geo, items, n);
-    else
-        hipLaunchKernelGGL((k_eval_h<5, 1>), grid, dim3(256), 0, s, p, geo, items, n);
     return hipGetLastError();
 }
 

@@ -328,7 +328,7 @@ class Solver:
 
     def mlp_forward(self, boards, thr) -> np.ndarray:
         b, t, tp = self._rows(boards, thr)
-        out = np.zeros(len(b), dtype=np.float32)
+        out = np.empty(len(b), dtype=np.float32)
         self._check(lib().spz_mlp_forward(self._ctx, _u8p(b), tp, len(b),
                                           out.ctypes.data_as(ctypes.POINTER(ctypes.c_float))),
                     "spz_mlp_forward")
@@ -350,7 +350,7 @@ class Solver:
         """Predictions of the learned load balancer's fused kernel: row i
         holds boards[i] at thresholds thr0[i], thr0[i] + 2, ... (16)."""
         b, t, tp = self._rows(boards, thr0)
-        out = np.zeros((len(b), 16), dtype=np.float32)
+        out = np.empty((len(b), 16), dtype=np.float32)
         self._check(lib().spz_mlp_predict(self._ctx, _u8p(b), tp, len(b),
                                           out.ctypes.data_as(ctypes.POINTER(ctypes.c_float))),
                     "spz_mlp_predict")
@@ -360,7 +360,7 @@ class Solver:
         b, t, tp = self._rows(boards, thr)
         tg = np.ascontiguousarray(target, dtype=np.float32)
         loss = ctypes.c_float()
-        g = np.zeros(self.mlp_param_count(), dtype=np.float32)
+        g = np.empty(self.mlp_param_count(), dtype=np.float32)
         self._check(lib().spz_mlp_grad(self._ctx, _u8p(b), tp,
                                        tg.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), len(b),
                                        ctypes.byref(loss),
@@ -419,7 +419,7 @@ class Solver:
 
     def eval_h(self, boards) -> np.ndarray:
         b = np.ascontiguousarray(np.asarray(boards, dtype=np.uint8).reshape(-1, self.width ** 2))
-        h = np.zeros(len(b), dtype=np.int32)
+        h = np.empty(len(b), dtype=np.int32)
         self._check(lib().spz_eval_h(self._ctx, _u8p(b), len(b),
                                      h.ctypes.data_as(ctypes.POINTER(ctypes.c_int32))),
                     "spz_eval_h")
@@ -429,7 +429,7 @@ class Solver:
         """eval_h through the allocation-free entry point (at most 65536
         boards; calls on one GPU share its scratch and must not overlap)."""
         b = np.ascontiguousarray(np.asarray(boards, dtype=np.uint8).reshape(-1, self.width ** 2))
-        h = np.zeros(len(b), dtype=np.int32)
+        h = np.empty(len(b), dtype=np.int32)
         self._check(lib().spz_eval_h_noalloc(self._ctx, _u8p(b), len(b),
                                              h.ctypes.data_as(ctypes.POINTER(ctypes.c_int32))),
                     "spz_eval_h_noalloc")
