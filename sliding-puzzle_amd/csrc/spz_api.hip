@@ -154,8 +154,7 @@ struct spz_ctx {
     DBuf q;
     DBuf head;    // control words, queue-control words, then the roots: one upload
     DBuf results; // per instance: optimum, last iteration, h0, then the counts: one download
-    HBuf stage;   // pinned staging of both, and of the control words polled
-    HBuf fetch;   // pinned staging of what an evaluation returns
+    HBuf stage;   // pinned staging of both, of the control words polled, of boards and values
     DBuf rows_items, rows_thr, rows_tgt, rows_y; // boards of the predictor's entry points
     DBuf list, mail, mail_head, ticket, mail_path; // waves without work
     size_t qcap = 0;
@@ -291,6 +290,8 @@ constexpr unsigned kOneBlockSplit = 16384;
 constexpr size_t kMaxStage = 16u << 20;
 // the staging's first words: the control words polled, or the bad-board flag
 constexpr size_t kStageHead = 256;
+// pinned with the context, so that a first small call pins nothing
+constexpr size_t kMinStage = 64u << 10;
 // Boards a launch of k_boards checks: the host copies the next ones to the
 // staging meanwhile.  A launch costs the host more than the overlap gives on
 // small pieces (40,003 boards: 4096 a launch 138 us, 8192 89, 16384 73, all in
@@ -421,7 +422,7 @@ int spz_create(spz_ctx **out, const spz_config *cfg) try {
         pdb_geo_build(&ctx->geo_h);
         if ((e = ctx->geo_d.ensure(sizeof(PdbGeo))) != hipSuccess ||
             (e = hipMemcpy(ctx->geo_d.p, &ctx->geo_h, sizeof(PdbGeo), hipMemcpyHostToDevice)) != hipSuccess ||
-            (e = ctx->head.ensure(kHeadRoots)) != hipSuccess || (e = ctx->stage.ensure(kStageHead)) != hipSuccess) {
+            (e = ctx->head.ensure(kHeadRoots)) != hipSuccess || (e = ctx->stage.ensure(kMinStage)) != hipSuccess) {
             rc = fail(ctx, SPZ_E_HIP, "context allocation: %s", hipGetErrorString(e));
             break;
         }
@@ -573,7 +574,6 @@ void spz_destroy(spz_ctx *ctx) {
     ctx->dd_items.release();
     ctx->dd_paths.release();
     ctx->stage.release();
-    ctx->fetch.release();
     if (ctx->mlp_alloced) mlp_free(ctx->mlp);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -860,10 +860,11 @@ static int bad_board(spz_ctx *ctx, const uint8_t *boards, int n) {
 static unsigned *bad_flag(spz_ctx *ctx) { return (unsigned *)ctx->stage.p; }
 
 // Boards (and thresholds, targets) through the pinned staging to k_boards,
-// which leaves their heuristics in h_d or packed boards in items_d.  The
-// caller waits for the stream, and fails with bad_board if *bad_flag is set.
-static int load_boards(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int n, int *h_d,
-                       Item *items_d, int *thr_d, float *tgt_d) {
+// which leaves packed boards in items_d, or their heuristics in h_d (null: in
+// the staging's first out_bytes, which the caller's results get).  The caller
+// waits for the stream, and fails with bad_board if *bad_flag is set.
+static int load_boards(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int n,
+                       size_t out_bytes, int *h_d, Item *items_d, int *thr_d, float *tgt_d) {
     const int w = ctx->cfg.width, n2 = w * w;
     if (ctx->cfg.heuristic == SPZ_H_PDB666 && !ctx->have_pdb) return fail(ctx, SPZ_E_NOPDB, "call spz_build_pdb first");
     // a piece's boards, thresholds and targets, 16-byte aligned each
@@ -871,12 +872,15 @@ static int load_boards(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, 
     const size_t per = piece_n * (size_t)(n2 + (thr ? 4 : 0) + (tgt ? 4 : 0));
     const size_t pieces = ((size_t)n + kBoardsPiece - 1) / kBoardsPiece;
     const size_t held = std::min(pieces, std::max<size_t>(1, kMaxStage / per));
-    HIPCHK(ctx->stage.ensure(kStageHead + held * per));
+    const size_t in = kStageHead + (out_bytes + 255) / 256 * 256;
+    HIPCHK(ctx->stage.ensure(in + held * per));
+    uint8_t *const stage = (uint8_t *)ctx->stage.p;
+    if (!h_d && !items_d) h_d = (int *)(stage + kStageHead);
     *bad_flag(ctx) = 0;
     for (size_t k = 0; k < pieces; ++k) {
         const size_t i0 = k * kBoardsPiece, m = std::min<size_t>((size_t)n - i0, kBoardsPiece);
         if (k && k % held == 0) HIPCHK(hipStreamSynchronize(ctx->stream)); // the staging is read
-        uint8_t *b = (uint8_t *)ctx->stage.p + kStageHead + (k % held) * per, *t = b + piece_n * n2;
+        uint8_t *b = stage + in + (k % held) * per, *t = b + piece_n * n2;
         uint8_t *g = t + (thr ? piece_n * 4 : 0);
         memcpy(b, boards + i0 * n2, m * n2);
         if (thr) memcpy(t, thr + i0, m * 4);
@@ -889,18 +893,17 @@ static int load_boards(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, 
     return SPZ_OK;
 }
 
-// What the stream leaves at src, to dst, once the boards turn out good:
-// through pinned staging up to kMaxStage bytes (src may be that staging).
-static int fetch_checked(spz_ctx *ctx, const uint8_t *boards, int n, void *dst, const void *src, size_t bytes) {
-    const bool pinned = bytes <= kMaxStage;
-    if (pinned && src != ctx->fetch.p) {
-        HIPCHK(ctx->fetch.ensure(bytes));
-        HIPCHK(hipMemcpyAsync(ctx->fetch.p, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    }
+// Once the boards of load_boards turn out good, dst gets its results: what the
+// stream leaves at src, through the staging (pinned), or what it leaves in the
+// staging (src null).
+static int fetch_checked(spz_ctx *ctx, const uint8_t *boards, int n, void *dst, const void *src, size_t bytes,
+                         bool pinned) {
+    void *const out = (uint8_t *)ctx->stage.p + kStageHead;
+    if (pinned && src) HIPCHK(hipMemcpyAsync(out, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (*bad_flag(ctx)) return bad_board(ctx, boards, n);
     if (pinned)
-        memcpy(dst, ctx->fetch.p, bytes);
+        memcpy(dst, out, bytes);
     else
         HIPCHK(hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
     return SPZ_OK;
@@ -912,15 +915,13 @@ int spz_eval_h(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t *h) try {
     HIPCHK(hipSetDevice(ctx->cfg.device));
     // the values go straight to pinned memory where there are not too many
     const size_t bytes = (size_t)n * 4;
+    const bool pinned = bytes <= kMaxStage;
     DBuf d;
-    if (bytes <= kMaxStage)
-        HIPCHK(ctx->fetch.ensure(bytes));
-    else
-        HIPCHK(d.ensure(bytes));
-    int *const h_d = (int *)(bytes <= kMaxStage ? ctx->fetch.p : d.p);
-    const int rc = load_boards(ctx, boards, nullptr, nullptr, n, h_d, nullptr, nullptr, nullptr);
+    if (!pinned) HIPCHK(d.ensure(bytes));
+    const int rc = load_boards(ctx, boards, nullptr, nullptr, n, pinned ? bytes : 0, d.as<int>(), nullptr, nullptr,
+                               nullptr);
     if (rc) return rc;
-    return fetch_checked(ctx, boards, n, h, h_d, bytes);
+    return fetch_checked(ctx, boards, n, h, d.p, bytes, pinned);
 } SPZ_CATCH(ctx)
 
 // spz_eval_h without any allocation: boards and values pass through the
@@ -1454,17 +1455,19 @@ int spz_mlp_get_params(spz_ctx *ctx, float *params) try {
 } SPZ_CATCH(ctx)
 
 // boards, thresholds and targets of a predictor call to the device
-static int mlp_load_rows(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int32_t n) {
+static int mlp_load_rows(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int32_t n,
+                         size_t out_bytes) {
     HIPCHK(ctx->rows_items.ensure((size_t)n * sizeof(Item)));
     HIPCHK(ctx->rows_thr.ensure((size_t)n * 4));
     if (tgt) HIPCHK(ctx->rows_tgt.ensure((size_t)n * 4));
-    return load_boards(ctx, boards, thr, tgt, n, nullptr, ctx->rows_items.as<Item>(), ctx->rows_thr.as<int>(),
-                       ctx->rows_tgt.as<float>());
+    return load_boards(ctx, boards, thr, tgt, n, out_bytes <= kMaxStage ? out_bytes : 0, nullptr,
+                       ctx->rows_items.as<Item>(), ctx->rows_thr.as<int>(), ctx->rows_tgt.as<float>());
 }
 
 // and the feature rows of them
-static int mlp_load_features(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int32_t n) {
-    const int rc = mlp_load_rows(ctx, boards, thr, tgt, n);
+static int mlp_load_features(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *tgt, int32_t n,
+                             size_t out_bytes) {
+    const int rc = mlp_load_rows(ctx, boards, thr, tgt, n, out_bytes);
     if (rc) return rc;
     HIPCHK(mlp_reserve(ctx->mlp, (size_t)n));
     HIPCHK(mlp_features_items(ctx->mlp, ctx->cfg.width, ctx->rows_items.as<Item>(), ctx->rows_thr.as<int>(), n,
@@ -1476,10 +1479,11 @@ int spz_mlp_forward(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, int
     if (!ctx || !boards || !thr || !out || n <= 0) return SPZ_E_ARG;
     if (!ctx->mlp_alloced || !ctx->mlp.ready) return fail(ctx, SPZ_E_ARG, "no MLP parameters");
     HIPCHK(hipSetDevice(ctx->cfg.device));
-    const int rc = mlp_load_features(ctx, boards, thr, nullptr, n);
+    const size_t bytes = (size_t)n * 4;
+    const int rc = mlp_load_features(ctx, boards, thr, nullptr, n, bytes);
     if (rc) return rc;
     HIPCHK(mlp_forward(ctx->mlp, n, ctx->stream));
-    return fetch_checked(ctx, boards, n, out, ctx->mlp.y, (size_t)n * 4);
+    return fetch_checked(ctx, boards, n, out, ctx->mlp.y, bytes, bytes <= kMaxStage);
 } SPZ_CATCH(ctx)
 
 static_assert(kPredK == kPredThr, "one prediction per threshold slot of the restart");
@@ -1488,12 +1492,13 @@ int spz_mlp_predict(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr0, in
     if (!ctx || !boards || !thr0 || !out || n <= 0) return SPZ_E_ARG;
     if (!ctx->mlp_alloced || !ctx->mlp.ready) return fail(ctx, SPZ_E_ARG, "no MLP parameters");
     HIPCHK(hipSetDevice(ctx->cfg.device));
-    const int rc = mlp_load_rows(ctx, boards, thr0, nullptr, n);
+    const size_t bytes = (size_t)n * kPredThr * 4;
+    const int rc = mlp_load_rows(ctx, boards, thr0, nullptr, n, bytes);
     if (rc) return rc;
-    HIPCHK(ctx->rows_y.ensure((size_t)n * kPredThr * 4));
+    HIPCHK(ctx->rows_y.ensure(bytes));
     HIPCHK(mlp_predict_items(ctx->mlp, ctx->cfg.width, ctx->rows_items.as<Item>(), ctx->rows_thr.as<int>(), n,
                              ctx->rows_y.as<float>(), ctx->stream));
-    return fetch_checked(ctx, boards, n, out, ctx->rows_y.p, (size_t)n * kPredThr * 4);
+    return fetch_checked(ctx, boards, n, out, ctx->rows_y.p, bytes, bytes <= kMaxStage);
 } SPZ_CATCH(ctx)
 
 int spz_mlp_grad(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const float *target, int32_t n,
@@ -1501,17 +1506,18 @@ int spz_mlp_grad(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const 
     if (!ctx || !boards || !thr || !target || !loss || !grad || n <= 0) return SPZ_E_ARG;
     if (!ctx->mlp_alloced || !ctx->mlp.ready) return fail(ctx, SPZ_E_ARG, "no MLP parameters");
     HIPCHK(hipSetDevice(ctx->cfg.device));
-    const int rc = mlp_load_features(ctx, boards, thr, target, n);
-    if (rc) return rc;
-    HIPCHK(mlp_forward(ctx->mlp, n, ctx->stream));
-    HIPCHK(mlp_backward(ctx->mlp, ctx->rows_tgt.as<float>(), n, ctx->stream));
     // the loss lies behind the gradient
-    HIPCHK(ctx->fetch.ensure((kMlpParams + 1) * 4));
-    HIPCHK(hipMemcpyAsync(ctx->fetch.p, ctx->mlp.grad, (kMlpParams + 1) * 4, hipMemcpyDeviceToHost, ctx->stream));
+    constexpr size_t bytes = (kMlpParams + 1) * 4;
+    const int rc = mlp_load_features(ctx, boards, thr, target, n, bytes);
+    if (rc) return rc;
+    HIPCHK(mlp_hidden(ctx->mlp, n, ctx->stream));
+    HIPCHK(mlp_backward(ctx->mlp, ctx->rows_tgt.as<float>(), n, ctx->stream));
+    const float *const out = (const float *)((uint8_t *)ctx->stage.p + kStageHead);
+    HIPCHK(hipMemcpyAsync((void *)out, ctx->mlp.grad, bytes, hipMemcpyDeviceToHost, ctx->stream));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     if (*bad_flag(ctx)) return bad_board(ctx, boards, n);
-    memcpy(grad, ctx->fetch.p, kMlpParams * 4);
-    memcpy(loss, (const float *)ctx->fetch.p + kMlpParams, 4);
+    memcpy(grad, out, kMlpParams * 4);
+    *loss = out[kMlpParams];
     return SPZ_OK;
 } SPZ_CATCH(ctx)
 
@@ -1532,7 +1538,7 @@ int spz_mlp_train(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const
     HIPCHK(perm_d.ensure((size_t)n * 4));
     HIPCHK(btgt.ensure((size_t)batch * 4));
     HIPCHK(eloss.ensure((size_t)epochs * 4));
-    const int rc = load_boards(ctx, boards, thr, target, n, nullptr, items.as<Item>(), thr_d.as<int>(),
+    const int rc = load_boards(ctx, boards, thr, target, n, 0, nullptr, items.as<Item>(), thr_d.as<int>(),
                                tgt_d.as<float>());
     HIPCHK(hipStreamSynchronize(s));
     if (rc) return rc;
@@ -1559,7 +1565,7 @@ int spz_mlp_train(spz_ctx *ctx, const uint8_t *boards, const int32_t *thr, const
             const int nbat = std::min(batch, n - b0);
             HIPCHK(mlp_features_gather(ctx->mlp, w, items.as<Item>(), thr_d.as<int>(), tgt_d.as<float>(),
                                        perm_d.as<int>() + b0, nbat, btgt.as<float>(), s));
-            HIPCHK(mlp_forward(ctx->mlp, nbat, s));
+            HIPCHK(mlp_hidden(ctx->mlp, nbat, s));
             HIPCHK(mlp_backward(ctx->mlp, btgt.as<float>(), nbat, s, el));
             HIPCHK(mlp_adam_step(ctx->mlp, lr, s));
             ++nbatches[ep];

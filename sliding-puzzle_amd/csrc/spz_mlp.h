@@ -46,7 +46,8 @@ struct MlpState {
     float *y = nullptr;         // [cap]
     float *dz = nullptr;        // [cap][256] scratch gradient
     uint16_t *dzb = nullptr;    // bf16 copy
-    float *part = nullptr;      // [cap/64][256] partial column sums
+    float *e = nullptr;         // [cap] squared errors / n
+    float *part = nullptr;      // [3][cap/64][256] partial column sums
     float *loss = nullptr;      // grad + kMlpParams
     uint16_t *w2frag = nullptr; // W2 in MFMA B-fragment order (prediction)
 };
@@ -60,10 +61,14 @@ hipError_t mlp_init_random(MlpState &m, uint64_t seed, hipStream_t s);
 
 // features of n boards (packed Items with h in meta) at thresholds thr[n]
 hipError_t mlp_features_items(MlpState &m, int width, const Item *items, const int *thr, int n, hipStream_t s);
-// forward over rows [0,n) of the feature buffer; y in m.y
+// hidden layers over rows [0,n) of the feature buffer, h2 and z2 left for
+// mlp_backward
+hipError_t mlp_hidden(MlpState &m, int n, hipStream_t s);
+// and the output, y in m.y
 hipError_t mlp_forward(MlpState &m, int n, hipStream_t s);
-// loss = mean (y - target)^2 (into m.loss, or added to *loss_acc) and the
-// full gradient into m.grad
+// after mlp_hidden on the same rows: loss = mean (y - target)^2 (into m.loss,
+// or added to *loss_acc, so an epoch's losses can add up on the device) and
+// the full gradient into m.grad
 hipError_t mlp_backward(MlpState &m, const float *target, int n, hipStream_t s, float *loss_acc = nullptr);
 // features of rows items[perm[i]] at thr[perm[i]], i < n, and their targets
 // tgt[perm[i]] into tout[i] (a training batch gathered on the device)

@@ -1921,6 +1921,8 @@ __global__ void __launch_bounds__(256) k_boards(const uint8_t *bytes, int n, con
     const int here = min(256, n - (int)blockIdx.x * 256);
     const uint4 *src = (const uint4 *)(bytes + (size_t)blockIdx.x * (256 * N2));
     for (int k = t; k < (here * N2 + 15) / 16; k += 256) raw[k] = src[k];
+    const int th = thr && t < here ? thr[i] : 0;
+    const float tg = tgt && t < here ? tgt[i] : 0.f;
     __syncthreads();
     if (t >= here) return;
     const uint8_t *b = (const uint8_t *)raw + t * N2;
@@ -1979,8 +1981,8 @@ __global__ void __launch_bounds__(256) k_boards(const uint8_t *bytes, int n, con
         it.inst = it.x0 = it.x1 = 0;
         items[i] = it;
     }
-    if (thr) thr_d[i] = thr[i];
-    if (tgt) tgt_d[i] = tgt[i];
+    if (thr) thr_d[i] = th;
+    if (tgt) tgt_d[i] = tg;
 }
 
 hipError_t launch_boards(int width, int heur, const uint8_t *bytes, int n, const PdbGeo *geo, const uint8_t *pdb,
