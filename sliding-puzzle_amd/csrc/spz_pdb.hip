@@ -280,6 +280,20 @@ hipError_t pdb_bfs_build(int pat, uint8_t *compact, uint32_t *work, unsigned *d_
     return hipGetLastError();
 }
 
+// n bytes to host memory, 16 at a time (both 16-byte aligned)
+__global__ void __launch_bounds__(256) k_copy_out(const uint8_t *__restrict__ src, uint8_t *dst, size_t n) {
+    const size_t at = ((size_t)blockIdx.x * 256 + threadIdx.x) * 16;
+    if (at + 16 <= n)
+        *(uint4 *)(dst + at) = *(const uint4 *)(src + at);
+    else
+        for (size_t i = at; i < n; ++i) dst[i] = src[i];
+}
+
+hipError_t launch_copy_out(const uint8_t *src, uint8_t *dst, size_t n, hipStream_t s) {
+    hipLaunchKernelGGL(k_copy_out, dim3((unsigned)((n + 4095) / 4096)), dim3(256), 0, s, src, dst, n);
+    return hipGetLastError();
+}
+
 hipError_t pdb_spread(const uint8_t *compact, uint8_t *direct, hipStream_t s) {
     dim3 grid((unsigned)((kPdbDirect + 255) / 256));
     hipLaunchKernelGGL(k_pdb_spread, grid, dim3(256), 0, s, compact, direct);
