@@ -272,7 +272,7 @@ int spz_get_paths(spz_ctx *ctx, uint8_t *moves, int32_t max_len, int32_t *lens);
  *  12 nodes (all instances, all iterations)
  *  13 setup ms (to the first restart's enqueue)  14 rounds wall ms (with
  *     what of the setup still ran)
- *  15 1 if the rounds ran from a hipGraph (all but the first poll period)
+ *  15 1 if the rounds run from a hipGraph (from the seventh poll on)
  *  16-19 with env SPZ_PROFILE=1: lane-steps idle, expanding, only popping,
  *        and wave-steps (x64 = lane-steps) of the search rounds;
  *  20-22 with SPZ_PROFILE=1 (PDB): moves into a sibling (2 table reads each),

@@ -23,9 +23,7 @@ hipError_t launch_round(int width, int heur, const KParams &p, const PdbGeo *geo
                         hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
 size_t round_lds_bytes(int width, int maxd, int wg, int heur);
 const void *round_kernel_ptr(int width, int heur);
-hipError_t launch_restart(int width, int heur, const KParams &p, const PdbGeo *geo, hipStream_t s);
-hipError_t launch_spec(const KParams &p, hipStream_t s);
-hipError_t launch_control(const KParams &p, hipStream_t s);
+hipError_t launch_turn(int width, int heur, const KParams &p, const PdbGeo *geo, bool spec, hipStream_t s);
 hipError_t launch_split_level(int width, int heur, const KParams &p, const PdbGeo *geo, const Item *lvl_in,
                               const unsigned *n_in, Item *lvl_out, unsigned *n_out, int *frozen, int depth,
                               int max_depth, unsigned target, const unsigned long long *lp_in,
@@ -1189,8 +1187,7 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
         (rt > 0 && ctx->wall_ticks_per_us > 0) ? (unsigned long long)(rt * ctx->wall_ticks_per_us) : 0ull;
     p.turn_ticks = ctx->wall_ticks_per_us > 0 ? (unsigned long long)(kTurnUs * ctx->wall_ticks_per_us) : 1ull << 40;
 
-    HIPCHK(launch_restart(w, heur, p, ctx->geo_d.as<PdbGeo>(), s));
-    HIPCHK(launch_control(p, s));
+    HIPCHK(launch_turn(w, heur, p, ctx->geo_d.as<PdbGeo>(), false, s));
     auto t_rounds = std::chrono::steady_clock::now();
     ctx->stats[13] = std::chrono::duration<double, std::milli>(t_rounds - t_start).count();
 
@@ -1219,9 +1216,7 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
             if (e == hipSuccess)
                 e = launch_round(w, heur, p, ctx->geo_d.as<PdbGeo>(), ctx->wg, s, timing ? ev[2 * k] : nullptr,
                                  timing ? ev[2 * k + 1] : nullptr);
-            if (e == hipSuccess && p.lookahead) e = launch_spec(p, s);
-            if (e == hipSuccess) e = launch_restart(w, heur, p, ctx->geo_d.as<PdbGeo>(), s);
-            if (e == hipSuccess) e = launch_control(p, s);
+            if (e == hipSuccess) e = launch_turn(w, heur, p, ctx->geo_d.as<PdbGeo>(), p.lookahead != 0, s);
         }
         if (e == hipSuccess) e = hipMemcpyAsync(h_ctl, ctx->head.p, 64 * 4, hipMemcpyDeviceToHost, s);
         return e;
@@ -1248,11 +1243,12 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
             (void)hipGetLastError();
         }
     };
+    constexpr long kGraphPeriod = 6;
     for (long period = 0;; ++period) {
-        // the first period is launched kernel by kernel: a short search is
-        // over sooner than the graph is made
-        if (period == 1 && use_graph) make_graph();
-        hipError_t e = period > 0 && use_graph ? hipGraphLaunch(gexec, s) : enqueue_period();
+        // the first periods are launched kernel by kernel, which the rounds
+        // before hide from the device: making the graph costs 165 us
+        if (period == kGraphPeriod && use_graph) make_graph();
+        hipError_t e = period >= kGraphPeriod && use_graph ? hipGraphLaunch(gexec, s) : enqueue_period();
         rounds += per_poll;
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (timing && e == hipSuccess) {

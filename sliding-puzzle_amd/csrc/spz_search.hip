@@ -1403,7 +1403,7 @@ __device__ int resolve_instance(const KParams &p, int inst) {
 constexpr int kRestartThreads = 1024;
 
 template <int W, int HEUR>
-__global__ void __launch_bounds__(kRestartThreads) k_restart(KParams p, const PdbGeo *geo_g) {
+__device__ __forceinline__ void restart_instance(const KParams &p, const PdbGeo *geo_g, int inst) {
     __shared__ unsigned long long s_cnt;
     __shared__ unsigned s_bucket[64];
     __shared__ unsigned long long s_base;
@@ -1411,7 +1411,6 @@ __global__ void __launch_bounds__(kRestartThreads) k_restart(KParams p, const Pd
     __shared__ float s_est;
     __shared__ unsigned s_nfit, s_items;
     __shared__ PdbGeo geo_s;
-    const int inst = (int)blockIdx.x;
     if (threadIdx.x == 0) {
         // nothing to do while the current iteration runs and no lookahead is
         // asked for
@@ -1591,6 +1590,11 @@ __global__ void __launch_bounds__(kRestartThreads) k_restart(KParams p, const Pd
     if (threadIdx.x == 0) p.want_next[inst] = 0;
 }
 
+template <int W, int HEUR>
+__global__ void __launch_bounds__(kRestartThreads) k_restart(KParams p, const PdbGeo *geo_g) {
+    restart_instance<W, HEUR>(p, geo_g, (int)blockIdx.x);
+}
+
 // k_spec (lookahead): after a round, while the waves without work outnumber
 // the queued items by more than 1/32 of the lanes, ask for lookahead for
 // instances that run a single iteration (no goal yet, and a previous
@@ -1609,7 +1613,7 @@ __device__ __forceinline__ unsigned long long q_waiting(const KParams &p, int r)
     return n;
 }
 
-__global__ void __launch_bounds__(256) k_spec(KParams p) {
+__device__ __forceinline__ void ask_lookahead(const KParams &p) {
     __shared__ unsigned long long s_room, s_used;
     const unsigned idle = idle_waves(p);
     if (threadIdx.x == 0) {
@@ -1642,13 +1646,13 @@ __global__ void __launch_bounds__(256) k_spec(KParams p) {
         p.want_next[inst] = 1;
     }
 }
+__global__ void __launch_bounds__(256) k_spec(KParams p) { ask_lookahead(p); }
 
 // k_control: between rounds.  Publishes the items appended to both rings
 // during the last round, sets how many a wave takes at once (an even share of
 // the queue, so that few items reach many waves), and clears the round's
 // words: whoever still waits on a list waits no more.  One wave, a word a lane.
-__global__ void __launch_bounds__(64) k_control(KParams p) {
-    const int lane = threadIdx.x;
+__device__ __forceinline__ void control(const KParams &p, int lane) {
     unsigned long long items = 0;
     if (lane < 2 * kGroups) {
         const int r = lane / kGroups, x = lane % kGroups;
@@ -1674,7 +1678,7 @@ __global__ void __launch_bounds__(64) k_control(KParams p) {
         given += shfl_xor_u64(given, off);
         idle += __shfl_xor(idle, off);
     }
-    __syncthreads(); // the limits are read
+    arrival_fence(); // the limits are read
     if (lane < 2) {
         unsigned long long *c = p.q_ctl + kQTail + lane * kQRing;
         c[1] = c[0];
@@ -1689,6 +1693,23 @@ __global__ void __launch_bounds__(64) k_control(KParams p) {
         p.ctl[4] = share < 1 ? 1u : share > 64 ? 64u : (unsigned)share;
         p.ctl[6] += 1;
     }
+}
+
+__global__ void __launch_bounds__(64) k_control(KParams p) { control(p, (int)threadIdx.x); }
+
+// k_turn: the three between the rounds of a single instance, in its one
+// workgroup.  As launches of their own k_spec and k_control take 4.6 and 4.9 us
+// a round, most of it the launch (one 15-puzzle of 8 to 16 rounds: 2.42 -> 2.23
+// and 4.25 -> 4.03 ms, the graph made later among it).
+template <int W, int HEUR>
+__global__ void __launch_bounds__(kRestartThreads) k_turn(KParams p, const PdbGeo *geo_g, int spec) {
+    if (spec) {
+        ask_lookahead(p);
+        __syncthreads();
+    }
+    restart_instance<W, HEUR>(p, geo_g, 0);
+    __syncthreads();
+    if (threadIdx.x < 64) control(p, (int)threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -2032,22 +2053,15 @@ const void *round_kernel_ptr(int width, int heur) {
     return (const void *)&k_round<5, 1, false>;
 }
 
-hipError_t launch_restart(int width, int heur, const KParams &p, const PdbGeo *geo, hipStream_t s) {
-    if (width == 4)
-        hipLaunchKernelGGL((k_restart<4, 0>), dim3(p.n_inst), dim3(kRestartThreads), 0, s, p, geo);
-    else if (heur == 0)
-        hipLaunchKernelGGL((k_restart<5, 0>), dim3(p.n_inst), dim3(kRestartThreads), 0, s, p, geo);
-    else
-        hipLaunchKernelGGL((k_restart<5, 1>), dim3(p.n_inst), dim3(kRestartThreads), 0, s, p, geo);
-    return hipGetLastError();
-}
-
-hipError_t launch_spec(const KParams &p, hipStream_t s) {
-    hipLaunchKernelGGL(k_spec, dim3(1), dim3(256), 0, s, p);
-    return hipGetLastError();
-}
-
-hipError_t launch_control(const KParams &p, hipStream_t s) {
+hipError_t launch_turn(int width, int heur, const KParams &p, const PdbGeo *geo, bool spec, hipStream_t s) {
+    if (p.n_inst == 1) {
+        auto *const k = width == 4 ? &k_turn<4, 0> : heur == 0 ? &k_turn<5, 0> : &k_turn<5, 1>;
+        hipLaunchKernelGGL(k, dim3(1), dim3(kRestartThreads), 0, s, p, geo, spec ? 1 : 0);
+        return hipGetLastError();
+    }
+    if (spec) hipLaunchKernelGGL(k_spec, dim3(1), dim3(256), 0, s, p);
+    auto *const k = width == 4 ? &k_restart<4, 0> : heur == 0 ? &k_restart<5, 0> : &k_restart<5, 1>;
+    hipLaunchKernelGGL(k, dim3(p.n_inst), dim3(kRestartThreads), 0, s, p, geo);
     hipLaunchKernelGGL(k_control, dim3(1), dim3(64), 0, s, p);
     return hipGetLastError();
 }
