@@ -318,6 +318,8 @@ template <int HEUR, class BD> struct Pos<4, HEUR, BD> {
     __device__ __forceinline__ void step(int d) { bl += dir_cell<4>(d); }
 };
 
+// the move that undoes move d, as a bit; none for DIR_NONE
+__device__ __forceinline__ uint32_t back_move(int d) { return 8u >> d; }
 // moves the blank can make from cell c (bit d: direction d stays on the board)
 template <int W> __device__ __forceinline__ uint32_t legal_moves(int r, int c) {
     return (r > 0 ? 1u : 0u) | (c < W - 1 ? 2u : 0u) | (c > 0 ? 4u : 0u) | (r < W - 1 ? 8u : 0u);
@@ -348,28 +350,34 @@ template <int W, int HEUR, class BD> __device__ __forceinline__ uint32_t legal_m
 // Manhattan: the moves of a blank at cell c that slide a tile nearer its
 // goal (h - 1), bit d for direction d.  Bits of moves off the board are
 // meaningless: callers mask them with the legal moves.
+//
+// 15-puzzle: the four comparisons run in one word.  The rotated board has the
+// tiles' goal rows or columns at bits 2 (up), 12 (left), 20 (right) and 26
+// (down, moved there); right and down, where the coordinate is to be at most
+// the blank's, are turned round (3 - t).  Adding 4 less each threshold carries
+// into the bit above a field where the move is nearer, and one multiplication
+// gathers the four bits.  Wave instructions of a comparison or a selection
+// take 4 cycles of a SIMD here, additions, logic and right shifts 2 (250 mixed
+// boards, with back_move: 378 -> 362 ms).
 template <int W, class BD> __device__ __forceinline__ uint32_t nearer_moves(const BD &bd, int c) {
     const int r = trow<W>(c), k = tcol<W>(c);
-    int tU, tD, tL, tR;
     if constexpr (W == 4) {
         // the board rotated so that cell c - 4 is at bits 0-3: the four
         // neighbours sit at bits 0, 12, 20 and 32 (off-board ones wrap to
         // some cell)
         const uint32_t sh = (uint32_t)(4 * c - 16) & 63u;
         const uint64_t w = (bd.b >> sh) | (bd.b << ((64u - sh) & 63u));
-        const uint32_t lo = (uint32_t)w;
-        tU = (int)(lo & 15u);
-        tL = (int)((lo >> 12) & 15u);
-        tR = (int)((lo >> 20) & 15u);
-        tD = (int)((uint32_t)(w >> 32) & 15u);
+        const uint32_t t = ((uint32_t)w & 0x0030300cu) | (((uint32_t)(w >> 32) & 0xcu) << 24);
+        const uint32_t least = 0x04104010u + (uint32_t)k * 0x000ff000u + (uint32_t)r * 0x03fffffcu;
+        return ((((t ^ 0x0c300000u) + least) & 0x10404010u) * 0x01010088u) >> 28;
     } else {
-        tU = bd.tile(r > 0 ? c - W : c);
-        tD = bd.tile(r < W - 1 ? c + W : c);
-        tL = bd.tile(k > 0 ? c - 1 : c);
-        tR = bd.tile(k < W - 1 ? c + 1 : c);
+        const int tU = bd.tile(r > 0 ? c - W : c);
+        const int tD = bd.tile(r < W - 1 ? c + W : c);
+        const int tL = bd.tile(k > 0 ? c - 1 : c);
+        const int tR = bd.tile(k < W - 1 ? c + 1 : c);
+        return (trow<W>(tU) >= r ? 1u : 0u) | (tcol<W>(tR) <= k ? 2u : 0u) | (tcol<W>(tL) >= k ? 4u : 0u) |
+               (trow<W>(tD) <= r ? 8u : 0u);
     }
-    return (trow<W>(tU) >= r ? 1u : 0u) | (tcol<W>(tR) <= k ? 2u : 0u) | (tcol<W>(tL) >= k ? 4u : 0u) |
-           (trow<W>(tD) <= r ? 8u : 0u);
 }
 
 // Manhattan move of the blank in direction d.  The tile slides one cell
@@ -391,12 +399,14 @@ __device__ __forceinline__ uint32_t move_md(Pos<W, 0, BD> &s, int d) {
         key = horiz ? tcol<W>(t) : trow<W>(t);
         at = horiz ? s.col() : s.row();
     }
-    // up / left: the tile moves to a larger row / column; right / down: smaller
+    // up / left: the tile moves to a larger row / column, nearer if its goal is
+    // at or beyond it (key >= at); right / down: to a smaller one (key <= at)
     const int ahead = (d & 1) ? at - key : key - at;
+    const uint32_t nearer = ahead >= 0 ? 1u : 0u;
     s.hs.h += ahead >= 0 ? -1 : 1;
     s.bd.slide(t, from, to);
     s.step(d);
-    return ahead >= 0 ? 1u : 0u;
+    return nearer;
 }
 
 // Undo of move_md(s, d) that returned `nearer`: the blank moves back.
@@ -404,7 +414,7 @@ template <int W, class BD>
 __device__ __forceinline__ void unmove_md(Pos<W, 0, BD> &s, int d, uint32_t nearer) {
     const int to = s.cell(), from = to - dir_cell<W>(d);
     s.bd.slide(s.bd.tile(from), from, to);
-    s.hs.h += nearer ? 1 : -1;
+    s.hs.h += 2 * (int)nearer - 1;
     s.step(3 - d);
 }
 

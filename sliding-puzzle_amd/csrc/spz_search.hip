@@ -1031,7 +1031,7 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
             int ng = 0;
             bool regfirst = true; // read the regular lookup first (else the reflected)
             if (st == ST_FRESH) {
-                gen = legal_moves(s) & ~(prev < 4 ? (1u << (3 - prev)) : 0u);
+                gen = legal_moves(s) & ~back_move(prev);
                 if constexpr (HEUR == 1) {
                     // lane-slot j reads the lane's j-th generated child, so the
                     // wave runs as many slots as its largest family (3 below the
@@ -1112,7 +1112,7 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
                             if (cand) {
                                 const int d = __builtin_ctz(cand);
                                 const int cc = s.cell() + dir_cell<W>(d);
-                                const uint32_t cgen = legal_cell<W>(cc) & ~(1u << (3 - d));
+                                const uint32_t cgen = legal_cell<W>(cc) & ~back_move(d);
                                 if (!(cgen & nearer_moves<W>(s.bd, cc))) {
                                     cnt += (uint32_t)__builtin_popcount(cgen);
                                     pass &= ~(1u << d);
@@ -1737,7 +1737,7 @@ __device__ __forceinline__ void split_expand(const KParams &p, const PdbCtx &P, 
             for (int sl = inst * 2; sl < inst * 2 + 2; ++sl)
                 if (atomicCAS(&p.sol_len[sl], -1, g) == -1) path_from_u64(*lp_in, p.sol, (uint32_t)sl * kPathWords);
     }
-    uint32_t gen = legal_moves(s) & ~(prev < 4 ? (1u << (3 - prev)) : 0u);
+    uint32_t gen = legal_moves(s) & ~back_move(prev);
     const unsigned n = (unsigned)__builtin_popcount(gen);
     hist(f < kFBins ? f : kFBins - 1, n);
     unsigned k = reserve(n);
