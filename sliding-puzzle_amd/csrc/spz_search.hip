@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
     int st = (int)(stw & 0xff);
     int sp = (int)(stw >> 8);
     // stack levels, then (width 5) the lanes' boards
-    Pos<W, HEUR, typename HotBoard<W>::T> s;
+    Pos<W, HEUR, typename HotBoard<W, HEUR>::T> s;
     // Sibling-value cache (PDB): when a lane enters the first passing child
     // of a node with at most two more, the values its f-test read for them
     // go into slot level % kSibLevels (tag = level in bits 24-31, 6+6 bits
@@ -1096,7 +1096,7 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
                         // with h-1 do.
                         const int slack = L - g - h;
                         if (slack <= 2) {
-                            const uint32_t near = nearer_moves<W>(s.bd, s.cell());
+                            const uint32_t near = nearer_moves<W>(s.bd, s.cell(), s.row(), s.col());
                             if (slack < 2) pass = gen & near;
                             // A child at slack 0 (slack 0 and nearer, or slack 2
                             // and farther) whose own children all fail the
@@ -1112,8 +1112,18 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
                             if (cand) {
                                 const int d = __builtin_ctz(cand);
                                 const int cc = s.cell() + dir_cell<W>(d);
-                                const uint32_t cgen = legal_cell<W>(cc) & ~back_move(d);
-                                if (!(cgen & nearer_moves<W>(s.bd, cc))) {
+                                int cr, ck;
+                                uint32_t cgen = ~back_move(d);
+                                if constexpr (W == 4) {
+                                    cr = cc >> 2;
+                                    ck = cc & 3;
+                                    cgen &= legal_cell<W>(cc);
+                                } else {
+                                    cr = s.row() + dir_dr(d);
+                                    ck = s.col() + dir_dc(d);
+                                    cgen &= legal_moves<W>(cr, ck);
+                                }
+                                if (!(cgen & nearer_moves<W>(s.bd, cc, cr, ck))) {
                                     cnt += (uint32_t)__builtin_popcount(cgen);
                                     pass &= ~(1u << d);
                                 }
@@ -2043,7 +2053,7 @@ hipError_t launch_round(int width, int heur, const KParams &p, const PdbGeo *geo
 // dynamic LDS of k_round: the stack levels, then (width 5) the boards, then
 // (PDB) the sibling-value cache
 size_t round_lds_bytes(int width, int maxd, int wg, int heur) {
-    return (size_t)maxd * wg * (heur == 1 ? 2 : 1) + (width == 5 ? (size_t)kLdsBoardBytes * wg : 0) +
+    return (size_t)maxd * wg * (heur == 1 ? 2 : 1) + (width == 5 ? (size_t)kLdsBoardBytes * wg + kLdsBoardPad : 0) +
            (heur == 1 ? (size_t)kSibLevels * 4 * wg : 0);
 }
 
