@@ -1269,10 +1269,6 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
                     64u * h_ctl[12], h_ctl[1], h_ctl[20]);
             fputc('\n', stderr);
         }
-        if (h_ctl[3] & 2u) {
-            rc = fail(ctx, SPZ_E_STALL, "a word of the work lists was never written");
-            break;
-        }
         if (h_ctl[3]) {
             rc = fail(ctx, SPZ_E_CAPACITY, "work queue overflow: raise queue_items (now %zu items)", ctx->qcap);
             break;

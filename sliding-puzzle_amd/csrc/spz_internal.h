@@ -130,9 +130,8 @@ struct KParams {
     int *done;
     int *opt;
     unsigned long long *iter_counts; // [n_inst][max_iters]
-    unsigned int *ctl;           // 1 active, 3 queue error (1: full, 2: a word
-                                 // never written), 4 items a wave takes at
-                                 // once, 5 step budget, 6 rounds, 7 nodes given
+    unsigned int *ctl;           // 1 active, 3 queue error (1: full), 4 items
+                                 // a wave takes at once, 5 step budget, 6 rounds, 7 nodes given
                                  // to waiting waves, 8 overflow exports, 12
                                  // waves with work at the last round's end, 13
                                  // lookahead iterations started, 14/15 frontier

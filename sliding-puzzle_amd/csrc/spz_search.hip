@@ -43,9 +43,6 @@ constexpr int kShareMin = 4;
 // this many levels above the giver's own
 constexpr int kGiveLevels = 2;
 constexpr int kFeedLevels = 4;
-// looks at a word another wave is about to write before the solve is given up
-// (tens of milliseconds; the writer is microseconds away)
-constexpr int kWriteSpins = 1 << 16;
 // naps of a wave waiting for work in one round at most (a round has its own
 // end; this bounds the wait whatever happens)
 constexpr int kMaxNaps = 1 << 16;
@@ -804,23 +801,20 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
         const uint64_t can = __ballot(lev < 255 && !ahead_ring(p, inst));
         const int n = (__popcll(can) + 1) / 2;
         if (n == 0) return;
+        // who waits first is read before it is taken off the list: as long as
+        // it is the first, its entry stays (a list has an entry for each of
+        // its waves, and only waves that wait hold one), but once it is off,
+        // the wave that comes a list's length after it overwrites that
+        const unsigned pos = (unsigned)w;
+        const unsigned long long e =
+            uniform(ld_agent(&p.list[(size_t)x * (p.list_mask + 1) + (pos & p.list_mask)]));
+        if ((unsigned)(e >> 32) != pos + 1) return; // not written yet, or taken off meanwhile
         bool got = false;
         if (lane == 0) {
             const unsigned long long seen = atomicCAS(list, w, w + 1);
             got = seen == w;
         }
         if (!__ballot(got)) return;
-        const unsigned pos = (unsigned)w;
-        unsigned long long e = 0;
-        for (int spin = 0; spin < kWriteSpins; ++spin) {
-            e = uniform(ld_agent(&p.list[(size_t)x * (p.list_mask + 1) + (pos & p.list_mask)]));
-            if ((unsigned)(e >> 32) == pos + 1) break;
-            __builtin_amdgcn_s_sleep(8);
-        }
-        if ((unsigned)(e >> 32) != pos + 1) {
-            if (lane == 0) atomicOr(&p.ctl[3], 2u);
-            return;
-        }
         const unsigned to = (unsigned)e;
         const uint64_t chosen = smallest(can, lev < 255 ? min(g - sp + lev, 255) : 255, n);
         const bool give = (chosen >> lane) & 1ull;
