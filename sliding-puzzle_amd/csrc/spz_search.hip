@@ -797,17 +797,17 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
         // about as many tries in a look's time as waves waiting
         const unsigned all = list_waves(p, x), donors = all > idle ? all - idle : 1u;
         if (__umulhi(rnd, donors) >= idle) return;
-        const int lev = give_level(kFeedLevels);
-        const uint64_t can = __ballot(lev < 255 && !ahead_ring(p, inst));
-        const int n = (__popcll(can) + 1) / 2;
-        if (n == 0) return;
         // who waits first is read before it is taken off the list: as long as
         // it is the first, its entry stays (a list has an entry for each of
         // its waves, and only waves that wait hold one), but once it is off,
         // the wave that comes a list's length after it overwrites that
         const unsigned pos = (unsigned)w;
-        const unsigned long long e =
-            uniform(ld_agent(&p.list[(size_t)x * (p.list_mask + 1) + (pos & p.list_mask)]));
+        const unsigned long long entry = ld_agent(&p.list[(size_t)x * (p.list_mask + 1) + (pos & p.list_mask)]);
+        const int lev = give_level(kFeedLevels);
+        const uint64_t can = __ballot(lev < 255 && !ahead_ring(p, inst));
+        const int n = (__popcll(can) + 1) / 2;
+        if (n == 0) return;
+        const unsigned long long e = uniform(entry);
         if ((unsigned)(e >> 32) != pos + 1) return; // not written yet, or taken off meanwhile
         bool got = false;
         if (lane == 0) {
