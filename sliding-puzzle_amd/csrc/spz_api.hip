@@ -303,10 +303,11 @@ constexpr int kHostCheck = 256;
 // A round ends early once the waves that ran out of work have waited, summed
 // over them and divided by all waves, this long: about what it costs to end a
 // round, save and restore the lanes, start iterations and feed the waves again.
-// 150 / 300 / 600 us: one random 15-puzzle 4.7 / 4.7 / 4.8 ms, 100 short walks
-// 6.5 / 6.0 / 5.9, one 24-puzzle with the PDB 5.3 / 5.0 / 4.4, 24 of them 182 /
-// 178 / 174.
-constexpr double kTurnUs = 300.0;
+// 300 us, 450, 600, 900: first solutions of three batches 139 ms, 138, 134, 139;
+// three 24-puzzles with tables 21.2, 20.6, 20.0, 19.7; two batches of them 223,
+// 216, 216, 219; three without tables 168, 168, 169, 171; one random 15-puzzle
+// and 100 short walks the same.
+constexpr double kTurnUs = 600.0;
 
 // Lane capacity (from occupancy unless given) and lane-context arrays for
 // the context's workgroup size and LDS stack depth.
