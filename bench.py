@@ -225,10 +225,13 @@ def cpu_baseline(width, heur, boards, res, solver, budget_s=15.0):
     order = sorted(range(n), key=lambda i: nodes_of[i])
     mean_nodes = sum(nodes_of) / n
     cores = cpu_cores()
+    # the port runs on one core, so its sample is one core's
+    have_ref = R.have("24puzzle_expand_with_pdb") if heur == spz.H_PDB666 else width == 4 and R.have("idas_cpu_expand")
+    sample_cores = cores if have_ref else 1
     est_rate = 30e6 if heur == spz.H_PDB666 else 60e6  # nodes/s of the CPU solvers, one core
     pick, acc = [], 0
     for i in order:
-        if pick and acc + nodes_of[i] > est_rate * budget_s * cores:
+        if pick and acc + nodes_of[i] > est_rate * budget_s * sample_cores:
             break
         pick.append(i)
         acc += nodes_of[i]
@@ -283,6 +286,7 @@ def cpu_baseline(width, heur, boards, res, solver, budget_s=15.0):
                               "pdb" if heur == spz.H_PDB666 else "manhattan", "all")
             assert (r, sum(c)) == (res[i].opt_len, res[i].total_nodes), i
             nodes += sum(c)
+            progress(f"CPU port: {nodes / 1e6:.0f} M nodes, {time.perf_counter() - t0:.0f} s")
         secs_sum = makespan = time.perf_counter() - t0
         kind, who, used = "port", "oracle/spz_oracle.c (C port)", 1
     wall = time.perf_counter() - wall0
