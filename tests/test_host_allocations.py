@@ -1,0 +1,72 @@
+"""The library's host code when memory runs out, and what it asks for: libspz
+over a stand-in for the HIP runtime (tests/host/fake_hip.c) in which device
+memory is host memory, kernels do nothing and allocations fail on request, so
+these run without a GPU.  Each test is a process of its own: the stand-in is
+preloaded."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+ROCM = "/opt/rocm/include"
+
+pytestmark = pytest.mark.skipif(shutil.which("gcc") is None or not os.path.isdir(ROCM),
+                                reason="needs gcc and the HIP headers")
+
+HEAD = """
+import ctypes, numpy as np, spz
+F = ctypes.CDLL(None)
+F.fake_fail.argtypes = [ctypes.c_int, ctypes.c_long]
+F.fake_count.restype = F.fake_bytes.restype = ctypes.c_long
+DEVICE, PINNED, LAUNCHES = 0, 1, 2
+def walks(width, n):
+    return np.stack([spz.gen_walk(width, 20, i) for i in range(n)])
+def refused(call, code=-2):
+    before = F.fake_count(LAUNCHES)
+    try:
+        call()
+    except spz.SpzError as e:
+        assert e.code == code, e
+        assert F.fake_count(LAUNCHES) == before, "a kernel was launched"
+        return str(e)
+    raise AssertionError("not refused")
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = tmp_path_factory.mktemp("fake") / "fake_hip.so"
+    r = subprocess.run(["gcc", "-std=c11", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", ROCM,
+                        os.path.join(HERE, "host", "fake_hip.c"), "-o", str(so)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-3000:]
+
+    def run(body):
+        preload = " ".join([str(so), os.environ.get("LD_PRELOAD", "")]).strip()
+        env = dict(os.environ, LD_PRELOAD=preload, PYTHONPATH=os.path.join(REPO, "sliding-puzzle_amd"))
+        r = subprocess.run([sys.executable, "-c", HEAD + body + "\nprint('OK')"], capture_output=True, text=True,
+                           timeout=240, env=env, cwd=REPO)
+        assert r.returncode == 0 and r.stdout.strip().endswith("OK"), (r.returncode, r.stdout[-2000:], r.stderr[-2000:])
+
+    return run
+
+
+@pytest.mark.parametrize("width", [4, 5])
+def test_noalloc_after_a_failed_pin(fake, width):
+    """A call that could not pin its staging leaves the context's staging as it
+    was: spz_eval_h_noalloc, which allocates nothing, works as before."""
+    fake(f"""
+s = spz.Solver(width={width}, frontier_target=4)
+b = walks({width}, 30000)
+F.fake_fail(PINNED, 0)
+refused(lambda: s.eval_h(b))
+for n in (1, 300):
+    assert len(s.eval_h_noalloc(b[:n])) == n
+F.fake_fail(PINNED, -1)
+assert len(s.eval_h(b)) == 30000
+s.close()
+assert F.fake_bytes(DEVICE) == 0 and F.fake_bytes(PINNED) == 0
+""")
