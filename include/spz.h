@@ -145,7 +145,9 @@ typedef struct spz_result {
 void spz_default_config(spz_config *cfg, int32_t width, int32_t heuristic);
 
 /* Create a context on cfg->device.  Replaces the per-process globals and
- * cudaMalloc of src/15puzzle_block_parallel.cu:424-452. */
+ * cudaMalloc of src/15puzzle_block_parallel.cu:424-452.  Where the device
+ * fails, *ctx is set all the same, for spz_last_error and spz_destroy; calls
+ * that would use the device are refused on it (SPZ_E_HIP). */
 int spz_create(spz_ctx **ctx, const spz_config *cfg);
 
 /* Change the launch configuration of a context (workgroup size, lanes,

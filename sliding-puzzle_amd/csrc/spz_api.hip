@@ -142,6 +142,7 @@ struct spz_ctx {
     int wg = 256;
     double wall_ticks_per_us = 0; // device wall clock (wall_clock64) rate
     std::string err;
+    bool created = false; // spz_create succeeded: without it only the message is of use
     double stats[SPZ_STATS_LEN] = {0};
     DBuf prof;             // lane-state counters (env SPZ_PROFILE=1)
     DBuf wtime;            // per-wave clocks of one round (env SPZ_WAVE_TIMES)
@@ -188,6 +189,10 @@ static int fail(spz_ctx *c, int code, const char *fmt, ...) {
     if (c) c->err = buf;
     return code;
 }
+
+// spz_create hands out a context also where it failed, for its message; calls
+// that would use the device are refused on it
+static int not_created(spz_ctx *c) { return fail(c, SPZ_E_HIP, "spz_create failed for this context"); }
 
 // No exception may leave a C entry point: a host-side failure (out of host
 // memory, a thread that cannot start) returns SPZ_E_HOST with its text.
@@ -433,6 +438,7 @@ int spz_create(spz_ctx **out, const spz_config *cfg) try {
             break;
         }
         rc = configure_lanes(ctx);
+        ctx->created = rc == SPZ_OK;
     } while (0);
     if (rc != SPZ_OK) {
         // keep the context so the caller can read the error, but report failure
@@ -445,6 +451,7 @@ int spz_create(spz_ctx **out, const spz_config *cfg) try {
 
 int spz_reconfigure(spz_ctx *ctx, const spz_config *cfg) try {
     if (!ctx || !cfg) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     if (cfg->width != ctx->cfg.width || cfg->heuristic != ctx->cfg.heuristic || cfg->device != ctx->cfg.device)
         return fail(ctx, SPZ_E_ARG, "width, heuristic and device are fixed for a context");
     spz_config ncfg;
@@ -476,6 +483,7 @@ void spz_get_config(spz_ctx *ctx, spz_config *cfg) {
 int spz_autotune(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_iters, int32_t passes,
                  spz_config *best, double *best_ms, int32_t *tried) try {
     if (!ctx || !boards || n <= 0 || !best) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     if (max_iters < 1 || max_iters > kMaxIters) return fail(ctx, SPZ_E_ARG, "max_iters must be in 1..%d", kMaxIters);
     if (passes <= 0) passes = 1;
     std::vector<spz_result> ref((size_t)n), cur((size_t)n);
@@ -690,6 +698,7 @@ static int write_cache(spz_ctx *ctx, const char *path) {
 
 int spz_build_pdb(spz_ctx *ctx, const char *cache_path) try {
     if (!ctx) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     if (ctx->cfg.width != 5) return fail(ctx, SPZ_E_ARG, "PDBs exist for the 24-puzzle only");
     HIPCHK(hipSetDevice(ctx->cfg.device));
     for (int t = 0; t < 2; ++t) HIPCHK(ctx->pdb_compact[t].ensure(kPlacementsHost));
@@ -730,6 +739,7 @@ int spz_build_pdb(spz_ctx *ctx, const char *cache_path) try {
 // placement (every pattern tile home) must be 0.
 int spz_load_pdb_tab(spz_ctx *ctx, const char *path_1256712, const char *path_34891314) try {
     if (!ctx || !path_1256712 || !path_34891314) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     if (ctx->cfg.width != 5) return fail(ctx, SPZ_E_ARG, "PDBs exist for the 24-puzzle only");
     HIPCHK(hipSetDevice(ctx->cfg.device));
     for (int t = 0; t < 2; ++t) HIPCHK(ctx->pdb_compact[t].ensure(kPlacementsHost));
@@ -960,6 +970,7 @@ static int fetch_checked(spz_ctx *ctx, const uint8_t *boards, int n, void *dst, 
 
 int spz_eval_h(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t *h) try {
     if (!ctx || !boards || !h || n < 0) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     if (n == 0) return SPZ_OK;
     HIPCHK(hipSetDevice(ctx->cfg.device));
     // the values go straight to pinned memory where there are not too many
@@ -978,10 +989,10 @@ int spz_eval_h(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t *h) try {
 // overlap on one GPU race), the kernel reads the tables the context holds.
 int spz_eval_h_noalloc(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t *h) try {
     if (!ctx || !boards || !h || n < 0) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     if (n == 0) return SPZ_OK;
     if (n > kNoAllocMaxBoards)
         return fail(ctx, SPZ_E_ARG, "spz_eval_h_noalloc takes at most %d boards (got %d)", kNoAllocMaxBoards, n);
-    if (!ctx->scratch_d) return fail(ctx, SPZ_E_HIP, "no scratch on this device");
     const int w = ctx->cfg.width, heur = ctx->cfg.heuristic, n2 = w * w;
     if (heur == SPZ_H_PDB666 && !ctx->have_pdb) return fail(ctx, SPZ_E_NOPDB, "call spz_build_pdb first");
     for (int i = 0; n <= kHostCheck && i < n; ++i)
@@ -1006,6 +1017,7 @@ int spz_eval_h_noalloc(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t *
 int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_iters, spz_result *out,
                     uint64_t *iter_counts) try {
     if (!ctx || !boards || !out || n < 0) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     if (max_iters < 1 || max_iters > kMaxIters)
         return fail(ctx, SPZ_E_ARG, "max_iters must be in 1..%d", kMaxIters);
     if (n == 0) return SPZ_OK;
@@ -1474,6 +1486,7 @@ static int mlp_ready_alloc(spz_ctx *ctx) {
 
 int spz_mlp_init(spz_ctx *ctx, uint64_t seed) try {
     if (!ctx) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     HIPCHK(hipSetDevice(ctx->cfg.device));
     int rc = mlp_ready_alloc(ctx);
     if (rc) return rc;
@@ -1483,6 +1496,7 @@ int spz_mlp_init(spz_ctx *ctx, uint64_t seed) try {
 
 int spz_mlp_set_params(spz_ctx *ctx, const float *params) try {
     if (!ctx || !params) return SPZ_E_ARG;
+    if (!ctx->created) return not_created(ctx);
     HIPCHK(hipSetDevice(ctx->cfg.device));
     int rc = mlp_ready_alloc(ctx);
     if (rc) return rc;

@@ -70,3 +70,40 @@ assert len(s.eval_h(b)) == 30000
 s.close()
 assert F.fake_bytes(DEVICE) == 0 and F.fake_bytes(PINNED) == 0
 """)
+
+
+@pytest.mark.parametrize("heur", ["H_MANHATTAN", "H_PDB666"])
+def test_a_context_that_was_not_created_is_refused(fake, heur):
+    """spz_create hands back a context even when it fails, for its message:
+    wherever it failed, every call that would use the device is refused."""
+    fake(f"""
+L = spz.lib()
+def made():
+    cfg = spz.Config()
+    L.spz_default_config(ctypes.byref(cfg), 5, spz.{heur})
+    s = spz.Solver.__new__(spz.Solver)
+    s.cfg, s.width, s._ctx = cfg, 5, ctypes.c_void_p()
+    return s, L.spz_create(ctypes.byref(s._ctx), ctypes.byref(cfg))
+b = walks(5, 400)
+thr, tgt = np.full(400, 40, np.int32), np.zeros(400, np.float32)
+failed = 0
+for kind in (DEVICE, PINNED):
+    for after in range(12):
+        F.fake_fail(kind, after)
+        s, rc = made()
+        F.fake_fail(kind, -1)
+        if rc == 0:
+            s.close()
+            break
+        failed += 1
+        assert rc == -2, rc
+        for call in (lambda: s.eval_h(b), lambda: s.eval_h_noalloc(b[:1]), lambda: s.eval_h_noalloc(b),
+                     lambda: s.solve(b), lambda: s.build_pdb(), lambda: s.mlp_init(1),
+                     lambda: s.load_pdb_tab("/dev/null", "/dev/null"),
+                     lambda: s.mlp_set_params(np.zeros(s.mlp_param_count(), np.float32)),
+                     lambda: s.reconfigure(frontier_target=8), lambda: s.autotune(b[:2])):
+            refused(call)
+        s.close()
+assert failed >= 4, failed
+assert F.fake_bytes(DEVICE) == 0 and F.fake_bytes(PINNED) == 0
+""")
