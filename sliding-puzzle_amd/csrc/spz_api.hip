@@ -337,7 +337,7 @@ static int configure_lanes(spz_ctx *ctx) {
         lanes = ctx->n_cu * blocks * wg;
     }
     lanes = (lanes + wg - 1) / wg * wg;
-    ctx->n_lanes = lanes;
+    ctx->n_lanes = 0; // until all of their state is there, no solve runs
     size_t L = (size_t)lanes;
     int maxd = cfg->lds_stack_depth;
     if ((e = ctx->c_st.ensure(L * 4)) != hipSuccess || (e = ctx->c_rows.ensure(L * 4 * 5)) != hipSuccess ||
@@ -345,6 +345,7 @@ static int configure_lanes(spz_ctx *ctx) {
         (e = ctx->c_cnt.ensure(L * 4)) != hipSuccess || (e = ctx->c_pdb.ensure(L * 4 * 10)) != hipSuccess ||
         (e = ctx->c_origin.ensure(L * 4)) != hipSuccess || (e = ctx->c_stack.ensure(L * (size_t)maxd * 2)) != hipSuccess)
         return fail(ctx, SPZ_E_HIP, "lane context allocation: %s", hipGetErrorString(e));
+    ctx->n_lanes = lanes;
     return SPZ_OK;
 }
 
@@ -1022,6 +1023,7 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
         return fail(ctx, SPZ_E_ARG, "max_iters must be in 1..%d", kMaxIters);
     if (n == 0) return SPZ_OK;
     if (n > (1 << 24)) return fail(ctx, SPZ_E_ARG, "batch too large");
+    if (ctx->n_lanes == 0) return fail(ctx, SPZ_E_HIP, "no lanes: the last spz_reconfigure failed");
     const int w = ctx->cfg.width, heur = ctx->cfg.heuristic;
     if (heur == SPZ_H_PDB666 && !ctx->have_pdb) return fail(ctx, SPZ_E_NOPDB, "call spz_build_pdb first");
     for (int i = 0; i < n; ++i)

@@ -107,3 +107,27 @@ for kind in (DEVICE, PINNED):
 assert failed >= 4, failed
 assert F.fake_bytes(DEVICE) == 0 and F.fake_bytes(PINNED) == 0
 """)
+
+
+@pytest.mark.parametrize("after", range(8))
+def test_a_failed_reconfiguration_leaves_nothing_to_solve_on(fake, after):
+    """A reconfiguration that finds no memory for the lanes' state: a solve is
+    refused until one succeeds, and launches nothing."""
+    fake(f"""
+s = spz.Solver(width=5, frontier_target=4, lanes=256, lds_stack_depth=16)
+b = walks(5, 3)
+F.fake_fail(DEVICE, {after})
+refused(lambda: s.reconfigure(lanes=1024, lds_stack_depth=32))
+refused(lambda: s.solve(b))
+assert len(s.eval_h_noalloc(b)) == 3
+F.fake_fail(DEVICE, -1)
+refused(lambda: s.solve(b))
+s.reconfigure(lanes=512)
+before = F.fake_count(LAUNCHES)
+try:
+    s.solve(b)
+except spz.SpzError as e:
+    assert e.code == -7, e  # the stand-in's kernels search nothing
+assert F.fake_count(LAUNCHES) > before
+s.close()
+""")
