@@ -131,3 +131,34 @@ except spz.SpzError as e:
 assert F.fake_count(LAUNCHES) > before
 s.close()
 """)
+
+
+def test_calls_that_grow_slowly_seldom_allocate(fake):
+    """Calls of a few rows more each time: the context's workspaces grow by
+    half, so few of the calls allocate or pin anything."""
+    fake("""
+b = walks(5, 1000)
+thr, tgt = np.full(1000, 40, np.int32), np.zeros(1000, np.float32)
+with spz.Solver(width=5, frontier_target=4) as s:
+    s.mlp_init(1)
+    s.mlp_predict(b[:700], thr[:700])
+    at = F.fake_count(DEVICE), F.fake_count(PINNED)
+    for n in range(701, 1001):
+        s.mlp_predict(b[:n], thr[:n])
+    new = F.fake_count(DEVICE) - at[0], F.fake_count(PINNED) - at[1]
+    assert new[0] <= 3 and new[1] <= 2, new
+    # the gradient's own buffers exist after the largest call
+    s.mlp_grad(b, thr, tgt)
+    at = F.fake_count(DEVICE)
+    for n in range(1, 1001, 7):
+        s.mlp_grad(b[:n], thr[:n], tgt[:n])
+    assert F.fake_count(DEVICE) == at
+many = np.repeat(walks(4, 1000), 20, axis=0)
+with spz.Solver(width=4, frontier_target=4) as s:
+    at = F.fake_count(DEVICE), F.fake_count(PINNED)
+    for n in range(4000, 20001, 50):
+        s.eval_h(many[:n])
+    assert F.fake_count(DEVICE) == at[0]
+    assert F.fake_count(PINNED) - at[1] <= 6, F.fake_count(PINNED) - at[1]
+assert F.fake_bytes(DEVICE) == 0 and F.fake_bytes(PINNED) == 0
+""")
