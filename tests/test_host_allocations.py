@@ -162,3 +162,35 @@ with spz.Solver(width=4, frontier_target=4) as s:
     assert F.fake_count(PINNED) - at[1] <= 6, F.fake_count(PINNED) - at[1]
 assert F.fake_bytes(DEVICE) == 0 and F.fake_bytes(PINNED) == 0
 """)
+
+
+def test_a_very_large_call_gives_its_buffers_back(fake):
+    """What a predictor call leaves allocated for the next one is bounded: a
+    call of a million rows holds no more after it than a common one may."""
+    fake("""
+n = 1_000_000
+b = np.tile(walks(5, 1000), (n // 1000, 1))
+thr = np.full(n, 40, np.int32)
+with spz.Solver(width=5, frontier_target=4) as s:
+    s.mlp_init(1)
+    s.mlp_predict(b[:4], thr[:4])
+    held = F.fake_bytes(DEVICE)
+    for rep in range(2):
+        assert len(s.mlp_predict(b, thr)) == n
+        assert F.fake_bytes(DEVICE) - held <= 32 << 20, F.fake_bytes(DEVICE) - held
+    # and where the call fails
+    F.fake_fail(DEVICE, 1)  # the packed boards find memory, the predictions none
+    try:
+        s.mlp_predict(b, thr)
+        raise AssertionError("not refused")
+    except spz.SpzError as e:
+        assert e.code == -2, e
+    assert F.fake_bytes(DEVICE) - held <= 32 << 20
+    F.fake_fail(DEVICE, -1)
+    # common calls keep theirs
+    s.mlp_predict(b[:20000], thr[:20000])
+    at = F.fake_count(DEVICE)
+    s.mlp_predict(b[:20000], thr[:20000])
+    assert F.fake_count(DEVICE) == at
+assert F.fake_bytes(DEVICE) == 0 and F.fake_bytes(PINNED) == 0
+""")
