@@ -6,8 +6,9 @@ A step is one solve of the configuration's whole batch of synthetic
 instances (seeded generators; seed = config_id * 10^6 + instance index),
 inputs already on the host in packed form; the per-step result (optimal
 lengths and node counts) is checked to be identical across steps.  The
-timed steps replay the search rounds from the solver's captured hipGraph;
-a separate step with every round launch timed by HIP events gives the
+timed steps replay the search rounds from the solver's captured hipGraph
+where solves run more than 24 (`rounds_replayed_frac` in the line); a
+separate step with every round launch timed by HIP events gives the
 kernel's average duration (the roofline).  The default policy is the
 learned predictor with re-splitting of nodes predicted above 2 x the mean.
 Prints one JSON line.  Configurations:
@@ -153,7 +154,7 @@ def progress(*a):
     print("bench:", *a, file=sys.stderr, flush=True)
 
 
-STAT_KEYS = ("round_kernel_ms", "round_launches", "solve_ms", "setup_ms", "split_ms",
+STAT_KEYS = ("graph_replays", "round_kernel_ms", "round_launches", "solve_ms", "setup_ms", "split_ms",
              "rounds_wall_ms", "rounds", "donated")
 
 
@@ -392,19 +393,20 @@ def main():
         progress("warmup step done")
     nodes_total = 0
     brk = dict.fromkeys(STAT_KEYS, 0.0)
-    graph_used = True
     t0 = time.perf_counter()
     for _ in range(args.steps):
         res, acc = solve_step(solver, boards, per_instance, args.max_iters)
         for k in brk:
             brk[k] += acc[k] / args.steps
-        graph_used = graph_used and solver.stats()["graph"] == 1.0
         nodes_total += sum(r.total_nodes for r in res)
         if ref is not None:
             assert same(res, ref)
         ref = res
         progress("timed step done")
     elapsed = time.perf_counter() - t0
+    # rounds replayed from the hipGraph, four a replay: a solve's first 24 are
+    # launched one by one
+    replayed = 4 * brk["graph_replays"] / max(brk["rounds"], 1.0)
     n = len(boards)
     ms_per_step = elapsed / args.steps * 1e3
     inst_per_s = n * args.steps / elapsed
@@ -477,8 +479,10 @@ def main():
                    "frontier_target": FRONTIER[args.config], "parallelism": "single GPU"},
         "nodes_per_s": nodes_per_s, "nodes_per_step": nodes_total / args.steps,
         "unsolved_within_max_iters": unsolved,
-        "timed_path": "hipGraph replay of the search rounds" if graph_used and not args.eager
-        else "eager launches (kernel timing on)",
+        "timed_path": "eager launches (kernel timing on)" if args.eager
+        else "hipGraph replay of the search rounds" if replayed > 0.5
+        else "search rounds launched one by one (most solves too short for the hipGraph)",
+        "rounds_replayed_frac": replayed,
         "eager_timed_step_instances_per_s": n / kdt,
         "roofline": roof,
         "breakdown_per_step": dict(brk, lanes=solver.stats()["lanes"]),

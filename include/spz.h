@@ -87,7 +87,8 @@ typedef struct spz_config {
                                 events on the solver's stream (stats 8-9);
                                 the rounds then run without the hipGraph */
     int32_t use_graph;       /* 1: replay the search rounds from a captured
-                                hipGraph (default); 0: launch them one by one */
+                                hipGraph, from the 25th on (default); 0:
+                                launch them one by one */
     int32_t log_samples;     /* >0: keep up to this many (frontier node,
                                 threshold, subtree count) samples per solve
                                 (spz_get_samples); training data of the MLP */
@@ -274,14 +275,17 @@ int spz_get_paths(spz_ctx *ctx, uint8_t *moves, int32_t max_len, int32_t *lens);
  *  12 nodes (all instances, all iterations)
  *  13 setup ms (to the first restart's enqueue)  14 rounds wall ms (with
  *     what of the setup still ran)
- *  15 1 if the rounds run from a hipGraph (from the seventh poll on)
+ *  15 1 unless the graph is off (use_graph, time_kernels) or could not be
+ *     captured; whether the solve was long enough for it (six polls of four
+ *     rounds are launched first) 26 tells
  *  16-19 with env SPZ_PROFILE=1: lane-steps idle, expanding, only popping,
  *        and wave-steps (x64 = lane-steps) of the search rounds;
  *  20-22 with SPZ_PROFILE=1 (PDB): moves into a sibling (2 table reads each),
  *        children's first-partition reads, second-partition reads
  *  23 iterations started as lookahead
  *  24 frontier nodes re-split (config resplit)  25 the queue items they became
- *  26-31 reserved (0)
+ *  26 polls (of four rounds) replayed from the hipGraph
+ *  27-31 reserved (0)
  * With env SPZ_TRACE=1 each poll of the round loop prints elapsed ms, busy
  * lanes, active instances and queued items to stderr. */
 #define SPZ_STATS_LEN 32

@@ -1240,7 +1240,7 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     long timed = 0;
     unsigned *const h_ctl = (unsigned *)ctx->stage.p; // pinned: 64 control words
     int rc = SPZ_OK;
-    long rounds = 0;
+    long rounds = 0, replays = 0;
 
     // one poll period: per_poll rounds, then the control words to the host
     auto enqueue_period = [&]() -> hipError_t {
@@ -1280,9 +1280,16 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
     constexpr long kGraphPeriod = 6;
     for (long period = 0;; ++period) {
         // the first periods are launched kernel by kernel, which the rounds
-        // before hide from the device: making the graph costs 165 us
+        // before hide from the device: making the graph costs 165 us, on the
+        // host's time where the device runs rounds meanwhile.  From period 0,
+        // 1, 3, 6, 12, never: one 30-move 15-puzzle 588 us, 630, 571, 569,
+        // 566, 565; 100 walks of 40 moves 3.31 ms, 3.40, 3.23, 3.25, 3.23,
+        // 3.24; 25 24-puzzles (33 rounds) 64.6 ms, 65.2, 64.7, 65.5, 65.8,
+        // 65.2; long batches the same to 0.5%
         if (period == kGraphPeriod && use_graph) make_graph();
-        hipError_t e = period >= kGraphPeriod && use_graph ? hipGraphLaunch(gexec, s) : enqueue_period();
+        const bool replay = period >= kGraphPeriod && use_graph;
+        hipError_t e = replay ? hipGraphLaunch(gexec, s) : enqueue_period();
+        replays += replay ? 1 : 0;
         rounds += per_poll;
         if (e == hipSuccess) e = hipStreamSynchronize(s);
         if (timing && e == hipSuccess) {
@@ -1328,6 +1335,7 @@ int spz_solve_batch(spz_ctx *ctx, const uint8_t *boards, int32_t n, int32_t max_
         for (auto &x : ev) (void)hipEventDestroy(x);
     if (rc != SPZ_OK) return rc;
     ctx->stats[15] = use_graph ? 1.0 : 0.0;
+    ctx->stats[26] = (double)replays;
     ctx->stats[14] = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_rounds).count();
     ctx->stats[8] = round_ms;
     ctx->stats[9] = (double)timed;

@@ -463,4 +463,5 @@ class Solver:
                 "setup_ms": s[13], "rounds_wall_ms": s[14], "graph": s[15],
                 "prof_idle": s[16], "prof_expand": s[17], "prof_pop": s[18], "prof_wave_steps": s[19],
                 "prof_sibling_moves": s[20], "prof_reads_first": s[21], "prof_reads_second": s[22],
-                "lookahead_starts": s[23], "resplit_nodes": s[24], "resplit_items": s[25]}
+                "lookahead_starts": s[23], "resplit_nodes": s[24], "resplit_items": s[25],
+                "graph_replays": s[26]}
