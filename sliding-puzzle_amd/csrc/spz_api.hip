@@ -354,7 +354,7 @@ static int configure_lanes(spz_ctx *ctx) {
     ctx->n_lanes = 0; // until all of their state is there, no solve runs
     size_t L = (size_t)lanes;
     int maxd = cfg->lds_stack_depth;
-    if ((e = ctx->c_st.ensure(L * 4)) != hipSuccess || (e = ctx->c_rows.ensure(L * 4 * 5)) != hipSuccess ||
+    if ((e = ctx->c_st.ensure(L * 4)) != hipSuccess || (e = ctx->c_rows.ensure(L * 4 * 4)) != hipSuccess ||
         (e = ctx->c_meta.ensure(L * 4)) != hipSuccess || (e = ctx->c_inst.ensure(L * 4)) != hipSuccess ||
         (e = ctx->c_cnt.ensure(L * 4)) != hipSuccess || (e = ctx->c_pdb.ensure(L * 4 * 10)) != hipSuccess ||
         (e = ctx->c_origin.ensure(L * 4)) != hipSuccess || (e = ctx->c_stack.ensure(L * (size_t)maxd * 2)) != hipSuccess)

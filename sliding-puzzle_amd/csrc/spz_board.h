@@ -203,8 +203,6 @@ constexpr uint32_t kWeightMask = 0x0fffffffu;
 // rf / rot90 / rot180 tables, src/24puzzle_with_pdb.cc:33-46).
 void pdb_geo_build(PdbGeo *g);
 
-__host__ __device__ inline uint32_t pdb_tab_of(int k) { return (k == 0 || k == 4) ? 0u : 1u; }
-
 constexpr uint64_t kPdbDirect = 244140625ull; // 25^6
 
 // Per-lane heuristic state.
@@ -247,24 +245,6 @@ __device__ __forceinline__ uint32_t set_byte(uint32_t w, int k, int v) {
 
 // idx carries its table's offset, so every lookup is one load from one base
 __device__ __forceinline__ int pdb_read(const PdbCtx &P, uint32_t idx) { return (int)P.tab[idx]; }
-
-// Heuristic of the child reached by moving tile t from cell a to cell b,
-// without changing the state (f-tests at expansion); the two values read
-// are returned packed (regular | reflected << 8) for reuse by pdb_apply_known.
-__device__ __forceinline__ int pdb_child_h(const PdbCtx &P, const HState<1> &s, int t, int a, int b,
-                                           uint32_t &vals) {
-    const PdbGeo &G = *P.geo;
-    const uint2 wa = G.w[t][a], wb = G.w[t][b];
-    const int kr = (int)(wa.x >> 28), kf = (int)(wa.y >> 28);
-    uint32_t ir = sel4(s.i0, s.i1, s.i2, s.i3, kr) + (wb.x - wa.x);
-    uint32_t iff = sel4(s.j0, s.j1, s.j2, s.j3, kf) + (wb.y - wa.y);
-    int vr = pdb_read(P, ir);
-    int vf = pdb_read(P, iff);
-    vals = (uint32_t)vr | ((uint32_t)vf << 8);
-    int A = s.A - byte_of(s.v0, kr) + vr;
-    int B = s.B - byte_of(s.v1, kf) + vf;
-    return A > B ? A : B;
-}
 
 // pdb_apply with the two new values already known (no gathers)
 __device__ __forceinline__ void pdb_apply_known(const PdbCtx &P, HState<1> &s, int t, int a, int b,
@@ -580,18 +560,6 @@ __device__ __forceinline__ void move_pdb_finish(HState<1> &h, const PendMove &m)
     h.v0 = set_byte(h.v0, m.kr, m.vr);
     h.v1 = set_byte(h.v1, m.kf, m.vf);
     h.h = h.A > h.B ? h.A : h.B;
-}
-
-// values, before the move, of the two lookups containing the tile that a
-// blank move in direction d slides (packed regular | reflected << 8)
-template <int W, class BD>
-__device__ __forceinline__ uint32_t pdb_moved_vals(const Pos<W, 1, BD> &s, int d, const PdbCtx &P) {
-    int nr = s.br + dir_dr(d);
-    int nc = s.bc + dir_dc(d);
-    int t = s.bd.tile(nr * W + nc);
-    const PdbGeo &G = *P.geo;
-    int kr = G.reg_k[t], kf = G.ref_k[t] - 4;
-    return (uint32_t)byte_of(s.hs.v0, kr) | ((uint32_t)byte_of(s.hs.v1, kf) << 8);
 }
 
 // One DFS stack level: the move d taken from it, the passing children R

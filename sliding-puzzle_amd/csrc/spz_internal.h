@@ -165,7 +165,7 @@ struct KParams {
     unsigned long long *wtime; // null, or [2][waves]: start and end clock of each wave in round wtime_round
     unsigned wtime_round;
     uint32_t *c_st;    // state | sp<<8
-    uint32_t *c_rows;  // [5][n_lanes]
+    uint32_t *c_rows;  // [4][n_lanes] packed board
     uint32_t *c_meta;  // blank,g,h,prev of the current node
     uint32_t *c_inst;
     uint32_t *c_cnt;

@@ -1829,7 +1829,7 @@ __global__ void __launch_bounds__(kBeginThreads) k_begin(KParams p, const PdbGeo
                                                          unsigned long long *lp0, unsigned long long *lp1, int split) {
     __shared__ PdbGeo geo_s;
     __shared__ unsigned s_n[2], s_hist[kFBins];
-    __shared__ int s_goal, s_h;
+    __shared__ int s_goal;
     PdbCtx P{&geo_s, p.pdb};
     load_geo<HEUR>(geo_s, geo_g);
     const int inst = (int)blockIdx.x, t = threadIdx.x;
@@ -1856,7 +1856,6 @@ __global__ void __launch_bounds__(kBeginThreads) k_begin(KParams p, const PdbGeo
         s_n[0] = 1;
         s_n[1] = 0;
         s_goal = kNoGoal;
-        s_h = h;
         p.it[inst] = 0;
         p.nlive[inst] = 0;
         p.want_next[inst] = 0;
