@@ -291,10 +291,11 @@ void spz_default_config(spz_config *cfg, int32_t width, int32_t heuristic) {
 // Step budget and time limit of a round when the configuration leaves them
 // open.  Waves share work while a round runs and end it themselves when many
 // have none, so a round is long: what it costs is that an instance whose
-// iteration ends inside it waits for its next one.  Measured on MI355X, 250
-// mixed 15-puzzles: 2 ms 1048 ms, 3.5 ms 1053, 4.5 ms 1037, 10 ms 1035; 24
-// 24-puzzles with the PDB 181 / 178 / 179 / 180.  The step budget only bounds
-// rounds whose time limit is off.
+// iteration ends inside it waits for its next one.  Measured on MI355X, limits
+// of 2 ms, 3.5, 4.5 and 10, two inputs each: 250 mixed 15-puzzles 984 ms, 979,
+// 981, 973 and 366, 365, 365, 363; 24 24-puzzles with the PDB 147, 142, 139,
+// 137 and 88, 79, 78, 75.  The step budget only bounds rounds whose time limit
+// is off.
 constexpr int kRoundSteps = 8192;
 constexpr int kRoundTimeUs = 4500;
 
@@ -302,12 +303,19 @@ constexpr int kRoundTimeUs = 4500;
 // LDS holds (stack, boards, sibling values: 53.6 KB per 256 lanes).
 constexpr int kLanesPerCuPdb = 768;
 // Lanes per initial work item (root-split frontier node) when the lane count
-// is automatic: a small search is over before many waves are fed (one random
-// 15-puzzle, 2048 frontier nodes: 65536 lanes 5.2 ms, 131072 4.7, 262144 5.0,
-// 524288 5.4; 250 mixed ones, 16 each: 131072 lanes 1513 ms, 256000 1040,
-// 524288 1030).
+// is automatic: a small search is over before many waves are fed.  16, 32, 64,
+// 128 and 256 an item, two inputs each: one random 15-puzzle, 2048 frontier
+// nodes (131,072 lanes at 64) 4.67 ms, 4.67, 4.23, 4.20, 4.32 and 2.21, 2.21,
+// 2.14, 2.26, 2.38; 250 mixed ones, 16 each (256,000 lanes at 64) 2564 ms, 1443,
+// 978, 926, 922 and 915, 521, 363, 373, 367.
 constexpr size_t kLanesPerItem = 64;
-// largest root-split target that a workgroup per instance splits (k_begin)
+// Largest root-split target that a workgroup per instance splits (k_begin).
+// Against a launch a level over the whole device, a whole solve of one easy
+// board (15-puzzle, 24-puzzle, 24-puzzle with the PDB): 16384 nodes 0.29 ms
+// against 0.58, 0.31/0.55, 0.45/0.62; 32768 0.50/0.93, 0.53/0.90, 0.84/0.99;
+// 65536 0.95/1.72, 1.12/1.87, 1.80/1.93, with eight boards a quarter or less.
+// The line lies well inside: one workgroup is one of 256 compute units, and
+// with larger frontiers a level is long enough to be worth the others.
 constexpr unsigned kOneBlockSplit = 16384;
 // largest upload or download through pinned staging; larger ones stream from
 // and to pageable memory
@@ -324,10 +332,12 @@ constexpr int kBoardsPiece = 65536;
 // boards spz_eval_h_noalloc checks on the host: waiting for the device's
 // verdict before the values are copied costs 8 us, a board's check 45 ns
 constexpr int kHostCheck = 256;
-// A round ends early once the waves that ran out of work have waited, summed
-// over them and divided by all waves, this long: about what it costs to end a
-// round, save and restore the lanes, start iterations and feed the waves again.
-// 300 us, 450, 600, 900: first solutions of three batches 139 ms, 138, 134, 139;
+// A round ends early once the time since a looking wave began to work, times
+// the share of the waves that wait at that look, is this long: about what it
+// costs to end a round, save and restore the lanes, start iterations and feed
+// the waves again.  It is an estimate of the waiting, not its sum: late in a
+// round a wave that has waited for a moment counts as much as one that has
+// waited since the start, and waits that a mail ended do not count.  300 us, 450, 600, 900: first solutions of three batches 139 ms, 138, 134, 139;
 // three 24-puzzles with tables 21.2, 20.6, 20.0, 19.7; two batches of them 223,
 // 216, 216, 219; three without tables 168, 168, 169, 171; one random 15-puzzle
 // and 100 short walks the same.

@@ -460,8 +460,8 @@ __device__ __forceinline__ void do_move(Pos<W, HEUR, BD> &s, int d, const PdbCtx
 
 // Blank move that updates the board and blank only.  Queue items of the PDB
 // search need no heuristic state: a lane starting an item recomputes all
-// eight lookups from the board (pdb_init), so the positions of donated and
-// exported items are built with these moves and no table reads.
+// eight lookups from the board (pdb_init), so the positions of nodes given
+// away and of overflow items are built with these moves and no table reads.
 template <int W, int HEUR, class BD>
 __device__ __forceinline__ void move_board_only(Pos<W, HEUR, BD> &s, int d) {
     const int to = s.cell(), from = to + dir_cell<W>(d);

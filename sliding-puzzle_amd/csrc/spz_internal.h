@@ -160,7 +160,7 @@ struct KParams {
     int n_lanes;
     int maxd;          // LDS stack levels per lane in use
     unsigned long long *prof; // null, or [waves][8]: lane-steps idle, expanding, popping only, wave-steps, table reads
-    unsigned long long turn_ticks;  // waves without work, together, wait this long times the waves before a round ends
+    unsigned long long turn_ticks;  // a round ends once its time so far times the share of waves waiting is this long
     unsigned long long round_ticks; // rounds end this many wall-clock ticks after a wave's start (0: off)
     unsigned long long *wtime; // null, or [2][waves]: start and end clock of each wave in round wtime_round
     unsigned wtime_round;

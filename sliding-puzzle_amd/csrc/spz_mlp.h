@@ -77,8 +77,9 @@ hipError_t mlp_features_gather(MlpState &m, int width, const Item *items, const 
 hipError_t mlp_adam_step(MlpState &m, float lr, hipStream_t s);
 
 // Predictions at kPredThr consecutive thresholds L0, L0+2, ... per node, by
-// one fused kernel (one wave per node; the thresholds of a node are the 16
-// rows of one MFMA tile and share layer 1 up to a rank-1 term).
+// one fused kernel (a wave takes one node, or two where there are many; the
+// thresholds of a node are the 16 rows of one MFMA tile and share layer 1 up
+// to a rank-1 term).
 constexpr int kPredThr = 16;
 // every frontier node of every instance:
 // pred[(inst*capl + i)*kPredThr + k] = y(frontier node i, L = h0[inst] + 2k)

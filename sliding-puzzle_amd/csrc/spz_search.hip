@@ -4,13 +4,15 @@
 // threshold sequence h0, h0+2, ... (src/24puzzle.cc:146-152).  An iteration
 // of an instance is:
 //   * its top tree (root split, src/15puzzle_block_parallel.cu:150-187, done
-//     once per solve by k_split_level): the count of every top node whose f
-//     fits the threshold is added from an f-histogram, and
+//     once per solve by k_begin, or by k_split_level where duplicates are
+//     pruned or the frontier is very large): the count of every top node whose
+//     f fits the threshold is added from an f-histogram, and
 //   * one work item per frontier node whose f fits the threshold; items are
-//     searched depth-first by single lanes (k_round), which may donate their
-//     shallowest unexplored children back to the queue when lanes go idle
-//     (device-wide work stealing; the reference steals only inside a block,
-//     src_horie/idas_dynamic.cu:199-247).
+//     searched depth-first by single lanes (k_round).  While a round runs, a
+//     wave's idle lanes take the shallowest open nodes of its busy ones, and
+//     waves without work are fed by others through mailboxes (the reference
+//     shares only inside a block, src_horie/idas_dynamic.cu:199-247); the
+//     queue holds frontier nodes and what overflows a stack.
 // The count of iteration L is  sum_{top u: F(u)<=L} gen(u)
 //                            + sum_{frontier v: F(v)<=L} subtree_count(v),
 // where gen(u) counts every in-bounds non-reverse child of an expanded node
@@ -241,10 +243,10 @@ __device__ __forceinline__ const KParams &params_again() {
 // full stacks) and evens out its work: its idle lanes take the shallowest
 // open nodes of its busy ones, by lane exchange.  A wave without any work
 // takes items of the queue, one where there are fewer items than waves, and
-// leaves the round when there are none; the round ends when the waves that
-// left have waited as long, together, as a new round costs, and the working
-// waves then queue nodes for them.  Busy lanes keep their state across rounds
-// in the c_* context arrays.
+// where there are none it waits to be fed by a wave with work, through its
+// mailbox.  The round ends after its time or steps, when every wave waits, or
+// when so many wait that a new round is worth its cost (turn_ticks).  Busy
+// lanes keep their state across rounds in the c_* context arrays.
 //
 // What bounds the sharing is that atomics on one address are served one after
 // another, 12 ns each on MI355X whatever the die (83 M/s; loads of a line that
@@ -902,8 +904,9 @@ __global__ void __launch_bounds__(256, (W == 4 ? 8 : 3)) k_round(KParams p, cons
             init = false;
         }
         // the time limit, the round's end as some wave saw it, and, every few
-        // blocks, whether the waves without work have waited long enough
-        // (never before a wave's first block: every round makes progress)
+        // blocks, whether the waves waiting now, had they waited since this
+        // wave began to work, would have waited long enough (never before a
+        // wave's first block: every round makes progress)
         if (blk >= least) {
             const long long now = wall_clock64();
             bool stop = steps_left <= 0 || (p.round_ticks && (unsigned long long)(now - t_start) >= p.round_ticks);
